@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "bvh_build.h"
+#include "node.h"
 
 namespace rtx {
 
@@ -48,7 +49,7 @@ constexpr int kScanBlock = 1024;
 #endif
 constexpr float kCostTrav = RTX_SAH_TRAV;
 constexpr float kCostIsect = 1.0f;
-constexpr float kFarAway = 1e38f;   // coordinate of the empty-slot boxes and the degenerate triangle
+constexpr float kFarAway = 1e38f;   // coordinate of the degenerate triangle
 
 struct BuildTask {
     uint32_t node, begin, end, depth;
@@ -1157,26 +1158,29 @@ __global__ void k_write4(const BNode* __restrict__ bn, const uint4* __restrict__
                          uint32_t n, uint32_t base_this, uint32_t base_next, uint32_t empty_ref,
                          float4* __restrict__ nodes4, uint32_t* __restrict__ next_front,
                          const uint32_t* __restrict__ meta, const uint32_t* __restrict__ ntri,
-                         const uint32_t* __restrict__ first) {
+                         const uint32_t* __restrict__ first, float plane_scale) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint4 c4 = cid[i];
-    float lx[4], hx[4], ly[4], hy[4], lz[4], hz[4];
+    float lo[4][3], hi[4][3];
+    bool used[4];
     uint32_t ref[4];
     uint32_t j = off[i];
     for (int k = 0; k < 4; k++) {
         const uint32_t c = k == 0 ? c4.x : k == 1 ? c4.y : k == 2 ? c4.z : c4.w;
-        if (c == kNoChild) {
-            // an empty slot: a point box far outside any scene, which a slab
-            // test accepts only for rays aimed at it with an unbounded tmax;
-            // its ref is a one-triangle leaf holding a degenerate triangle
-            // (no ray hits it), so even then the traversal stays in bounds
-            lx[k] = hx[k] = ly[k] = hy[k] = lz[k] = hz[k] = kFarAway;
+        used[k] = c != kNoChild;
+        if (!used[k]) {
+            // an empty slot: an inverted box, which no slab test accepts; its
+            // ref is a one-triangle leaf holding a degenerate triangle (no
+            // ray hits it), so even then the traversal would stay in bounds
+            for (int a = 0; a < 3; a++) lo[k][a] = hi[k][a] = 0.f;
             ref[k] = empty_ref;
             continue;
         }
         const BNode b = bn[c];
-        lx[k] = b.lo.x; hx[k] = b.hi.x; ly[k] = b.lo.y; hy[k] = b.hi.y; lz[k] = b.lo.z; hz[k] = b.hi.z;
+        lo[k][0] = b.lo.x; hi[k][0] = b.hi.x;
+        lo[k][1] = b.lo.y; hi[k][1] = b.hi.y;
+        lo[k][2] = b.lo.z; hi[k][2] = b.hi.z;
         const uint32_t cntp = __float_as_uint(b.hi.w);
         if (meta && (meta[c] & 1u)) {
             ref[k] = leaf_ref(first[c], ntri[c]);
@@ -1188,16 +1192,7 @@ __global__ void k_write4(const BNode* __restrict__ bn, const uint4* __restrict__
             j++;
         }
     }
-    float4* o = nodes4 + kWideNodeF4 * (size_t)(base_this + i);
-    o[0] = make_float4(lx[0], lx[1], lx[2], lx[3]);
-    o[1] = make_float4(hx[0], hx[1], hx[2], hx[3]);
-    o[2] = make_float4(ly[0], ly[1], ly[2], ly[3]);
-    o[3] = make_float4(hy[0], hy[1], hy[2], hy[3]);
-    o[4] = make_float4(lz[0], lz[1], lz[2], lz[3]);
-    o[5] = make_float4(hz[0], hz[1], hz[2], hz[3]);
-    o[6] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
-                       __uint_as_float(ref[3]));
-    o[7] = make_float4(0.f, 0.f, 0.f, 0.f);
+    encode_node(nodes4 + kWideNodeF4 * (size_t)(base_this + i), lo, hi, used, ref, plane_scale);
 }
 
 // single-block exclusive scan of n uints -> out, total -> *total
@@ -1430,6 +1425,8 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
     const uint32_t *wmeta = nullptr, *wntri = nullptr, *wfirst = nullptr;
 #endif
 
+    out.plane_scale = plane_scale_for(std::max(std::max(root.hi.x - root.lo.x, root.hi.y - root.lo.y),
+                                               root.hi.z - root.lo.z));
     // 4-wide nodes: at most one per binary inner node
     uint32_t nwide = 0, wide_depth = 0;
     if (ninner) {
@@ -1458,7 +1455,7 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
 #endif
             scan_u32(cnt.p, n, off.p);
             hipLaunchKernelGGL(k_write4, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes.p, cid.p, off.p, n,
-                               nwide, nwide + n, leaf_ref(N, 1), wide.p, nxt, wmeta, wntri, wfirst);
+                               nwide, nwide + n, leaf_ref(N, 1), wide.p, nxt, wmeta, wntri, wfirst, out.plane_scale);
             RTX_TRY(hipGetLastError());
             uint32_t nn = 0;
             RTX_TRY(hipMemcpyAsync(&nn, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));

@@ -63,7 +63,7 @@ struct ThingRec {
 };
 
 struct Built {
-    rtx::DevScene hdr;                 // host copy of what the handle points at
+    rtx::DevScene hdr{};               // host copy of what the handle points at
     rtx::DevScene* d_hdr = nullptr;    // device copy; its address is the handle
     float4* nodes = nullptr;
     float4* tris = nullptr;
@@ -75,7 +75,8 @@ struct Built {
     // two-level scenes
     bool two_level = false;
     float4* xinst = nullptr;           // instance records (kInstF4 float4 each, + the null instance)
-    float4* ibox = nullptr;            // instance world boxes (lo, hi), + the null instance
+    float4* ibox = nullptr;            // instance world boxes (lo, hi), + the null instance, then the top-level nodes' own
+    float4* tbox = nullptr;            // the latter (inside ibox's allocation)
     std::vector<uint32_t> tlas_levels; // first top-level node of each level, then the count
     std::vector<uint32_t> blas_root;   // per mesh: bottom-level root in the scene arrays
     std::vector<float> blas_box;       // per mesh: object-space bounds lo.xyz, hi.xyz
@@ -89,7 +90,7 @@ struct Built {
         if (tri_world) (void)hipFree(tri_world);
         if (xinst) (void)hipFree(xinst);
         if (ibox) (void)hipFree(ibox);
-        d_hdr = nullptr; nodes = tris = insts = tri_world = xinst = ibox = nullptr;
+        d_hdr = nullptr; nodes = tris = insts = tri_world = xinst = ibox = tbox = nullptr;
     }
 };
 
@@ -561,6 +562,7 @@ static rtx_status build_scene_flat(rtx_ctx* c, hipStream_t s, Built** out) {
     b->hdr.root = bvh.root;
     b->hdr.num_prims = (uint32_t)N;
     b->hdr.num_nodes = bvh.num_wide;
+    b->hdr.plane_scale = bvh.plane_scale;
     b->hdr.num_insts = ninst;
     if ((e = hipMalloc((void**)&b->d_hdr, sizeof(rtx::DevScene))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(handle)"));
     if ((e = hipMemcpyAsync(b->d_hdr, &b->hdr, sizeof(rtx::DevScene), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload handle"));
@@ -847,13 +849,17 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
         if ((e = hipMemcpyAsync(b->nodes, tb.nodes, sizeof(float4) * rtx::kWideNodeF4 * tb.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy top level"));
         if ((e = rtx::tlas_leaves(b->nodes, tb.num_wide, tb.order, M, d_inst_of.p, ninst, s)) != hipSuccess) return bail(hip_fail(e, "top-level leaves"));
     }
+    // one scale for the planes of every tree
+    float plane_scale = M ? tb.plane_scale : 1.f;
+    for (size_t m = 0; m < nm; m++)
+        if (used[m]) plane_scale = std::max(plane_scale, bl.v[m].plane_scale);
     for (size_t m = 0; m < nm; m++) {
         if (!used[m]) continue;
         const rtx::BuiltBVH& x = bl.v[m];
         const uint32_t nb = (uint32_t)(tb.num_wide + node_off[m]), tbm = (uint32_t)tri_base[m];
         if (x.num_wide) {
             if ((e = hipMemcpyAsync(b->nodes + (size_t)rtx::kWideNodeF4 * nb, x.nodes, sizeof(float4) * rtx::kWideNodeF4 * x.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy bottom level"));
-            if ((e = rtx::relocate_blas(b->nodes, x.num_wide, nb, tbm, s)) != hipSuccess) return bail(hip_fail(e, "relocate"));
+            if ((e = rtx::relocate_blas(b->nodes, x.num_wide, nb, tbm, x.plane_scale / plane_scale, s)) != hipSuccess) return bail(hip_fail(e, "relocate"));
         }
         if ((e = hipMemcpyAsync(b->tris + 3 * (size_t)tbm, x.tris, sizeof(float4) * 3 * ((size_t)c->meshes[m].ni + 1), hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy triangles"));
         b->blas_root[m] = (x.root & rtx::kLeafFlag) ? x.root + tbm : x.root + nb;
@@ -861,14 +867,16 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     // records with the roots, then the top level's boxes from them
     tl_records(c, b, xrec, wbox);
     if ((e = hipMalloc((void**)&b->xinst, sizeof(float4) * xrec.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance records)"));
-    if ((e = hipMalloc((void**)&b->ibox, sizeof(float4) * wbox.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
+    if ((e = hipMalloc((void**)&b->ibox, sizeof(float4) * (wbox.size() + 2 * (size_t)tb.num_wide))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
+    b->tbox = b->ibox + wbox.size();
     if ((e = hipMalloc((void**)&b->insts, sizeof(float4) * irec.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(inst records)"));
     if ((e = hipMemcpyAsync(b->xinst, xrec.data(), sizeof(float4) * xrec.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload instance records"));
     if ((e = hipMemcpyAsync(b->ibox, wbox.data(), sizeof(float4) * wbox.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload instance boxes"));
     if ((e = hipMemcpyAsync(b->insts, irec.data(), sizeof(float4) * irec.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload inst records"));
     b->tlas_levels = tb.level_begin;
+    b->hdr.plane_scale = plane_scale;
     if (tb.num_wide) {
-        if ((e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, rtx::kInstLeaf | ninst, s)) != hipSuccess) return bail(hip_fail(e, "refit"));
+        if ((e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, b->hdr.plane_scale, s)) != hipSuccess) return bail(hip_fail(e, "refit"));
     }
 
     uint32_t root = rtx::kEmptyRoot;
@@ -906,7 +914,7 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     b->stats.sah_cost = (float)tb.sah;
     b->stats.build_ms = ms;
     b->stats.device_bytes = sizeof(float4) * ((uint64_t)rtx::kWideNodeF4 * total_nodes + 3ull * tri_total + irec.size() +
-                                              xrec.size() + wbox.size());
+                                              xrec.size() + wbox.size() + 2ull * tb.num_wide);
     b->stats.wide_nodes = (uint32_t)total_nodes;
     b->stats.wide_depth = tb.wide_depth + blas_wide_depth;
     b->stats.two_level = 1;
@@ -938,7 +946,7 @@ static rtx_status refit_scene_tl(rtx_ctx* c, Built* b, hipStream_t s) {
     if (e == hipSuccess) e = hipMemcpyAsync(b->xinst, xrec.data(), sizeof(float4) * xrec.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(b->ibox, wbox.data(), sizeof(float4) * wbox.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(b->insts, irec.data(), sizeof(float4) * irec.size(), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && b->tlas_levels.size() > 1) e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, rtx::kInstLeaf | ninst, s);
+    if (e == hipSuccess && b->tlas_levels.size() > 1) e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, b->hdr.plane_scale, s);
     if (e == hipSuccess) e = hipEventRecord(e1, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     float ms = 0.f;

@@ -27,14 +27,12 @@ template <int BLOCK, bool TL>
 __global__ __launch_bounds__(BLOCK) void k_trace(const DevScene sc, const rtx_ray* __restrict__ rays, uint32_t n,
                                                  rtx_hit* __restrict__ hits, uint32_t* gstack, uint32_t gstride,
                                                  uint32_t* counter, int batch) {
-    __shared__ uint32_t s_stack[kStackLDS * BLOCK];
+    __shared__ uint32_t s_stack[(kStackLDS + 1) * BLOCK];
     LaneStack<BLOCK> stk;
-    stk.lds = (lds_u32*)(s_stack + threadIdx.x);
-    stk.glob = gstack + blockIdx.x * BLOCK + threadIdx.x;
-    stk.gstride = gstride;
+    stk.init(s_stack, gstack + blockIdx.x * BLOCK + threadIdx.x, gstride);
     const uint32_t lane = threadIdx.x & 63u;
     Trav s;
-    trav_begin(s, sc, f3(0.f, 0.f, 0.f), f3(0.f, 0.f, 1.f), 0.f, 0.f);
+    trav_begin<TL>(s, sc, stk.bottom, f3(0.f, 0.f, 0.f), f3(0.f, 0.f, 1.f), 0.f, 0.f);
     bool going = false, held = false, exhausted = false;
     uint32_t i = 0;
     for (;;) {
@@ -49,7 +47,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(const DevScene sc, const rtx_ra
                 i = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
                 if (i < n) {
                     const rtx_ray ray = rays[i];
-                    trav_begin(s, sc, f3(ray.ori.x, ray.ori.y, ray.ori.z), f3(ray.dir.x, ray.dir.y, ray.dir.z),
+                    trav_begin<TL>(s, sc, stk.bottom, f3(ray.ori.x, ray.ori.y, ray.ori.z), f3(ray.dir.x, ray.dir.y, ray.dir.z),
                                ray.tmin, ray.tmax);
                     held = going = true;
                 } else {

@@ -104,26 +104,17 @@ __device__ __forceinline__ uint32_t find_job(const Job* jobs, uint32_t njobs, ui
 #ifndef RTX_COMPACT_LEAVES
 #define RTX_COMPACT_LEAVES 1
 #endif
-// the two-level frame kernels take the (P - o) * idir slab form: its six
-// fewer registers keep them from spilling next to the compacted leaf phase
-// (1080p / 64 spp: level-6 scene 98.7 -> 96.7 ms, mixed levels 114.1 ->
-// 109.8 ms against the FMA form)
-#ifndef RTX_TL_FMA
-#define RTX_TL_FMA 0
-#endif
 constexpr bool kCompactLeaves = RTX_COMPACT_LEAVES != 0;
 
-template <int BLOCK, bool COUNT, bool BATCH, int SLDS, bool ADJ = false, bool TL = false, bool FMA = true,
-          bool PROBE = false, int TOPN = 0>
+template <int BLOCK, bool COUNT, bool BATCH, int SLDS, bool ADJ = false, bool TL = false, bool PROBE = false,
+          int TOPN = 0>
 __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_stack, float* s_grad = nullptr,
                                             const lds_f4* top = nullptr) {
     constexpr bool CL = kCompactLeaves;
     __shared__ uint32_t s_cl[CL ? (BLOCK / 64) * kLeafScratchWords : 1];
     lds_u32* cl = (lds_u32*)(s_cl + (CL ? (threadIdx.x >> 6) * kLeafScratchWords : 0u));
     LaneStack<BLOCK, SLDS> stk;
-    stk.lds = (lds_u32*)(s_stack + threadIdx.x);
-    stk.glob = a.gstack + blockIdx.x * BLOCK + threadIdx.x;
-    stk.gstride = a.gstride;
+    stk.init(s_stack, a.gstack + blockIdx.x * BLOCK + threadIdx.x, a.gstride);
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tw = 1u << a.tile_log2w;
@@ -142,7 +133,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
     float3 thr = f3(1, 1, 1);
     float3 acc = f3(0, 0, 0), nacc = f3(0, 0, 0), aacc = f3(0, 0, 0), gN = f3(0, 0, 0), gA = f3(0, 0, 0);
     Trav tv;
-    trav_begin(tv, sc, f3(0, 0, 0), f3(0, 0, 1), 1e-3f, 1e16f);
+    trav_begin<TL>(tv, sc, stk.bottom, f3(0, 0, 0), f3(0, 0, 1), 1e-3f, 1e16f);
     uint64_t cyc_trav = 0;
     uint32_t wave_iters[2] = {0, 0};
     const uint64_t cyc_start = COUNT ? clock64() : 0;
@@ -242,7 +233,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
             gA = f3(0.f, 0.f, 0.f);
         }
         if (newsample || cont) {
-            trav_begin(tv, sc, ro, rdv, 1e-3f, 1e16f);     // optx/optics_r.cu:115-132 for a scattered ray
+            trav_begin<TL>(tv, sc, stk.bottom, ro, rdv, 1e-3f, 1e16f);     // optx/optics_r.cu:115-132 for a scattered ray
             going = true;
         }
         newsample = cont = false;
@@ -250,7 +241,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
         // traverse until a batch of lanes has a final closest hit; the others
         // keep their traversal state and resume after the shading below
         const uint64_t c0 = COUNT ? clock64() : 0;
-        trav_run<BLOCK, COUNT, TL, FMA, BATCH, TOPN, CL>(sc, tv, going, active, (int)a.batch,
+        trav_run<BLOCK, COUNT, TL, BATCH, TOPN, CL>(sc, tv, going, active, (int)a.batch,
                                                                      (int)a.inner_frac, stk, &cnt_nodes, &cnt_tris,
                                                                      wave_iters, top, cl);
         if (COUNT) cyc_trav += clock64() - c0;
@@ -465,19 +456,19 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
 
 // nodes of the top levels that each block of the frame kernels copies to LDS
 // (0: none; the node array is breadth-first, so these are nodes 0..N-1).
-// With the 32-entry LDS stack (32 KB per block) and the compacted leaf
-// phase's scratch (4 KB per block), 32 nodes (3.5 KB: the top two 4-wide
-// levels and 11 of the third) fill the CU's 160 KB at 4 blocks per CU.
-// Measured: on the 1080p / 500 spp frame of the level-6 scene (2.3 M nodes),
-// before the leaf phase was compacted, 21 nodes -0.5 %, 42 -0.4 %, 64 -1.1 %
-// time, and with it 32 nodes -0.8 %; on scenes whose arrays fit the MALL
-// (the level-4 scene, 0.15 M nodes: +2.5 %; the batch's small scenes: +4 %)
-// and on short frames of the level-6 scene (1 spp: +3 %) the waves whose
-// lanes split between LDS and global nodes issue both loads for too little
-// latency saved.  So frames of at least kOrderMinSpp samples per pixel of
-// scenes of at least kLdsTopMinNodes nodes take the staged kernels.
+// With the 32-entry LDS stack (33 KB per block with its bottom row) and the
+// compacted leaf phase's scratch (4 KB), 24 nodes (3 KB: the top two 4-wide
+// levels and 19 of the third) fill the CU's 160 KB at 4 blocks per CU.
+// Measured on the 1080p / 100 spp frame of the level-6 scene (1.8 M nodes):
+// 108.0 ms with them, 110.3 ms without.  Scenes whose arrays fit the MALL (the
+// level-4 scene, 0.1 M nodes: +2.5 % time; the batch's small scenes: +4 %) and
+// short frames of the level-6 scene (1 spp: +3 %) lose by them: the waves
+// whose lanes split between LDS and global nodes issue both loads for too
+// little latency saved (measured with 128-byte float nodes).  So frames of at
+// least kOrderMinSpp samples per pixel of scenes of at least kLdsTopMinNodes
+// nodes take the staged kernels.
 #ifndef RTX_LDS_TOP
-#define RTX_LDS_TOP 32
+#define RTX_LDS_TOP 24
 #endif
 constexpr int kLdsTop = RTX_LDS_TOP;
 constexpr uint32_t kLdsTopMinNodes = 1u << 20;   // 128 MB of nodes
@@ -493,20 +484,19 @@ __device__ __forceinline__ void stage_top(const DevScene& sc, float4* s_top) {
 // single frame: one block of 256 lanes per SIMD wave slot
 template <int BLOCK, bool COUNT, int SLDS, bool TL, int TOPN>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_RENDER_WAVES))) void k_render(const RenderArgs a) {
-    __shared__ uint32_t s_stack[SLDS * BLOCK];
+    __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
     __shared__ float4 s_top[TOPN > 0 ? TOPN * kWideNodeF4 : 1];
     if (TOPN > 0) stage_top<BLOCK, TOPN>(a.job.sc, s_top);
-    render_body<BLOCK, COUNT, false, SLDS, false, TL, !TL || RTX_TL_FMA, false, TOPN>(a, s_stack, nullptr,
-                                                                                   (const lds_f4*)s_top);
+    render_body<BLOCK, COUNT, false, SLDS, false, TL, false, TOPN>(a, s_stack, nullptr, (const lds_f4*)s_top);
 }
 
 // the probe of a plain frame: one sample per pixel, rays counted per tile
 template <int BLOCK, int SLDS, bool TL, int TOPN>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_RENDER_WAVES))) void k_probe(const RenderArgs a) {
-    __shared__ uint32_t s_stack[SLDS * BLOCK];
+    __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
     __shared__ float4 s_top[TOPN > 0 ? TOPN * kWideNodeF4 : 1];
     if (TOPN > 0) stage_top<BLOCK, TOPN>(a.job.sc, s_top);
-    render_body<BLOCK, false, false, SLDS, false, TL, true, true, TOPN>(a, s_stack, nullptr, (const lds_f4*)s_top);
+    render_body<BLOCK, false, false, SLDS, false, TL, true, TOPN>(a, s_stack, nullptr, (const lds_f4*)s_top);
 }
 
 __global__ void k_zero_n(uint32_t* p, uint32_t n) {
@@ -580,13 +570,13 @@ __global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost
 // of 3 waves
 template <int BLOCK, int SLDS, bool TL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_BATCH_WAVES))) void k_render_batch(const RenderArgs a) {
-    __shared__ uint32_t s_stack[SLDS * BLOCK];
-    render_body<BLOCK, false, true, SLDS, false, false, false>(a, s_stack);
+    __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
+    render_body<BLOCK, false, true, SLDS>(a, s_stack);
 }
 template <int BLOCK, int SLDS>
 __global__ __launch_bounds__(BLOCK) void k_render_batch_tl(const RenderArgs a) {
-    __shared__ uint32_t s_stack[SLDS * BLOCK];
-    render_body<BLOCK, false, true, SLDS, false, true, false>(a, s_stack);
+    __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
+    render_body<BLOCK, false, true, SLDS, false, true>(a, s_stack);
 }
 
 // adjoint: replays every sample path of a frame (same per-pixel Frand48
@@ -595,7 +585,7 @@ __global__ __launch_bounds__(BLOCK) void k_render_batch_tl(const RenderArgs a) {
 // (when the instances fit) are flushed with one global atomic per entry
 template <int BLOCK, int SLDS, bool TL>
 __global__ __launch_bounds__(BLOCK) void k_adjoint(const RenderArgs a) {
-    __shared__ uint32_t s_stack[SLDS * BLOCK];
+    __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
     extern __shared__ float s_grad[];
     const uint32_t ng = 4u * a.job.sc.num_insts;
     if (a.lds_grad) {
@@ -639,12 +629,10 @@ __global__ void k_get_materials(const float4* __restrict__ insts, uint32_t n, fl
 // optx/optics_r.cu:24-28 / optx/camera_r.cu:125-129
 template <bool TL>
 __global__ __launch_bounds__(64) void k_pick(const RenderArgs a) {
-    __shared__ uint32_t s_stack[kStackLDS * 64];
+    __shared__ uint32_t s_stack[(kStackLDS + 1) * 64];
     if (threadIdx.x != 0) return;
     LaneStack<64> stk;
-    stk.lds = (lds_u32*)s_stack;
-    stk.glob = a.gstack;
-    stk.gstride = a.gstride;
+    stk.init(s_stack, a.gstack, a.gstride);
     const rtx_lp_general& lp = a.job.lp;
     const uint32_t W = lp.image_w, H = lp.image_h;
     const uint32_t x = lp.pick_x, y = lp.pick_y;
@@ -657,7 +645,7 @@ __global__ __launch_bounds__(64) void k_pick(const RenderArgs a) {
     const float3 o = ld(lp.camera.eye) + off;
     const float3 d = ((s * ld(lp.camera.wvec) + t * ld(lp.camera.hvec)) - ld(lp.camera.dvec)) - off;
     TRay r;
-    tray_init(r, o, d, 1e-3f);
+    tray_init<!TL>(r, o, d, 1e-3f, 1e16f);
     HitFull h;
     traverse<64, TL>(a.job.sc, r, 1e16f, h, stk);
     *lp.pick_id = h.tri == kNoHit ? 0xFFFFFFFFu

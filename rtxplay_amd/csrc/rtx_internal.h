@@ -1,15 +1,23 @@
 // rtx_internal.h -- device data layouts and helpers shared by the kernels.
 //
 // Layout in HBM of a built scene (what a traversable handle points at):
-//   nodes : 4-wide BVH nodes, 128 B each = 8 x float4, structure of arrays
-//           over the 4 children: lo.x[4], hi.x[4], lo.y[4], hi.y[4],
-//           lo.z[4], hi.z[4], refs[4] (uint bits), unused
+//   nodes : 4-wide BVH nodes, 128 B each, 112 B used:
+//             0  x planes: lo[4], hi[4], lo[4] as halves (24 B)
+//            24  y planes, the same
+//            48  origin.xyz, 0 (float4)
+//            64  z planes, the same as x
+//            96  refs[4] (float4 of uint bits)
+//           a plane is at origin + plane_scale * half, rounded outwards
+//           (encode_node in node.h); a ray that enters a box through its lo
+//           plane reads an axis from its first lo on, else from hi on, and
+//           gets the entry planes followed by the exit planes either way
 //           ref without bit 31: inner node index; ref with bit 31 set: leaf,
 //           bits 27..30 = count-1, bits 0..26 = first leaf-ordered triangle;
 //           bits 27..31 all set (kInstLeaf): a top-level leaf holding one
 //           instance, whose id is in bits 0..26 (two-level scenes only).
-//           An empty child slot is a point box at 1e38 with a leaf ref to a
-//           degenerate triangle (or to the null instance of a top level).
+//           An empty child slot is an inverted box (lo inf, hi -inf) with a leaf
+//           ref to a degenerate triangle (or to the null instance of a top
+//           level).
 //   tris  : leaf-ordered triangles, 48 B each = 3 x float4
 //           (v0.xyz | global prim id), (v1.xyz | instance id),
 //           (v2.xyz | primitive index inside the instance's mesh)
@@ -44,6 +52,9 @@ constexpr uint32_t kNoHit = 0xFFFFFFFFu;
 constexpr uint32_t kEmptyRoot = 0xFFFFFFFFu;
 constexpr uint32_t kNoChild = 0x7FFFFFFFu;  // empty slot of a 4-wide node (no leaf flag, no valid node)
 constexpr int kWideNodeF4 = 8;             // float4 per 4-wide node (128 B)
+constexpr int kNodeOrigin = 3;             // the float4 of a node that holds its origin
+constexpr int kNodeRefs = 6;               // the float4 of a node that holds the refs
+constexpr uint32_t kNodePlanes[3] = {0u, 24u, 64u};   // byte offset of each axis's planes
 constexpr uint32_t kInstLeaf = 0xF8000000u; // top-level leaf of one instance: kInstLeaf | instance id
 constexpr uint32_t kInstMarker = 0x7FFFFFFEu;  // stack entry below an instance's bottom-level entries
 constexpr int kInstF4 = 8;                 // float4 per instance record of a two-level scene (128 B)
@@ -91,6 +102,8 @@ struct DevScene {
     uint32_t num_prims;
     uint32_t num_nodes;   // 4-wide nodes in the node array
     uint32_t num_insts;
+    float plane_scale;    // world units of a node plane's half (a power of two)
+    uint32_t pad;         // 0 (headers are compared as bytes)
 };
 
 __host__ __device__ inline uint32_t leaf_ref(uint32_t first, uint32_t count) {

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bvh_build.h"
+#include "node.h"
 
 namespace rtx {
 
@@ -25,19 +26,22 @@ __device__ __forceinline__ void set_comp(float4& v, int j, float x) {
     if (j == 0) v.x = x; else if (j == 1) v.y = x; else if (j == 2) v.z = x; else v.w = x;
 }
 
-// bottom-level tree copied to node index node_base / triangle index tri_base
-__global__ void k_relocate(float4* __restrict__ nodes, uint32_t n, uint32_t node_base, uint32_t tri_base) {
+// bottom-level tree copied to node index node_base / triangle index tri_base,
+// its planes at the scene's scale
+__global__ void k_relocate(float4* __restrict__ nodes, uint32_t n, uint32_t node_base, uint32_t tri_base,
+                           float plane_factor) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4* o = nodes + (size_t)kWideNodeF4 * (node_base + i);
-    float4 rf = o[6];
+    if (plane_factor != 1.f) rescale_node(o, plane_factor);
+    float4 rf = o[kNodeRefs];
     for (int j = 0; j < 4; j++) {
         uint32_t r = __float_as_uint(comp(rf, j));
         if (r & kLeafFlag) r += tri_base;           // first triangle (bits 0..26; the host checks the range)
         else if (r != kNoChild) r += node_base;
         set_comp(rf, j, __uint_as_float(r));
     }
-    o[6] = rf;
+    o[kNodeRefs] = rf;
 }
 
 // top-level tree: leaf k (one primitive, order[k]) holds instance
@@ -47,7 +51,7 @@ __global__ void k_tlas_leaves(float4* __restrict__ nodes, uint32_t n, const uint
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4* o = nodes + (size_t)kWideNodeF4 * i;
-    float4 rf = o[6];
+    float4 rf = o[kNodeRefs];
     for (int j = 0; j < 4; j++) {
         const uint32_t r = __float_as_uint(comp(rf, j));
         if (!(r & kLeafFlag)) continue;
@@ -55,55 +59,51 @@ __global__ void k_tlas_leaves(float4* __restrict__ nodes, uint32_t n, const uint
         const uint32_t id = first < nprim ? inst_of[order[first]] : null_inst;
         set_comp(rf, j, __uint_as_float(kInstLeaf | id));
     }
-    o[6] = rf;
+    o[kNodeRefs] = rf;
 }
 
 // one level of the top-level refit: each child slot gets the instance's world
-// box (ibox: lo, hi per instance) or the union of the inner child's slots
-// (refit before, one level deeper); slots of the null instance keep its box
-// and are left out of unions
+// box (ibox: lo, hi per instance) or the inner child's own box (tbox: lo, hi
+// per top-level node, written here one level deeper before); slots of the null
+// instance stay empty
 __global__ void k_refit4(float4* __restrict__ nodes, uint32_t begin, uint32_t n, const float4* __restrict__ ibox,
-                         uint32_t null_ref) {
+                         float4* __restrict__ tbox, uint32_t null_ref, float plane_scale) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4* o = nodes + (size_t)kWideNodeF4 * (begin + i);
-    const float4 rf = o[6];
-    float4 lx = rf, hx = rf, ly = rf, hy = rf, lz = rf, hz = rf;   // every component is set below
+    const float4 rf = o[kNodeRefs];
+    float lo[4][3], hi[4][3], bl[3], bh[3];
+    bool used[4];
+    uint32_t ref[4];
+    for (int k = 0; k < 3; k++) { bl[k] = __builtin_huge_valf(); bh[k] = -__builtin_huge_valf(); }
     for (int j = 0; j < 4; j++) {
         const uint32_t r = __float_as_uint(comp(rf, j));
-        float bl[3], bh[3];
-        if ((r & kInstLeaf) == kInstLeaf) {
-            const uint32_t id = r & kLeafFirstMask;
-            const float4 a = ibox[2 * (size_t)id], b = ibox[2 * (size_t)id + 1];
-            bl[0] = a.x; bl[1] = a.y; bl[2] = a.z;
-            bh[0] = b.x; bh[1] = b.y; bh[2] = b.z;
-        } else {
-            const float4* c = nodes + (size_t)kWideNodeF4 * r;
-            const float4 cl[3] = {c[0], c[2], c[4]}, ch[3] = {c[1], c[3], c[5]};
-            const float4 crf = c[6];
-            for (int k = 0; k < 3; k++) { bl[k] = __builtin_huge_valf(); bh[k] = -__builtin_huge_valf(); }
-            for (int q = 0; q < 4; q++) {
-                if (__float_as_uint(comp(crf, q)) == null_ref) continue;
-                for (int k = 0; k < 3; k++) {
-                    bl[k] = fminf(bl[k], comp(cl[k], q));
-                    bh[k] = fmaxf(bh[k], comp(ch[k], q));
-                }
-            }
+        ref[j] = r;
+        used[j] = r != null_ref;
+        const float4* b = (r & kInstLeaf) == kInstLeaf ? ibox + 2 * (size_t)(r & kLeafFirstMask) : tbox + 2 * (size_t)r;
+        const float4 a = b[0], c = b[1];
+        lo[j][0] = a.x; lo[j][1] = a.y; lo[j][2] = a.z;
+        hi[j][0] = c.x; hi[j][1] = c.y; hi[j][2] = c.z;
+        if (!used[j]) continue;
+        for (int k = 0; k < 3; k++) {
+            bl[k] = fminf(bl[k], lo[j][k]);
+            bh[k] = fmaxf(bh[k], hi[j][k]);
         }
-        set_comp(lx, j, bl[0]); set_comp(hx, j, bh[0]);
-        set_comp(ly, j, bl[1]); set_comp(hy, j, bh[1]);
-        set_comp(lz, j, bl[2]); set_comp(hz, j, bh[2]);
     }
-    o[0] = lx; o[1] = hx; o[2] = ly; o[3] = hy; o[4] = lz; o[5] = hz;
+    encode_node(o, lo, hi, used, ref, plane_scale);
+    tbox[2 * (size_t)(begin + i)] = make_float4(bl[0], bl[1], bl[2], 0.f);
+    tbox[2 * (size_t)(begin + i) + 1] = make_float4(bh[0], bh[1], bh[2], 0.f);
 }
 
 inline uint32_t blocks256(uint32_t n) { return (n + 255u) / 256u; }
 
 }  // namespace
 
-hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, hipStream_t s) {
+hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, float plane_factor,
+                         hipStream_t s) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_relocate, dim3(blocks256(n)), dim3(256), 0, s, nodes, n, node_base, tri_base);
+    hipLaunchKernelGGL(k_relocate, dim3(blocks256(n)), dim3(256), 0, s, nodes, n, node_base, tri_base,
+                       plane_factor);
     return hipGetLastError();
 }
 
@@ -115,13 +115,14 @@ hipError_t tlas_leaves(float4* nodes, uint32_t n, const uint32_t* order, uint32_
     return hipGetLastError();
 }
 
-hipError_t refit_tlas(float4* nodes, const std::vector<uint32_t>& level_begin, const float4* ibox, uint32_t null_ref,
-                      hipStream_t s) {
+hipError_t refit_tlas(float4* nodes, const std::vector<uint32_t>& level_begin, const float4* ibox, float4* tbox,
+                      uint32_t null_ref, float plane_scale, hipStream_t s) {
     // level_begin: first node of each level, then the node count
     for (size_t l = level_begin.size(); l-- > 1;) {
         const uint32_t b = level_begin[l - 1], n = level_begin[l] - b;
         if (n == 0) continue;
-        hipLaunchKernelGGL(k_refit4, dim3(blocks256(n)), dim3(256), 0, s, nodes, b, n, ibox, null_ref);
+        hipLaunchKernelGGL(k_refit4, dim3(blocks256(n)), dim3(256), 0, s, nodes, b, n, ibox, tbox, null_ref,
+                           plane_scale);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -3,7 +3,7 @@
 //
 // Software traversal of the 4-wide BVH (layout in rtx_internal.h) with a
 // per-lane stack whose first SLDS entries live in LDS (one column per lane,
-// bank-conflict free) and the rest in a global overflow area.  A step pushes
+// bank-conflict free) and the rest in a global overflow area (LaneStack).  A step pushes
 // at most 3 entries per level, so the stack holds at most 3 x (wide-tree
 // depth) entries; the launch sizes the overflow area for that.
 //
@@ -30,12 +30,36 @@
 
 namespace rtx {
 
-// slab test pad on the far distance: 1 + 2*gamma(3) (Ize 2013), conservative
-constexpr float kBoxPad = 1.0000004f;
+// Two forms of the slab test.
+//
+// Flat scenes (REL): slab distances are in units of the best hit so far (tau =
+// (t - tmin) / T, T the best hit's t, TRay::inv), so the clamp of the FMAs to
+// [0, 1] takes the place of a maximum with tmin and a minimum with the hit per
+// child: a box is met where entry < exit, and one beyond the hit or behind
+// tmin has both clamped to the same end.  kSlabPad: how far c = (origin - o) * inv - tmin / T is moved out (down for
+// entry planes, up for exit planes), relative to itself: 2^-20, where its two
+// roundings and the FMA's are within 3 * 2^-24 of the larger of c and the
+// distance (the planes' own margin covers what is relative to their distance
+// from the origin, node.h).
+constexpr float kSlabPad = 0x1p-20f;
+// kHitBias: a new hit makes T this much larger than its t, for the roundings
+// of the rescaling and of hits at equal distance
+constexpr float kHitBias = 1.f - 0x1p-20f;
+// T stays in this range (a smaller hit culls like one at the low end)
+constexpr float kLeastT = 1e-9f, kMostT = 1e30f;
+// Two-level scenes: distances are in units of t, clamped by maximum and
+// minimum, with the pad on the far distance: 2^-18, where the roundings of an
+// entry and an exit distance are together within 2^-20 of the distance (the
+// planes' own margin covers the rest).  Eight more instructions per visit, but
+// the two-level kernels have no registers for the rescaling (17 spilled; the
+// 1080p mixed-level frame 101.7 ms against 105.7 ms).
+constexpr float kBoxPad = 1.0000038f;
 
 struct TRay {
-    float3 o, d, idir;
+    float3 o, d;
+    float3 inv;     // 1 / (d * T); REL false: 1 / d
     float tmin;
+    float stmin;    // REL: tmin / T, a little less
     // the watertight test's axis order (kx, ky, kz) as a rotation that puts
     // the dominant axis kz last (rz0: kz = x, rz1: kz = y, else kz = z).
     // Woop et al. (2013) also swap kx and ky when d[kz] < 0 to keep the
@@ -43,16 +67,9 @@ struct TRay {
     // for bit the same, and nothing here depends on the winding
     bool rz0, rz1;
     float Sx, Sy, Sz;
-    // byte offsets, inside a 4-wide node, of the child planes the ray enters
-    // through on each axis (lo when the direction component is >= 0, else
-    // hi); the exit planes are at offset ^ 16
+    // byte offsets, inside a 4-wide node, of each axis's planes in the order
+    // the ray meets them: entry planes, then exit planes
     uint32_t nx, ny, nz;
-    // for slab distances as one FMA per plane, P * idir - c: c = o * idir
-    // moved by s = 2^-22 |o * idir| (down for entry planes, up for exit
-    // planes), which covers the roundings of o * idir and of c +- s, so
-    // an entry distance never comes out above (P - o) * idir rounded
-    // once, nor an exit distance below it
-    float3 ce, cx;
 };
 
 
@@ -64,7 +81,10 @@ __device__ __forceinline__ float3 permute(const TRay& r, float3 a) {
     return f3(p, q, w);
 }
 
-__device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmin) {
+__device__ __forceinline__ float tray_T(float t) { return fminf(fmaxf(t, kLeastT), kMostT); }
+
+template <bool REL>
+__device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmin, float tmax) {
     r.o = o;
     r.d = d;
     r.tmin = tmin;
@@ -74,20 +94,29 @@ __device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmi
     r.rz0 = kz == 0;
     r.rz1 = kz == 1;
     const float3 dp = permute(r, d);       // (d[kx], d[ky], d[kz])
-    r.idir = f3(1.f / (d.x != 0.f ? d.x : 1e-30f), 1.f / (d.y != 0.f ? d.y : 1e-30f),
-                1.f / (d.z != 0.f ? d.z : 1e-30f));
+    const float3 idir = f3(1.f / (d.x != 0.f ? d.x : 1e-24f), 1.f / (d.y != 0.f ? d.y : 1e-24f),
+                           1.f / (d.z != 0.f ? d.z : 1e-24f));
     // Sz = 1 / d[kz]: that is idir[kz] unless d is the zero vector
-    const float iz = r.rz0 ? r.idir.x : (r.rz1 ? r.idir.y : r.idir.z);
+    const float iz = r.rz0 ? idir.x : (r.rz1 ? idir.y : idir.z);
     r.Sz = dz != 0.f ? iz : __builtin_copysignf(__builtin_inff(), dz);
     r.Sx = dp.x * r.Sz;                     // shear by the reciprocal: no division of its own
     r.Sy = dp.y * r.Sz;
-    r.nx = r.idir.x >= 0.f ? 0u : 16u;
-    r.ny = r.idir.y >= 0.f ? 32u : 48u;
-    r.nz = r.idir.z >= 0.f ? 64u : 80u;
-    const float3 c = f3(o.x * r.idir.x, o.y * r.idir.y, o.z * r.idir.z);
-    const float3 sl = f3(fabsf(c.x) * 0x1p-22f, fabsf(c.y) * 0x1p-22f, fabsf(c.z) * 0x1p-22f);
-    r.ce = f3(c.x + sl.x, c.y + sl.y, c.z + sl.z);
-    r.cx = f3(c.x - sl.x, c.y - sl.y, c.z - sl.z);
+    r.nx = kNodePlanes[0] + (idir.x >= 0.f ? 0u : 8u);
+    r.ny = kNodePlanes[1] + (idir.y >= 0.f ? 0u : 8u);
+    r.nz = kNodePlanes[2] + (idir.z >= 0.f ? 0u : 8u);
+    const float f = REL ? 1.f / tray_T(tmax) : 1.f;
+    r.inv = REL ? f * idir : idir;
+    // (a little early, for the rounding of (origin - o) * inv where tmin / T cancels it)
+    r.stmin = REL ? f * (tmin - fabsf(tmin) * kSlabPad) : 0.f;
+}
+
+// the best hit moved from told to tnew (the ray's T with it)
+template <bool REL>
+__device__ __forceinline__ void tray_rescale(TRay& r, float told, float tnew) {
+    if (!REL) return;
+    const float f = (tray_T(told) * kHitBias) * __builtin_amdgcn_rcpf(tray_T(tnew));
+    r.inv = f * r.inv;
+    r.stmin = f * r.stmin;
 }
 
 // true with t > tmin and barycentrics (u,v) of v1 and v2 on a hit
@@ -134,32 +163,75 @@ __device__ __forceinline__ float4 lld4(const char __attribute__((address_space(3
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
+// an axis's planes of a node (16 B at a multiple of 8) as halves
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float rtx_f4a8 __attribute__((ext_vector_type(4), aligned(8)));
+template <bool G>
+__device__ __forceinline__ half8 ld_planes(const char* p) {
+    if constexpr (G) return __builtin_bit_cast(half8, (rtx_f4v)*(const RTX_GLOBAL rtx_f4a8*)p);
+    else return __builtin_bit_cast(half8, (rtx_f4v)*(const rtx_f4a8*)p);
+}
+__device__ __forceinline__ half8 lld_planes(const char __attribute__((address_space(3)))* p) {
+    return __builtin_bit_cast(half8, (rtx_f4v)*(const rtx_f4a8 __attribute__((address_space(3)))*)p);
+}
+
+// the address of an LDS pointer
+__device__ __forceinline__ uint32_t lds_addr(const lds_u32* p) { return (uint32_t)(uintptr_t)p; }
+
+// The traversal stack of a lane: a column of SLDS + 1 LDS slots, BLOCK words
+// apart, and an overflow column in global memory.  Slot 0 holds kNoChild for
+// good, entry i >= 1 is slot i, and the entries above SLDS are in global
+// memory.  The stack pointer is the LDS address of the top slot (past the
+// column once the top entry is in global memory; only its slot number is used
+// then), so a push or pop in LDS needs no address arithmetic beyond moving the
+// pointer, and popping an empty stack gives kNoChild without a test.
 template <int BLOCK, int SLDS = kStackLDS>
 struct LaneStack {
-    lds_u32* lds;      // LDS column of this lane: entry i at lds[i * BLOCK]
-    uint32_t* glob;    // overflow column: entry i at glob[(i - SLDS) * gstride]
+    static constexpr uint32_t kRowBytes = 4u * BLOCK;
+    lds_u32* bottom;   // slot 0 of this lane: the pointer of the empty stack
+    uint32_t fast;     // with the pointer at or below this, three pushes stay in LDS
+    uint32_t* glob;    // overflow column: slot i at glob[(i - SLDS - 1) * gstride]
     uint32_t gstride;
-    __device__ __forceinline__ void push(int& sp, uint32_t v) {
-        if (sp < SLDS) lds[sp * BLOCK] = v;
-        else glob[(size_t)(sp - SLDS) * gstride] = v;
-        sp++;
+    // s_stack: (SLDS + 1) * BLOCK words of LDS
+    __device__ __forceinline__ void init(uint32_t* s_stack, uint32_t* glob_column, uint32_t stride) {
+        lds_u32* row0 = (lds_u32*)s_stack;
+        bottom = row0 + threadIdx.x;
+        fast = lds_addr(row0) + (SLDS - 3) * kRowBytes + (kRowBytes - 1u);
+        glob = glob_column;
+        gstride = stride;
+        *bottom = kNoChild;
     }
-    __device__ __forceinline__ uint32_t pop(int& sp) {
-        sp--;
-        uint32_t v;
-        if (sp < SLDS) v = lds[sp * BLOCK];
-        else v = glob[(size_t)(sp - SLDS) * gstride];
+    __device__ __forceinline__ uint32_t slot(const lds_u32* sp) const {
+        return (lds_addr(sp) - lds_addr(bottom)) / kRowBytes;
+    }
+    // whether slot sp is in LDS
+    __device__ __forceinline__ bool in_lds(const lds_u32* sp) const { return lds_addr(sp) <= fast + 3u * kRowBytes; }
+    __device__ __forceinline__ void put(lds_u32* sp, uint32_t v) {
+        if (in_lds(sp)) *sp = v;
+        else glob[(size_t)(slot(sp) - SLDS - 1) * gstride] = v;
+    }
+    // the entry at sp (the top one; kNoChild at the bottom)
+    __device__ __forceinline__ uint32_t peek(const lds_u32* sp) const {
+        if (in_lds(sp)) return *sp;
+        return glob[(size_t)(slot(sp) - SLDS - 1) * gstride];
+    }
+    __device__ __forceinline__ void push(lds_u32*& sp, uint32_t v) {
+        sp += BLOCK;
+        put(sp, v);
+    }
+    __device__ __forceinline__ uint32_t pop(lds_u32*& sp) {
+        const uint32_t v = peek(sp);
+        sp -= BLOCK;
         return v;
     }
     // pushes v[0..N-1] (v[N-1] ends on top) with one range check when all N
     // slots are in LDS
     template <int N>
-    __device__ __forceinline__ void push_n(int& sp, const uint32_t (&v)[N]) {
-        if (sp + N <= SLDS) {
-            lds_u32* p = lds + sp * BLOCK;
+    __device__ __forceinline__ void push_n(lds_u32*& sp, const uint32_t (&v)[N]) {
+        if (in_lds(sp + N * BLOCK)) {
 #pragma unroll
-            for (int i = 0; i < N; i++) p[i * BLOCK] = v[i];
-            sp += N;
+            for (int i = 0; i < N; i++) sp[(i + 1) * BLOCK] = v[i];
+            sp += N * BLOCK;
         } else {
 #pragma unroll
             for (int i = 0; i < N; i++) push(sp, v[i]);
@@ -167,54 +239,40 @@ struct LaneStack {
     }
     // pops N entries into v[0..N-1] (v[N-1] is the old top), the inverse of push_n
     template <int N>
-    __device__ __forceinline__ void pop_n(int& sp, uint32_t (&v)[N]) {
-        if (sp <= SLDS) {
-            sp -= N;
-            const lds_u32* p = lds + sp * BLOCK;
+    __device__ __forceinline__ void pop_n(lds_u32*& sp, uint32_t (&v)[N]) {
+        if (in_lds(sp)) {
+            sp -= N * BLOCK;
 #pragma unroll
-            for (int i = 0; i < N; i++) v[i] = p[i * BLOCK];
+            for (int i = 0; i < N; i++) v[i] = sp[(i + 1) * BLOCK];
         } else {
 #pragma unroll
             for (int i = N - 1; i >= 0; i--) v[i] = pop(sp);
         }
     }
-    // writes slot sp (the free slot above the top) without pushing
-    __device__ __forceinline__ void put(int sp, uint32_t v) {
-        if (sp < SLDS) lds[sp * BLOCK] = v;
-        else glob[(size_t)(sp - SLDS) * gstride] = v;
-    }
-    // reads the top entry (slot sp-1; slot 0 when empty, value unused then)
-    __device__ __forceinline__ uint32_t peek(int sp) {
-        const int i = sp > 0 ? sp - 1 : 0;
-        if (i < SLDS) return lds[i * BLOCK];
-        return glob[(size_t)(i - SLDS) * gstride];
-    }
-    // One node step: returns the top entry (slot sp-1) and writes the hit
-    // children r1..r3 of a sorted 4-wide node above it, farthest lowest:
-    // child j (j = 1..nhit-1) goes to slot sp + nhit-1-j.  When every slot
-    // the step touches (sp-1 .. sp+2) is in LDS, the writes are unconditional
-    // and a child that is not pushed goes to the free slot sp+2 instead.
-    __device__ __forceinline__ uint32_t step4(int sp, int nhit, uint32_t r1, uint32_t r2, uint32_t r3) {
-        if (sp + 3 <= SLDS) {
-            const uint32_t top = lds[(sp > 0 ? sp - 1 : 0) * BLOCK];
-            // slot addresses from one base: r1's slot, then one and two
-            // slots below it; a child not pushed goes to the free slot sp+2
-            // (a base below the column is never selected: p1 is chosen only
-            // for hit children, whose slots are >= sp)
-            lds_u32* const p1 = lds + (sp + nhit - 2) * BLOCK;
-            lds_u32* const fr = lds + (sp + 2) * BLOCK;
-            lds_u32* const a3 = nhit > 3 ? p1 - 2 * BLOCK : fr;
-            lds_u32* const a2 = nhit > 2 ? p1 - BLOCK : fr;
-            lds_u32* const a1 = nhit > 1 ? p1 : fr;
-            *a3 = r3;
-            *a2 = r2;
-            *a1 = r1;
-            return top;
+    // One node step: pushes the hit ones of children 1..3 of a sorted 4-wide
+    // node (h1..h3; the hit children come first, so h3 implies h2 implies h1),
+    // the farthest first, and returns the old top entry.  In LDS every child
+    // is written, to the slot above a pointer that moves only past hit ones: a
+    // child that is not hit is overwritten by the next or stays above the top.
+    __device__ __forceinline__ uint32_t step4(lds_u32*& sp, bool h1, bool h2, bool h3, uint32_t r1, uint32_t r2,
+                                              uint32_t r3) {
+        lds_u32* a = sp;
+        uint32_t top;
+        if (lds_addr(a) <= fast) {
+            top = *a;
+            a[BLOCK] = r3;
+            a += h3 ? BLOCK : 0;
+            a[BLOCK] = r2;
+            a += h2 ? BLOCK : 0;
+            a[BLOCK] = r1;
+            a += h1 ? BLOCK : 0;
+        } else {
+            top = peek(a);
+            if (h3) push(a, r3);
+            if (h2) push(a, r2);
+            if (h1) push(a, r1);
         }
-        const uint32_t top = peek(sp);
-        if (nhit > 1) put(sp + nhit - 2, r1);
-        if (nhit > 2) put(sp + nhit - 3, r2);
-        if (nhit > 3) put(sp, r3);
+        sp = a;
         return top;
     }
 };
@@ -223,12 +281,36 @@ __device__ __forceinline__ float comp4(const float4& v, int j) {
     return j == 0 ? v.x : (j == 1 ? v.y : (j == 2 ? v.z : v.w));
 }
 
-// compare-exchange of (key, ref) pairs: smaller key first
-__device__ __forceinline__ void sort_ce(float& ka, uint32_t& ra, float& kb, uint32_t& rb) {
-    const bool sw = kb < ka;
-    const float k0 = sw ? kb : ka, k1 = sw ? ka : kb;
-    const uint32_t r0 = sw ? rb : ra, r1 = sw ? ra : rb;
-    ka = k0; kb = k1; ra = r0; rb = r1;
+// the distance of a plane, half * ds + c (one v_fma_mix_f32), and the same
+// clamped to [0, 1]
+__device__ __forceinline__ float slab(_Float16 h, float ds, float c) { return __builtin_fmaf((float)h, ds, c); }
+__device__ __forceinline__ float slab01(_Float16 h, float ds, float c) {
+    return __builtin_amdgcn_fmed3f(slab(h, ds, c), 0.f, 1.f);
+}
+
+// A child of a node step as one double, the entry distance's bits above the
+// ref's: doubles order by their high word first, so one v_min_f64 and one
+// v_max_f64 exchange a pair where two 32-bit words take a compare and four
+// selects, and a 64-bit minimum issues at the rate of a 32-bit one (measured:
+// 4.7 against 4.3 clocks per wave and SIMD, 4.4 for a select).  A float's
+// infinity, the distance of a child that is not hit, is an ordinary number
+// there (exponent 0x7F8), and a distance is never NaN.
+__device__ __forceinline__ double child_key(float t, uint32_t ref) {
+    return __builtin_bit_cast(double, ((uint64_t)__float_as_uint(t) << 32) | ref);
+}
+__device__ __forceinline__ uint32_t key_ref(double k) { return (uint32_t)__builtin_bit_cast(uint64_t, k); }
+__device__ __forceinline__ bool key_hit(double k) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(f2v, k).y < __builtin_inff();
+}
+// compare-exchange: smaller key first (as instructions, since fmin on doubles
+// would quiet its operands first)
+__device__ __forceinline__ void sort_ce(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
 }
 
 struct HitFull {
@@ -246,11 +328,11 @@ struct Trav {
     uint32_t node;    // next node to visit (kNoChild: none left)
     uint32_t leaf;    // a leaf found but not tested yet (kNoChild: none)
     uint32_t leaf2;   // a second one (set only while leaf is)
-    int sp;
+    lds_u32* sp;      // stack pointer (LaneStack)
     uint32_t inst;    // two-level scenes: the instance the lane is in (kNoHit: top level)
 };
 
-__device__ __forceinline__ void trav_reset(Trav& s, const DevScene& sc, float tmax) {
+__device__ __forceinline__ void trav_reset(Trav& s, const DevScene& sc, lds_u32* bottom, float tmax) {
     s.h.t = tmax;
     s.h.u = s.h.v = 0.f;
     s.h.tri = kNoHit;
@@ -259,13 +341,15 @@ __device__ __forceinline__ void trav_reset(Trav& s, const DevScene& sc, float tm
     s.node = sc.root;
     s.leaf = kNoChild;
     s.leaf2 = kNoChild;
-    s.sp = 0;
+    s.sp = bottom;
     s.inst = kNoHit;
 }
 
-__device__ __forceinline__ void trav_begin(Trav& s, const DevScene& sc, float3 o, float3 d, float tmin, float tmax) {
-    tray_init(s.r, o, d, tmin);
-    trav_reset(s, sc, tmax);
+template <bool TL>
+__device__ __forceinline__ void trav_begin(Trav& s, const DevScene& sc, lds_u32* bottom, float3 o, float3 d, float tmin,
+                                           float tmax) {
+    tray_init<!TL>(s.r, o, d, tmin, tmax);
+    trav_reset(s, sc, bottom, tmax);
 }
 
 // row . (p, 1) and row . (v, 0) of a 3x4 transform, one rounding per operation
@@ -303,7 +387,7 @@ __device__ __forceinline__ void inst_step(const DevScene& sc, Trav& s, bool goin
         o = f3(__uint_as_float(w[0]), __uint_as_float(w[1]), __uint_as_float(w[2]));
         d = f3(__uint_as_float(w[3]), __uint_as_float(w[4]), __uint_as_float(w[5]));
         s.inst = kNoHit;
-        s.node = s.sp == 0 ? kNoChild : st.pop(s.sp);
+        s.node = st.pop(s.sp);
     }
     const bool enter = going && (s.node & kInstLeaf) == kInstLeaf;
     if (enter) {
@@ -319,7 +403,7 @@ __device__ __forceinline__ void inst_step(const DevScene& sc, Trav& s, bool goin
         s.inst = id;
         s.node = __float_as_uint(m.x);
     }
-    if (leave || enter) tray_init(s.r, o, d, s.r.tmin);
+    if (leave || enter) tray_init<false>(s.r, o, d, s.r.tmin, s.h.t);
 }
 
 // first active lane of the wave (counts wave-level loop iterations in COUNT mode)
@@ -473,6 +557,7 @@ __device__ __forceinline__ void leaves_compact(const DevScene& sc, Trav& s, uint
             const uint32_t prim = (uint32_t)kk;
             const bool lower = TL ? (s.inst < s.h.inst || (s.inst == s.h.inst && prim < s.h.prim)) : prim < s.h.prim;
             if (t < s.h.t || (t == s.h.t && lower)) {
+                tray_rescale<!TL>(s.r, s.h.t, t);
                 s.h.t = t;
                 s.h.u = bu;
                 s.h.v = bv;
@@ -501,17 +586,14 @@ __device__ __forceinline__ void leaves_compact(const DevScene& sc, Trav& s, uint
 // least `batch` of the wave's `busy` lanes have finished, so that the caller
 // can shade them while the others keep their state and resume later.
 // COUNT adds node-visit and triangle-test counts (statistics launches only).
-// FMA selects the slab form: one FMA per plane with the per-ray offsets
-// (fewer instructions), or (P - o) * idir (six fewer registers, for kernels
-// that are short of them).
 // TOPN > 0: the first TOPN nodes of the node array (the top levels: the
 // array is breadth-first) are read from a copy in LDS at `top` instead of
 // global memory.
 // CL: the leaf phase spreads the parked leaves' triangles over the wave
 // (leaves_compact, with the wave's kLeafScratchWords of LDS at `cl`);
 // otherwise each lane tests its own leaves.
-template <int BLOCK, bool COUNT = false, bool TL = false, bool FMA = true, bool G = false, int TOPN = 0,
-          bool CL = false, class Stack>
+template <int BLOCK, bool COUNT = false, bool TL = false, bool G = false, int TOPN = 0, bool CL = false,
+          class Stack>
 __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& going, bool busy, int batch,
                                          int inner_frac, Stack& st, uint32_t* nn = nullptr,
                                          uint32_t* nt = nullptr, uint32_t* wi = nullptr,
@@ -521,7 +603,12 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
         // node phase (no lane starts or stops going in it)
         const uint64_t m_going = __ballot(going);
         const uint32_t n_going = (uint32_t)__popcll(m_going);
-        for (;;) {
+        // (one scalar condition ends the loop and guards its step, and the step
+        // is a block at its end: the loop's branch is then a scalar one, with
+        // no mask of lanes that left; 2 % on every frame)
+        const uint32_t least = n_going ? ((uint32_t)inner_frac * n_going + 63u) >> 6 : 1u;
+        bool step;
+        do {
             if (TL) {
                 // Instance transitions: leave a finished instance (not while
                 // one of its leaves is parked), then enter the instance the
@@ -543,102 +630,98 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
                 (s.leaf == kNoChild || s.leaf2 == kNoChild)) {
                 if (s.leaf == kNoChild) s.leaf = s.node;
                 else s.leaf2 = s.node;
-                s.node = s.sp == 0 ? kNoChild : st.pop(s.sp);
+                s.node = st.pop(s.sp);
             }
             // no leaf flag, not kNoChild (nor the instance marker): one unsigned
             // compare, balloted as it is and masked with the going lanes
             const bool below = s.node < (TL ? kInstMarker : kNoChild);
             const bool inner = going && below;
             const uint32_t n_inner = (uint32_t)__popcll(__ballot(below) & m_going);
-            if (n_inner == 0) break;
-            if (n_inner * 64u < (uint32_t)inner_frac * n_going) break;
-            // the node step as a block, not behind a `continue`: every exit of
-            // this loop is then wave-uniform (the two breaks above), and the
-            // loop's control stays in scalar registers (2-3 % faster frames)
-            if (inner) {
+            step = n_inner >= least;
+            if (inner && step) {
                 if (COUNT) {
                     (*nn)++;
                     if (first_active_lane()) wi[0]++;
                 }
-                // one 4-wide node: six float4 of child bounds (SoA: lo.x, hi.x,
-                // lo.y, hi.y, lo.z, hi.z) + one of refs.  The ray loads each
-                // axis's entry and exit planes by its direction signs, so the
-                // slab test needs no min/max per axis.
+                // one 4-wide node: five loads.  The ray reads each axis's
+                // entry and exit planes by its direction signs, so the slab
+                // test needs no min/max per axis; the halves go into the FMAs
+                // as they are (v_fma_mix_f32).
                 // (32-bit byte offsets: the builder keeps the node array below 4 GiB)
-                typedef const float4 cf4;
-                const char* nb = (const char*)sc.nodes;
                 const uint32_t no = s.node * (16u * kWideNodeF4);
                 const TRay& r = s.r;
-                float4 ex, fx, ey, fy, ez, fz, rf;
+                half8 px, py, pz;
+                float4 og, rf;
                 if (TOPN > 0 && s.node < (uint32_t)TOPN) {
                     typedef const char __attribute__((address_space(3))) lchar;
                     lchar* lb = (lchar*)top;
-                    ex = lld4(lb + (no + r.nx));
-                    fx = lld4(lb + (no + (r.nx ^ 16u)));
-                    ey = lld4(lb + (no + r.ny));
-                    fy = lld4(lb + (no + (r.ny ^ 16u)));
-                    ez = lld4(lb + (no + r.nz));
-                    fz = lld4(lb + (no + (r.nz ^ 16u)));
-                    rf = lld4(lb + (no + 96u));
+                    px = lld_planes(lb + (no + r.nx));
+                    py = lld_planes(lb + (no + r.ny));
+                    pz = lld_planes(lb + (no + r.nz));
+                    og = lld4(lb + (no + 16u * kNodeOrigin));
+                    rf = lld4(lb + (no + 16u * kNodeRefs));
                 } else {
-                    ex = ld4<G>((cf4*)(nb + (no + r.nx)));
-                    fx = ld4<G>((cf4*)(nb + (no + (r.nx ^ 16u))));
-                    ey = ld4<G>((cf4*)(nb + (no + r.ny)));
-                    fy = ld4<G>((cf4*)(nb + (no + (r.ny ^ 16u))));
-                    ez = ld4<G>((cf4*)(nb + (no + r.nz)));
-                    fz = ld4<G>((cf4*)(nb + (no + (r.nz ^ 16u))));
-                    rf = ld4<G>((cf4*)(nb + (no + 96u)));
+                    typedef const float4 cf4;
+                    const char* nb = (const char*)sc.nodes;
+                    px = ld_planes<G>(nb + (no + r.nx));
+                    py = ld_planes<G>(nb + (no + r.ny));
+                    pz = ld_planes<G>(nb + (no + r.nz));
+                    og = ld4<G>((cf4*)(nb + (no + 16u * kNodeOrigin)));
+                    rf = ld4<G>((cf4*)(nb + (no + 16u * kNodeRefs)));
                 }
-                float key[4];
-                uint32_t ref[4];
-                int nhit = 0;
+                // all five in flight before the first is waited for (the
+                // compiler would hold some back to reuse registers: the
+                // 1080p mixed-level frame 109 ms without, 102 ms with)
+                __builtin_amdgcn_sched_barrier(0);
+                const float3 ds = f3(sc.plane_scale * r.inv.x, sc.plane_scale * r.inv.y, sc.plane_scale * r.inv.z);
+                const float3 oo = f3(og.x - r.o.x, og.y - r.o.y, og.z - r.o.z);
+                double key[4];
+                if (!TL) {
+                    const float3 c = f3(__builtin_fmaf(oo.x, r.inv.x, -r.stmin), __builtin_fmaf(oo.y, r.inv.y, -r.stmin),
+                                        __builtin_fmaf(oo.z, r.inv.z, -r.stmin));
+                    const float3 ce = f3(__builtin_fmaf(fabsf(c.x), -kSlabPad, c.x),
+                                         __builtin_fmaf(fabsf(c.y), -kSlabPad, c.y),
+                                         __builtin_fmaf(fabsf(c.z), -kSlabPad, c.z));
+                    const float3 cx = f3(__builtin_fmaf(fabsf(c.x), kSlabPad, c.x),
+                                         __builtin_fmaf(fabsf(c.y), kSlabPad, c.y),
+                                         __builtin_fmaf(fabsf(c.z), kSlabPad, c.z));
     #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    float x0, x1, y0, y1, z0, z1;
-                    if (FMA) {
-                        x0 = __builtin_fmaf(comp4(ex, j), r.idir.x, -r.ce.x);
-                        x1 = __builtin_fmaf(comp4(fx, j), r.idir.x, -r.cx.x);
-                        y0 = __builtin_fmaf(comp4(ey, j), r.idir.y, -r.ce.y);
-                        y1 = __builtin_fmaf(comp4(fy, j), r.idir.y, -r.cx.y);
-                        z0 = __builtin_fmaf(comp4(ez, j), r.idir.z, -r.ce.z);
-                        z1 = __builtin_fmaf(comp4(fz, j), r.idir.z, -r.cx.z);
-                    } else {
-                        x0 = (comp4(ex, j) - r.o.x) * r.idir.x;
-                        x1 = (comp4(fx, j) - r.o.x) * r.idir.x;
-                        y0 = (comp4(ey, j) - r.o.y) * r.idir.y;
-                        y1 = (comp4(fy, j) - r.o.y) * r.idir.y;
-                        z0 = (comp4(ez, j) - r.o.z) * r.idir.z;
-                        z1 = (comp4(fz, j) - r.o.z) * r.idir.z;
+                    for (int j = 0; j < 4; j++) {
+                        const float x0 = slab01(px[j], ds.x, ce.x), x1 = slab01(px[4 + j], ds.x, cx.x);
+                        const float y0 = slab01(py[j], ds.y, ce.y), y1 = slab01(py[4 + j], ds.y, cx.y);
+                        const float z0 = slab01(pz[j], ds.z, ce.z), z1 = slab01(pz[4 + j], ds.z, cx.z);
+                        const float tn = fmaxf(fmaxf(x0, y0), z0);
+                        const float tf = fminf(fminf(x1, y1), z1);
+                        key[j] = child_key(tn < tf ? tn : __builtin_inff(), __float_as_uint(comp4(rf, j)));
                     }
-                    const float tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
-                    const float tf = fminf(fminf(x1, y1), fminf(z1, s.h.t));
-                    // empty slots hold a point box at 1e38 that no slab test accepts
-                    const uint32_t c = __float_as_uint(comp4(rf, j));
-                    const bool hit = tn <= tf * kBoxPad;
-                    key[j] = hit ? tn : __uint_as_float(0x7F800000u);
-                    ref[j] = c;
-                    nhit += hit ? 1 : 0;
+                } else {
+                    const float3 c = f3(oo.x * r.inv.x, oo.y * r.inv.y, oo.z * r.inv.z);
+    #pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float x0 = slab(px[j], ds.x, c.x), x1 = slab(px[4 + j], ds.x, c.x);
+                        const float y0 = slab(py[j], ds.y, c.y), y1 = slab(py[4 + j], ds.y, c.y);
+                        const float z0 = slab(pz[j], ds.z, c.z), z1 = slab(pz[4 + j], ds.z, c.z);
+                        const float tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
+                        const float tf = fminf(fminf(x1, y1), fminf(z1, s.h.t));
+                        key[j] = child_key(tn <= tf * kBoxPad ? tn : __builtin_inff(), __float_as_uint(comp4(rf, j)));
+                    }
                 }
                 // ascending by entry distance (misses last): 5 compare-exchanges
-                sort_ce(key[0], ref[0], key[1], ref[1]);
-                sort_ce(key[2], ref[2], key[3], ref[3]);
-                sort_ce(key[0], ref[0], key[2], ref[2]);
-                sort_ce(key[1], ref[1], key[3], ref[3]);
-                sort_ce(key[1], ref[1], key[2], ref[2]);
-                // visit the nearest; push the others farthest first (slot
-                // sp + nhit-1-j for child j), so the next nearest is on top.
-                // With no hit the top of the stack is next (read before any
-                // write: the writes go to slots >= sp).
-                const uint32_t top = st.step4(s.sp, nhit, ref[1], ref[2], ref[3]);
-                if (nhit == 0) {
-                    s.node = s.sp == 0 ? kNoChild : top;
-                    s.sp = s.sp > 0 ? s.sp - 1 : 0;
-                } else {
-                    s.sp += nhit - 1;
-                    s.node = ref[0];
-                }
+                sort_ce(key[0], key[1]);
+                sort_ce(key[2], key[3]);
+                sort_ce(key[0], key[2]);
+                sort_ce(key[1], key[3]);
+                sort_ce(key[1], key[2]);
+                // visit the nearest; push the others farthest first, so the
+                // next nearest is on top.  With no hit the top of the stack
+                // (kNoChild when it is empty) is next.
+                const uint32_t top = st.step4(s.sp, key_hit(key[1]), key_hit(key[2]), key_hit(key[3]),
+                                              key_ref(key[1]), key_ref(key[2]), key_ref(key[3]));
+                const bool any = key_hit(key[0]);
+                s.node = any ? key_ref(key[0]) : top;
+                s.sp -= any ? 0 : BLOCK;
             }
-        }
+        } while (step);
         // leaf phase (compacted when the whole wave is here)
         if (CL && __builtin_amdgcn_read_exec() == ~0ull) {
             uint32_t f1 = 0, c1 = 0, f2 = 0, c2 = 0;
@@ -680,6 +763,7 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
                     const bool lower = TL ? (s.inst < s.h.inst || (s.inst == s.h.inst && prim < s.h.prim))
                                           : prim < s.h.prim;
                     if (tt < s.h.t || (tt == s.h.t && lower)) {
+                        tray_rescale<!TL>(s.r, s.h.t, tt);
                         s.h.t = tt;
                         s.h.u = uu;
                         s.h.v = vv;
@@ -709,7 +793,7 @@ template <int BLOCK, bool TL = false, class Stack>
 __device__ __forceinline__ void traverse(const DevScene& sc, const TRay& r, float tmax, HitFull& h, Stack& st) {
     Trav s;
     s.r = r;
-    trav_reset(s, sc, tmax);
+    trav_reset(s, sc, st.bottom, tmax);
     bool going = true;
     trav_run<BLOCK, false, TL>(sc, s, going, true, 64, 32, st);
     h = s.h;
