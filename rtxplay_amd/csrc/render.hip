@@ -22,6 +22,7 @@
 // multiplies them on the way down (same factors, other association).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 
 #include "kernels.h"
@@ -51,6 +52,8 @@ struct RenderArgs {
     uint32_t batch;       // lanes that must finish a ray before a wave shades (64: whole wave)
     uint32_t inner_frac;  // node phase ends below inner_frac/64 of the going lanes
     uint32_t tile_log2w;  // tile width = 1 << tile_log2w, tile height = 64 / width
+    uint32_t lanes;       // lanes of a wave that take pixels (64 but for spread frames)
+    uint32_t spread;      // spread frames: tile slots between the pixels of neighbouring lanes, else 0
     TraceCounters tc;
     // adjoint launch only
     const rtx_float3* dldi;   // dL/d rawRGB per pixel
@@ -168,7 +171,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
     for (;;) {
         // lanes without a pixel take one; tile slots outside the frame are skipped
         for (;;) {
-            const bool need = !active && !exhausted;
+            const bool need = !active && !exhausted && lane < a.lanes;
             const uint64_t mask = __ballot(need);
             if (mask == 0) break;
             const uint32_t leader = __ffsll((unsigned long long)mask) - 1;
@@ -188,7 +191,11 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
                         spp = J->lp.spp;
                         maxd = J->lp.depth;
                     }
-                    const uint32_t li = wi - J->work_begin;
+                    uint32_t li = wi - J->work_begin;
+                    if (!BATCH && a.spread) {
+                        li = (wi % a.lanes) * a.spread + wi / a.lanes;
+                        if (li >= J->work_end) continue;   // (the last lane's share may be shorter)
+                    }
                     const uint32_t in = li & 63u;
                     const uint32_t tile = !BATCH && a.tile_order ? a.tile_order[li >> 6] : li >> 6;
                     if (PROBE) tslot = li >> 6;
@@ -694,6 +701,7 @@ RenderArgs base_args(const LaunchScratch& ls) {
     a.inner_frac = ls.inner_frac ? ls.inner_frac : 36u;
     a.tile_log2w = log2u(ls.tile_w ? ls.tile_w : 8u);
     a.iterative = ls.iterative;
+    a.lanes = 64u;
     return a;
 }
 
@@ -760,6 +768,32 @@ void order_tiles(RenderArgs& a, const LaunchScratch& ls, hipStream_t s) {
 }
 }  // namespace
 
+namespace {
+// A frame of fewer than two pixels per lane of the persistent grid is bound by
+// its most expensive pixels, whose samples are traced one after the other, not
+// by the chip: a lane alone in its wave takes 0.54 us per node visit, one of a
+// full wave 1.2 us.  So such a frame is spread over the waves: the lanes of a
+// wave take pixels from all over the frame (`spread` slots apart) instead of
+// one tile, so that the expensive pixels, which lie together, do not share
+// waves, and only as many lanes of each wave take one as half the grid's waves
+// need.  The wave's shading batch shrinks with its lanes.  Measured (level 4,
+// 400x225, 10 spp: 3.96 -> 2.95 ms; level 3, 320x180, 64 spp: 19.8 -> 14.6 ms;
+// mixed levels, two-level, 400x225, 10 spp: 8.0 -> 5.5 ms; level 4, 896x504,
+// 8 and 64 spp: 4.65 -> 3.87 and 31.9 -> 25.9 ms; 640x360, 1 spp: 0.627 ->
+// 0.641 ms).  With two pixels per lane and more the waves stay full, and
+// neighbouring rays share cache lines (1100x640 and 1280x720 at 8 and 4 spp:
+// 2 % slower spread); those of 16+ spp go longest first (kOrderMinSpp).
+void spread_pixels(RenderArgs& a, const LaunchScratch& ls) {
+    const uint32_t waves = ls.grid * (kRenderBlock / 64u);
+    if (a.tile_order || a.nwork >= kOrderMinPixelsPerLane * waves * 64u) return;
+    const uint32_t half = (waves + 1u) / 2u;
+    a.lanes = std::min(64u, (a.nwork + half - 1u) / half);
+    a.spread = (a.nwork + a.lanes - 1u) / a.lanes;
+    a.nwork = a.spread * a.lanes;
+    if (a.batch < 64u) a.batch = std::max(1u, (a.batch * a.lanes + 63u) / 64u);
+}
+}  // namespace
+
 hipError_t launch_render(const DevScene& sc, const rtx_lp_general& lp, float3 ambient, const LaunchScratch& ls,
                          hipStream_t s) {
     RenderArgs a = base_args(ls);
@@ -767,6 +801,7 @@ hipError_t launch_render(const DevScene& sc, const rtx_lp_general& lp, float3 am
     a.njobs = 1;
     a.nwork = a.job.work_end;
     order_tiles(a, ls, s);
+    spread_pixels(a, ls);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     return launch_frame<false>(a, ls, s);
 }
@@ -817,6 +852,7 @@ hipError_t launch_adjoint(const DevScene& sc, const rtx_lp_general& lp, float3 a
     const uint32_t ng = 4u * sc.num_insts;
     if (ng) hipLaunchKernelGGL(k_fill, dim3((ng + 255) / 256), dim3(256), 0, s, dparams, ng, 0.f);
     order_tiles(a, ls, s);
+    spread_pixels(a, ls);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     const size_t shm = a.lds_grad ? sizeof(float) * ng : 0;
     const dim3 g(ls.grid), b(kRenderBlock);
