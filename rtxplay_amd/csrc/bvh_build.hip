@@ -71,7 +71,7 @@ struct BNode {
 };
 
 struct BuildStats {
-    uint32_t leaves, max_depth, max_leaf, pad;
+    uint32_t max_leaf, pad;
     double sah;
 };
 
@@ -176,17 +176,43 @@ __global__ void k_iota(uint32_t* __restrict__ idx, uint32_t N) {
     if (p < N) idx[p] = p;
 }
 
+// inclusive scans over the 64 lanes of a wave (all of them active) in six DPP
+// steps: shifts by 1, 2, 4 and 8 within the 16-lane rows, then the rows' last
+// lanes broadcast to the rows above.  Lanes without a source keep their value.
+// (Shuffles go through LDS: the SAH decision of a 64-bin task took 290 of them.)
+template <class Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t none, Op op) {
+#define RTX_SCAN_STEP(ctrl, rows) \
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, ctrl, rows, 0xf, false))
+    RTX_SCAN_STEP(0x111, 0xf);   // row_shr:1
+    RTX_SCAN_STEP(0x112, 0xf);   // row_shr:2
+    RTX_SCAN_STEP(0x114, 0xf);   // row_shr:4
+    RTX_SCAN_STEP(0x118, 0xf);   // row_shr:8
+    RTX_SCAN_STEP(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+    RTX_SCAN_STEP(0x143, 0xc);   // row_bcast:31 into rows 2 and 3
+#undef RTX_SCAN_STEP
+    return v;
+}
+__device__ __forceinline__ uint32_t scan_add(uint32_t v) {
+    return wave_scan(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ float scan_min(float v) {
+    return __uint_as_float(wave_scan(__float_as_uint(v), __float_as_uint(FLT_MAX), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(fminf(__uint_as_float(a), __uint_as_float(b)));
+    }));
+}
+__device__ __forceinline__ float scan_max(float v) {
+    return __uint_as_float(wave_scan(__float_as_uint(v), __float_as_uint(-FLT_MAX), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b)));
+    }));
+}
+
 // block-wide exclusive scan of one value per thread; returns the prefix and
 // the block total.  `ws` holds one slot per wave plus one.
 template <int BLOCK>
 __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* ws, uint32_t& total) {
     const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= (uint32_t)off) x += y;
-    }
+    const uint32_t x = scan_add(v);
     if (lane == 63u) ws[wid] = x;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -306,7 +332,7 @@ __device__ __forceinline__ void bins_add(LevelLds& L, const TaskGeom& g, const u
 
 // SAH decision from the task's bins (every thread of the block calls it):
 // the first wave evaluates the splits, one lane per bin -- inclusive prefix
-// (bins 0..b) and suffix (bins b..63) bounds and counts by shuffles; min and
+// (bins 0..b) and suffix (bins b..63) bounds and counts by wave scans; min and
 // max are exact, so they equal a bin-by-bin sweep.  The split after bin b
 // costs area(prefix b) * count + area(suffix b+1) * count; the cheapest wins,
 // the lowest bin on ties (the order of a sweep with a strict <).  Thread 0
@@ -314,48 +340,34 @@ __device__ __forceinline__ void bins_add(LevelLds& L, const TaskGeom& g, const u
 __device__ __forceinline__ void sah_decide(LevelLds& L, const BuildTask& task, uint32_t n,
                                            BNode* __restrict__ bnodes, uint32_t max_leaf) {
     if (threadIdx.x < 64) {
-        const int b = (int)threadIdx.x;
+        const int b = (int)threadIdx.x, m = kBins - 1 - b;
         for (int ax = 0; ax < 3; ax++) {
-            const uint32_t cb = L.cnt[ax][b];
-            float pl[3], ph[3], sl[3], sh[3];
+            const uint32_t cb = L.cnt[ax][b], cm = L.cnt[ax][m];
+            // bins 0..b, and in lane b the bins 63-b..63 (a prefix of the mirrored bins)
+            float pl[3], ph[3], ml[3], mh[3];
             for (int k = 0; k < 3; k++) {
-                pl[k] = sl[k] = cb ? o2f(L.b[ax][b][k]) : FLT_MAX;
-                ph[k] = sh[k] = cb ? o2f(L.b[ax][b][3 + k]) : -FLT_MAX;
+                pl[k] = scan_min(cb ? o2f(L.b[ax][b][k]) : FLT_MAX);
+                ph[k] = scan_max(cb ? o2f(L.b[ax][b][3 + k]) : -FLT_MAX);
+                ml[k] = scan_min(cm ? o2f(L.b[ax][m][k]) : FLT_MAX);
+                mh[k] = scan_max(cm ? o2f(L.b[ax][m][3 + k]) : -FLT_MAX);
             }
-            uint32_t pc = cb, sc = cb;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const bool up = b >= off, dn = b + off < 64;
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    const float ul = __shfl_up(pl[k], off, 64), uh = __shfl_up(ph[k], off, 64);
-                    const float dl = __shfl_down(sl[k], off, 64), dh = __shfl_down(sh[k], off, 64);
-                    if (up) { pl[k] = fminf(pl[k], ul); ph[k] = fmaxf(ph[k], uh); }
-                    if (dn) { sl[k] = fminf(sl[k], dl); sh[k] = fmaxf(sh[k], dh); }
-                }
-                const uint32_t uc = __shfl_up(pc, off, 64), dc = __shfl_down(sc, off, 64);
-                if (up) pc += uc;
-                if (dn) sc += dc;
-            }
-            float rl[3], rh[3];
-#pragma unroll
-            for (int k = 0; k < 3; k++) { rl[k] = __shfl_down(sl[k], 1, 64); rh[k] = __shfl_down(sh[k], 1, 64); }
-            const uint32_t rc0 = __shfl_down(sc, 1, 64);
+            const uint32_t pc = scan_add(cb), mc = scan_add(cm);
+            // the suffix from bin b + 1 on is lane 62 - b's
+            const float mt = area3(ml[0], ml[1], ml[2], mh[0], mh[1], mh[2]) * (float)mc;
+            const int from = (kBins - 2 - b) & 63;
+            const float rt = __shfl(mt, from, 64);
+            const uint32_t rc0 = __shfl(mc, from, 64);
             const uint32_t rc = b < kBins - 1 ? rc0 : 0u;
-            const float cost = area3(pl[0], pl[1], pl[2], ph[0], ph[1], ph[2]) * (float)pc +
-                               area3(rl[0], rl[1], rl[2], rh[0], rh[1], rh[2]) * (float)rc;
+            const float cost = area3(pl[0], pl[1], pl[2], ph[0], ph[1], ph[2]) * (float)pc + rt;
             const bool valid = b < kBins - 1 && pc != 0 && rc != 0 && cost < FLT_MAX;
-            // costs are >= 0, so their bits order like their values
-            uint64_t key = valid ? ((uint64_t)__float_as_uint(cost) << 32) | (uint32_t)b : ~0ull;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const uint64_t o = __shfl_xor(key, off, 64);
-                key = o < key ? o : key;
-            }
+            // the least cost, its lowest bin
+            const float least = __uint_as_float(
+                (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(scan_min(valid ? cost : FLT_MAX)), 63));
+            const uint64_t at = __ballot(valid && cost == least);
             L.pcnt[ax][b] = pc;
             if (b == 0) {
-                L.best_cost[ax] = key == ~0ull ? FLT_MAX : __uint_as_float((uint32_t)(key >> 32));
-                L.best_bin[ax] = key == ~0ull ? -1 : (int)(uint32_t)key;
+                L.best_cost[ax] = least;
+                L.best_bin[ax] = __ffsll((unsigned long long)at) - 1;
             }
             if (ax == 0 && b == kBins - 1) {
                 // node bounds: the union of the axis-0 bins
@@ -413,16 +425,13 @@ __device__ __forceinline__ void split_out(const LevelLds& L, const BuildTask& ta
                 v[9 + k] = has && !left ? hi : -FLT_MAX;
             }
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    v[k] = fminf(v[k], __shfl_xor(v[k], off, 64));
-                    v[3 + k] = fmaxf(v[3 + k], __shfl_xor(v[3 + k], off, 64));
-                    v[6 + k] = fminf(v[6 + k], __shfl_xor(v[6 + k], off, 64));
-                    v[9 + k] = fmaxf(v[9 + k], __shfl_xor(v[9 + k], off, 64));
-                }
+            for (int k = 0; k < 3; k++) {
+                v[k] = scan_min(v[k]);
+                v[3 + k] = scan_max(v[3 + k]);
+                v[6 + k] = scan_min(v[6 + k]);
+                v[9 + k] = scan_max(v[9 + k]);
             }
-            if (b == 0) {
+            if (b == kBins - 1) {   // the last lane's scans hold all bins
                 so.clo_l = make_float4(v[0], v[1], v[2], 0.f);
                 so.chi_l = make_float4(v[3], v[4], v[5], 0.f);
                 so.clo_r = make_float4(v[6], v[7], v[8], 0.f);
@@ -810,31 +819,18 @@ __global__ __launch_bounds__(BLOCK) void k_decide_wide(const BuildTask* __restri
     if (threadIdx.x == 0) wsplit[blockIdx.x] = make_uint4((uint32_t)L.kind, (uint32_t)L.axis, (uint32_t)L.bin, L.nleft);
 }
 
-// big tasks, step 3: primitives left of the split in each chunk
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_count_wide(const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
-                                                      const float4* __restrict__ phi, const uint32_t* __restrict__ idx,
-                                                      uint32_t G, const uint4* __restrict__ wsplit,
-                                                      uint32_t* __restrict__ lcount) {
-    __shared__ uint32_t s_n;
+// big tasks, step 3: primitives left of the split in each chunk, from the
+// chunk's own bins (a wave per chunk, a lane per bin; a pass over the
+// primitives took 0.12 ms per level of 8 M)
+__global__ __launch_bounds__(256) void k_count_wide(uint32_t G, const uint32_t* __restrict__ partial,
+                                                    const uint4* __restrict__ wsplit, uint32_t* __restrict__ lcount) {
+    const uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6), b = threadIdx.x & 63u;
     const uint4 w = wsplit[blockIdx.y];
-    if (w.x != 1u) return;   // the whole block: no SAH split
-    const BuildTask task = tasks[blockIdx.y];
-    const TaskGeom g = task_geom(task);
-    uint32_t r0, r1;
-    chunk_range(task, G, blockIdx.x, r0, r1);
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-    const int ax = (int)w.y, sb = (int)w.z;
-    uint32_t nl = 0;
-    for (uint32_t i = r0 + threadIdx.x; i < r1; i += BLOCK) {
-        const uint32_t p = idx[i];
-        const float4 a = plo[p], h = phi[p];
-        if (bin_of(.5f * (comp4(a, ax) + comp4(h, ax)), g.cl[ax], g.scale[ax]) <= sb) nl++;
-    }
-    atomicAdd(&s_n, nl);
-    __syncthreads();
-    if (threadIdx.x == 0) lcount[blockIdx.y * G + blockIdx.x] = s_n;
+    if (w.x != 1u || c >= G) return;   // the whole wave: no SAH split, or past the last chunk
+    const size_t chunk = (size_t)blockIdx.y * G + c;
+    uint32_t n = b <= w.z ? partial[chunk * kPartialWords + w.y * kBins + b] : 0u;
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (b == 0) lcount[chunk] = n;
 }
 
 // big tasks, step 4: each chunk partitions stably into tmp after the left
@@ -852,11 +848,11 @@ __global__ __launch_bounds__(BLOCK) void k_scatter_wide(const BuildTask* __restr
     const BuildTask task = tasks[blockIdx.y];
     uint32_t r0, r1;
     chunk_range(task, G, blockIdx.x, r0, r1);
-    if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (uint32_t k = 0; k < blockIdx.x; k++) s += lcount[blockIdx.y * G + k];
-        s_lb = s;
-    }
+    if (threadIdx.x == 0) s_lb = 0;
+    __syncthreads();
+    uint32_t before_me = 0;
+    for (uint32_t k = threadIdx.x; k < blockIdx.x; k += BLOCK) before_me += lcount[blockIdx.y * G + k];
+    if (before_me) atomicAdd(&s_lb, before_me);
     __syncthreads();
     const uint32_t lb = s_lb, before = r0 - task.begin;
     partition_range<BLOCK>(task_geom(task), (int)w.y, (int)w.z, idx, tmp, plo, phi, r0, r1, task.begin + lb,
@@ -930,78 +926,66 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(Get get, uint32_t n, 
 
 __global__ void k_emit(const BuildTask* __restrict__ tasks, const SplitOut* __restrict__ so,
                        const uint32_t* __restrict__ rank, uint32_t ntasks, uint32_t node_base,
-                       BNode* __restrict__ bnodes, BuildTask* __restrict__ next,
-                       BuildStats* __restrict__ st) {
+                       BNode* __restrict__ bnodes, BuildTask* __restrict__ next) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t leaf_depth = 0, leaf_n = 0;   // of a leaf, for the statistics
-    bool leaf = false;
-    if (i < ntasks) {
-        const BuildTask t = tasks[i];
-        const SplitOut s = so[i];
-        const uint32_t n = t.end - t.begin;
-        if (s.kind == 0) {
-            bnodes[t.node].lo.w = __uint_as_float(t.begin);
-            bnodes[t.node].hi.w = __uint_as_float(n);
-            leaf = true;
-            leaf_depth = t.depth + 1;
-            leaf_n = n;
-        } else {
-            const uint32_t L = node_base + 2 * rank[i];
-            bnodes[t.node].lo.w = __uint_as_float(L);
-            bnodes[t.node].hi.w = __uint_as_float(0u);
-            BuildTask a, b;
-            a.node = L; a.begin = t.begin; a.end = t.begin + s.nleft; a.depth = t.depth + 1;
-            a.clo = s.clo_l; a.chi = s.chi_l;
-            b.node = L + 1; b.begin = t.begin + s.nleft; b.end = t.end; b.depth = t.depth + 1;
-            b.clo = s.clo_r; b.chi = s.chi_r;
-            next[2 * rank[i]] = a;
-            next[2 * rank[i] + 1] = b;
-        }
+    if (i >= ntasks) return;
+    const BuildTask t = tasks[i];
+    const SplitOut s = so[i];
+    if (s.kind == 0) {
+        bnodes[t.node].lo.w = __uint_as_float(t.begin);
+        bnodes[t.node].hi.w = __uint_as_float(t.end - t.begin);
+        return;
     }
-    // leaf count, deepest leaf and largest leaf with one atomic each per wave
-    // (millions of leaves on one address otherwise serialise in L2)
-    const uint64_t m = __ballot(leaf);
-    if (m == 0) return;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        leaf_depth = max(leaf_depth, (uint32_t)__shfl_xor(leaf_depth, off, 64));
-        leaf_n = max(leaf_n, (uint32_t)__shfl_xor(leaf_n, off, 64));
-    }
-    if ((threadIdx.x & 63u) == (uint32_t)(__ffsll((unsigned long long)m) - 1)) {
-        atomicAdd(&st->leaves, (uint32_t)__popcll(m));
-        atomicMax(&st->max_depth, leaf_depth);
-        atomicMax(&st->max_leaf, leaf_n);
-    }
+    const uint32_t L = node_base + 2 * rank[i];
+    bnodes[t.node].lo.w = __uint_as_float(L);
+    bnodes[t.node].hi.w = __uint_as_float(0u);
+    BuildTask a, b;
+    a.node = L; a.begin = t.begin; a.end = t.begin + s.nleft; a.depth = t.depth + 1;
+    a.clo = s.clo_l; a.chi = s.chi_l;
+    b.node = L + 1; b.begin = t.begin + s.nleft; b.end = t.end; b.depth = t.depth + 1;
+    b.clo = s.clo_r; b.chi = s.chi_r;
+    next[2 * rank[i]] = a;
+    next[2 * rank[i] + 1] = b;
 }
 
-// SAH cost of the finished tree (relative to the root area)
-// SAH cost of the binary tree (statistics): grid-strided partial sums, a wave
-// reduction, then one atomic per block (the order of the double sums varies
-// from run to run in the last bits)
+// SAH cost (relative to the root area) and largest leaf of the finished binary
+// tree (statistics): grid-strided partial sums, a wave reduction, then one
+// atomic per block (the order of the double sums varies from run to run in the
+// last bits).  The counts of leaves and inner nodes and the depth follow from
+// the counts of nodes and levels: every inner node has two children, and the
+// last level holds only leaves.
 constexpr uint32_t kSahBlocks = 1024;
 __global__ __launch_bounds__(256) void k_sah(const BNode* __restrict__ bnodes, uint32_t nnodes,
                                              BuildStats* __restrict__ st) {
     __shared__ double s_v[256 / 64];
+    __shared__ uint32_t s_m[256 / 64];
     double v = 0.0;
+    uint32_t most = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nnodes; i += gridDim.x * blockDim.x) {
         const BNode nd = bnodes[i];
         const float a = area3(nd.lo.x, nd.lo.y, nd.lo.z, nd.hi.x, nd.hi.y, nd.hi.z);
         const uint32_t cnt = __float_as_uint(nd.hi.w);
         v += cnt ? (double)kCostIsect * cnt * a : (double)kCostTrav * a;
+        most = max(most, cnt);
     }
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    if ((threadIdx.x & 63) == 0) s_v[threadIdx.x >> 6] = v;
+    for (int off = 32; off > 0; off >>= 1) {
+        v += __shfl_down(v, off, 64);
+        most = max(most, (uint32_t)__shfl_down(most, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_v[threadIdx.x >> 6] = v;
+        s_m[threadIdx.x >> 6] = most;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.0;
-        for (int w = 0; w < 256 / 64; w++) t += s_v[w];
+        for (int w = 0; w < 256 / 64; w++) {
+            t += s_v[w];
+            most = max(most, s_m[w]);
+        }
         if (t != 0.0) atomicAdd(&st->sah, t);
+        if (most) atomicMax(&st->max_leaf, most);
     }
-}
-
-__global__ void k_inner_flag(const BNode* __restrict__ bnodes, uint32_t nnodes, SplitOut* __restrict__ flag) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nnodes) flag[i].kind = __float_as_uint(bnodes[i].hi.w) == 0u ? 1u : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -1351,8 +1335,8 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
                                merged.p);
             hipLaunchKernelGGL(k_decide_wide<kBuildBlock>, dim3(ntasks), dim3(kBuildBlock), 0, s, cur, 1u, merged.p,
                                bnodes.p, so.p, wsplit.p, max_leaf);
-            hipLaunchKernelGGL(k_count_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, cur, d_plo, d_phi, idx.p, G,
-                               wsplit.p, lcount.p);
+            hipLaunchKernelGGL(k_count_wide, dim3((G + 3) / 4, ntasks), dim3(256), 0, s, G, partial.p, wsplit.p,
+                               lcount.p);
             hipLaunchKernelGGL(k_scatter_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, cur, d_plo, d_phi, idx.p,
                                tmp.p, G, wsplit.p, lcount.p);
             hipLaunchKernelGGL(k_copy_wide, gw, dim3(256), 0, s, cur, G, wsplit.p, tmp.p, idx.p);
@@ -1370,7 +1354,7 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
                                tmp.p, bnodes.p, so.p, max_leaf);
         scan_kind(ntasks);
         hipLaunchKernelGGL(k_emit, dim3(blocks_for(ntasks, 256)), dim3(256), 0, s, cur, so.p, rank.p, ntasks,
-                           nnodes, bnodes.p, nxt, st.p);
+                           nnodes, bnodes.p, nxt);
         RTX_TRY(hipGetLastError());
         uint32_t nsplit = 0;
         RTX_TRY(hipMemcpyAsync(&nsplit, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -1382,13 +1366,9 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
 
     hipLaunchKernelGGL(k_sah, dim3(std::min(blocks_for(nnodes, 256), kSahBlocks)), dim3(256), 0, s, bnodes.p, nnodes,
                        st.p);
-    // compact inner nodes into the traversal layout (BFS order of the build)
-    hipLaunchKernelGGL(k_inner_flag, dim3(blocks_for(nnodes, 256)), dim3(256), 0, s, bnodes.p, nnodes, so.p);
-    scan_kind(nnodes);
     RTX_TRY(hipGetLastError());
-    uint32_t ninner = 0;
+    const uint32_t ninner = (nnodes - 1) / 2;
     BuildStats hst;
-    RTX_TRY(hipMemcpyAsync(&ninner, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     RTX_TRY(hipMemcpyAsync(&hst, st.p, sizeof(BuildStats), hipMemcpyDeviceToHost, s));
     BNode root;
     RTX_TRY(hipMemcpyAsync(&root, bnodes.p, sizeof(BNode), hipMemcpyDeviceToHost, s));
@@ -1486,8 +1466,8 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
     out.num_nodes = ninner;
     out.num_wide = nwide;
     out.wide_depth = wide_depth;
-    out.num_leaves = hst.leaves;
-    out.max_depth = hst.max_depth;
+    out.num_leaves = nnodes - ninner;
+    out.max_depth = (uint32_t)level_first.size() - 1;
     out.max_leaf = hst.max_leaf;
     out.sah = root_area > 0.0 ? hst.sah / root_area : 0.0;
     *outp = out;
