@@ -42,8 +42,51 @@ struct BuiltBVH {
 
 struct BvhOptions {
     uint32_t max_leaf = kMaxLeaf;   // primitives per leaf at most (1..kMaxLeaf)
-    bool gather = true;             // write the leaf-ordered triangles (else return the leaf order)
+    bool gather = true;             // write the leaf-ordered triangles (else return the leaf order; not with owned)
+    bool owned = true;              // the result's arrays are allocations of their own (else parts of the workspace)
 };
+
+// Device memory of one build: a block that the builds of a device share (one
+// at a time; a build that finds it taken by another thread has its own) and
+// what does not fit it as allocations of their own, freed with the lease.
+// Allocating and freeing the temporaries took 7.5 ms of the 28 ms of the
+// 8M-triangle level-6 scene and 9 of 18 ms of the mixed two-level one (now,
+// with the levels launched ahead, 21.5 and 8.0 ms, host to host).  The
+// block is kept between builds up to kKeepBytes and freed with the device's
+// last context (build_workspace_drop).  A build ends with its stream
+// synchronized, so the next one may use the block on any stream.
+class BuildWorkspace {
+public:
+    static constexpr size_t kKeepBytes = (size_t)4 << 30;
+    // for a build that takes `bytes` at once at most (with that device current)
+    BuildWorkspace(int device, size_t bytes);
+    ~BuildWorkspace();
+    BuildWorkspace(const BuildWorkspace&) = delete;
+    BuildWorkspace& operator=(const BuildWorkspace&) = delete;
+    template <class T>
+    hipError_t get(T** p, size_t n) { return take((void**)p, sizeof(T) * (n ? n : 1)); }
+    size_t mark() const { return used_; }
+    void reset(size_t m) { used_ = m; }       // gives back what was taken since mark()
+    // kHostWords words of pinned host memory that kernels write counts to
+    static constexpr uint32_t kHostWords = 1024;
+    hipError_t host_words(uint32_t** h);
+    // the build's stream has been synchronized after its last use of the memory
+    void done() { done_ = true; }
+
+private:
+    hipError_t take(void** p, size_t bytes);
+    int device_;
+    bool shared_ = false, done_ = false;
+    uint8_t* base_ = nullptr;
+    uint32_t* host_ = nullptr;
+    size_t cap_ = 0, used_ = 0;
+    std::vector<void*> more_;
+};
+void build_workspace_drop(int device);
+// the workspace bytes that build_bvh over N primitives usually takes (what
+// goes beyond is allocated then) and that its result takes when not owned
+size_t bvh_workspace_bytes(uint32_t N);
+size_t bvh_result_bytes(uint32_t N);
 
 // world-space triangles (3 float4 each: xyz | prim id, inst id, mesh prim) and
 // per-primitive bounds, in instance-major order
@@ -53,7 +96,8 @@ hipError_t flatten_scene(const InstBuild* d_insts, uint32_t ninst, const MeshRef
 // binned SAH BVH over N flattened triangles; synchronous on s
 // (without gather, d_tri_world is not read and may be null)
 hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float4* d_phi, uint32_t N,
-                     hipStream_t s, BuiltBVH* out, std::string* err, const BvhOptions& opt = BvhOptions());
+                     hipStream_t s, BuildWorkspace& ws, BuiltBVH* out, std::string* err,
+                     const BvhOptions& opt = BvhOptions());
 
 // ---- two-level scenes (tlas.hip) ----
 // adds node_base / tri_base to the refs of a bottom-level tree of n wide

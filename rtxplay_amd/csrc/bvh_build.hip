@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -74,6 +75,15 @@ struct BuildStats {
     uint32_t max_leaf, pad;
     double sah;
 };
+
+// One level of the binary tree (tasks) or of the 4-wide tree (nodes): how many
+// and the index of the first.  The counts stay on the device: the kernels of a
+// level read theirs, and a level's scan writes the next one's (and its count
+// to the host, which runs a level ahead with grids for the most there can be).
+struct Level {
+    uint32_t n, first;
+};
+constexpr uint32_t kMaxLevels = 128;   // levels held at once (a deeper tree wraps round)
 
 __device__ __forceinline__ uint32_t f2o(float f) {
     uint32_t u = __float_as_uint(f);
@@ -140,8 +150,15 @@ __global__ void k_flatten(const InstBuild* __restrict__ insts, uint32_t ninst,
 // root task: centroid bounds of all primitives as ordered ints (minima of x,
 // y, z, then maxima), reduced per block and merged across blocks by atomics;
 // min and max are exact, so the result does not depend on their order
-__global__ void k_root_init(uint32_t* __restrict__ rb) {
+__global__ void k_root_init(uint32_t* __restrict__ rb, BuildStats* __restrict__ st, Level* __restrict__ lev,
+                            Level* __restrict__ wlev) {
     if (threadIdx.x < 6) rb[threadIdx.x] = threadIdx.x < 3 ? 0xFFFFFFFFu : 0u;
+    if (threadIdx.x == 0) {
+        st->max_leaf = 0u;
+        st->sah = 0.0;
+        lev->n = wlev->n = 1u;
+        lev->first = wlev->first = 0u;
+    }
 }
 __global__ __launch_bounds__(256) void k_root_bounds(const float4* __restrict__ plo, const float4* __restrict__ phi,
                                                      uint32_t N, uint32_t* __restrict__ rb) {
@@ -170,6 +187,11 @@ __global__ void k_root_task(const uint32_t* __restrict__ rb, uint32_t N, BuildTa
     t.chi = make_float4(o2f(rb[3]), o2f(rb[4]), o2f(rb[5]), 0.f);
     *task = t;
 }
+
+// lev[0] takes lev[kMaxLevels]'s place: levels kMaxLevels and up use the array again
+__global__ void k_level_wrap(Level* lev) { lev[0] = lev[kMaxLevels]; }
+
+__global__ void k_zero_word(uint32_t* p) { *p = 0u; }
 
 __global__ void k_iota(uint32_t* __restrict__ idx, uint32_t N) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -511,11 +533,12 @@ __device__ __forceinline__ void level_task(LevelLds& L, uint32_t* s_ws, const Bu
 // one block per task
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_level(
-        const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
+        const Level* __restrict__ lev, const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
         const float4* __restrict__ phi, uint32_t* __restrict__ idx, uint32_t* __restrict__ tmp,
         BNode* __restrict__ bnodes, SplitOut* __restrict__ out, uint32_t max_leaf) {
     __shared__ LevelLds L;
     __shared__ uint32_t s_ws[BLOCK / 64 + 1];
+    if (blockIdx.x >= lev->n) return;
     level_task<BLOCK>(L, s_ws, tasks[blockIdx.x], blockIdx.x, plo, phi, idx, tmp, bnodes, out, max_leaf);
 }
 
@@ -687,7 +710,7 @@ __device__ void tiny_task(const BuildTask& task, uint32_t slot, const float4* __
 // a thread per task; tasks above kTinyTask primitives are appended to `big`
 // (one atomic per wave: their order in the list does not matter, each task
 // writes only its own slot and primitive range)
-__global__ __launch_bounds__(256) void k_level_tiny(const BuildTask* __restrict__ tasks, uint32_t ntasks,
+__global__ __launch_bounds__(256) void k_level_tiny(const Level* __restrict__ lev, const BuildTask* __restrict__ tasks,
                                                     const float4* __restrict__ plo, const float4* __restrict__ phi,
                                                     uint32_t* __restrict__ idx, uint32_t* __restrict__ tmp,
                                                     BNode* __restrict__ bnodes, SplitOut* __restrict__ out,
@@ -695,7 +718,7 @@ __global__ __launch_bounds__(256) void k_level_tiny(const BuildTask* __restrict_
                                                     uint32_t* __restrict__ nbig) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     bool is_big = false;
-    if (t < ntasks) {
+    if (t < lev->n) {
         const BuildTask task = tasks[t];
         if (task.end - task.begin > kTinyTask) is_big = true;
         else tiny_task(task, t, plo, phi, idx, tmp, bnodes, out, max_leaf);
@@ -738,10 +761,12 @@ __device__ __forceinline__ void chunk_range(const BuildTask& task, uint32_t G, u
 }
 
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_bin_wide(const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
+__global__ __launch_bounds__(BLOCK) void k_bin_wide(const Level* __restrict__ lev,
+                                                    const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
                                                     const float4* __restrict__ phi, const uint32_t* __restrict__ idx,
                                                     uint32_t G, uint32_t* __restrict__ partial) {
     __shared__ LevelLds L;
+    if (blockIdx.y >= lev->n) return;
     const BuildTask task = tasks[blockIdx.y];
     uint32_t r0, r1;
     chunk_range(task, G, blockIdx.x, r0, r1);
@@ -762,9 +787,11 @@ __global__ __launch_bounds__(BLOCK) void k_bin_wide(const BuildTask* __restrict_
 // threads each reduce every 16th chunk, then the first group the groups.
 constexpr uint32_t kMergeWords = 16;
 static_assert(kPartialWords % kMergeWords == 0, "whole blocks of merged words");
-__global__ __launch_bounds__(256) void k_merge_wide(uint32_t G, const uint32_t* __restrict__ partial,
+__global__ __launch_bounds__(256) void k_merge_wide(const Level* __restrict__ lev,
+                                                    uint32_t G, const uint32_t* __restrict__ partial,
                                                     uint32_t* __restrict__ merged) {
     __shared__ uint32_t s_v[256 / kMergeWords][kMergeWords + 1];
+    if (blockIdx.y >= lev->n) return;
     const uint32_t w = threadIdx.x % kMergeWords, grp = threadIdx.x / kMergeWords;
     const uint32_t i = blockIdx.x * kMergeWords + w;
     // word kind: 0 count (sum), 1 lower bound (min), 2 upper bound (max)
@@ -790,11 +817,13 @@ __global__ __launch_bounds__(256) void k_merge_wide(uint32_t G, const uint32_t* 
 // k_merge_wide), merges them and decides as k_level does; wsplit[t] = (kind,
 // axis, bin, nleft) for the partition
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_decide_wide(const BuildTask* __restrict__ tasks, uint32_t G,
+__global__ __launch_bounds__(BLOCK) void k_decide_wide(const Level* __restrict__ lev,
+                                                       const BuildTask* __restrict__ tasks, uint32_t G,
                                                        const uint32_t* __restrict__ partial,
                                                        BNode* __restrict__ bnodes, SplitOut* __restrict__ out,
                                                        uint4* __restrict__ wsplit, uint32_t max_leaf) {
     __shared__ LevelLds L;
+    if (blockIdx.x >= lev->n) return;
     const BuildTask task = tasks[blockIdx.x];
     const uint32_t* P = partial + (size_t)blockIdx.x * G * kPartialWords;
     uint32_t* c = &L.cnt[0][0];
@@ -822,9 +851,11 @@ __global__ __launch_bounds__(BLOCK) void k_decide_wide(const BuildTask* __restri
 // big tasks, step 3: primitives left of the split in each chunk, from the
 // chunk's own bins (a wave per chunk, a lane per bin; a pass over the
 // primitives took 0.12 ms per level of 8 M)
-__global__ __launch_bounds__(256) void k_count_wide(uint32_t G, const uint32_t* __restrict__ partial,
+__global__ __launch_bounds__(256) void k_count_wide(const Level* __restrict__ lev,
+                                                    uint32_t G, const uint32_t* __restrict__ partial,
                                                     const uint4* __restrict__ wsplit, uint32_t* __restrict__ lcount) {
     const uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6), b = threadIdx.x & 63u;
+    if (blockIdx.y >= lev->n) return;
     const uint4 w = wsplit[blockIdx.y];
     if (w.x != 1u || c >= G) return;   // the whole wave: no SAH split, or past the last chunk
     const size_t chunk = (size_t)blockIdx.y * G + c;
@@ -836,13 +867,16 @@ __global__ __launch_bounds__(256) void k_count_wide(uint32_t G, const uint32_t* 
 // big tasks, step 4: each chunk partitions stably into tmp after the left
 // and right primitives of the chunks before it
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_scatter_wide(const BuildTask* __restrict__ tasks, const float4* __restrict__ plo,
+__global__ __launch_bounds__(BLOCK) void k_scatter_wide(const Level* __restrict__ lev,
+                                                        const BuildTask* __restrict__ tasks,
+                                                        const float4* __restrict__ plo,
                                                         const float4* __restrict__ phi, const uint32_t* __restrict__ idx,
                                                         uint32_t* __restrict__ tmp, uint32_t G,
                                                         const uint4* __restrict__ wsplit,
                                                         const uint32_t* __restrict__ lcount) {
     __shared__ uint32_t s_ws[BLOCK / 64 + 1];
     __shared__ uint32_t s_lb;
+    if (blockIdx.y >= lev->n) return;
     const uint4 w = wsplit[blockIdx.y];
     if (w.x != 1u) return;
     const BuildTask task = tasks[blockIdx.y];
@@ -860,60 +894,93 @@ __global__ __launch_bounds__(BLOCK) void k_scatter_wide(const BuildTask* __restr
 }
 
 // big tasks, step 5: the partitioned ranges back into idx
-__global__ void k_copy_wide(const BuildTask* __restrict__ tasks, uint32_t G, const uint4* __restrict__ wsplit,
+__global__ void k_copy_wide(const Level* __restrict__ lev,
+                            const BuildTask* __restrict__ tasks, uint32_t G, const uint4* __restrict__ wsplit,
                             const uint32_t* __restrict__ tmp, uint32_t* __restrict__ idx) {
-    if (wsplit[blockIdx.y].x != 1u) return;
+    if (blockIdx.y >= lev->n || wsplit[blockIdx.y].x != 1u) return;
     uint32_t r0, r1;
     chunk_range(tasks[blockIdx.y], G, blockIdx.x, r0, r1);
     for (uint32_t i = r0 + threadIdx.x; i < r1; i += blockDim.x) idx[i] = tmp[i];
 }
 
-// single-block exclusive scan of `n` uints (kind flags) -> out, total -> *total
-__global__ __launch_bounds__(kScanBlock) void k_scan_kind(const SplitOut* __restrict__ so, uint32_t n,
-                                                         uint32_t* __restrict__ out, uint32_t* __restrict__ total) {
+// The values of a level to scan: its tasks' split flags (each split makes two
+// tasks) or its wide nodes' counts of inner children.
+struct KindOf {
+    const SplitOut* so;
+    static constexpr uint32_t kMakes = 2;
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return so[i].kind; }
+};
+struct CountOf {
+    const uint32_t* p;
+    static constexpr uint32_t kMakes = 1;
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return p[i]; }
+};
+// the next level, after lev[0], from the sum of a level's values
+__device__ __forceinline__ void level_next(Level* lev, uint32_t n, uint32_t* host) {
+    lev[1].n = n;
+    lev[1].first = lev[0].first + lev[0].n;
+    __hip_atomic_store(host, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// exclusive scan of a level's values by one block -> out; the next level
+template <class Get>
+__global__ __launch_bounds__(kScanBlock) void k_scan(Level* __restrict__ lev, Get get, uint32_t* __restrict__ out,
+                                                    uint32_t* __restrict__ host) {
     __shared__ uint32_t s_ws[kScanBlock / 64 + 1];
+    const uint32_t n = lev->n;
     uint32_t carry = 0;
     for (uint32_t base = 0; base < n; base += kScanBlock) {
         const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < n ? so[i].kind : 0u;
+        const uint32_t v = i < n ? get(i) : 0u;
         uint32_t tot;
         const uint32_t ex = block_scan<kScanBlock>(v, s_ws, tot);
         if (i < n) out[i] = carry + ex;
         carry += tot;
     }
-    if (threadIdx.x == 0) *total = carry;
+    if (threadIdx.x == 0) level_next(lev, Get::kMakes * carry, host);
 }
 
-// the same scan over many blocks, for long arrays: tile sums, a scan of
-// them (k_scan_u32), then each tile rescanned from its offset
+// the same scan over many blocks, for long levels: tile sums, a scan of
+// them by one block, then each tile rescanned from its offset
 constexpr uint32_t kScanTile = 4 * kScanBlock;
-// the values to scan: the split flags of a level, or plain counts
-struct KindOf {
-    const SplitOut* so;
-    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return so[i].kind; }
-};
-struct U32Of {
-    const uint32_t* p;
-    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return p[i]; }
-};
 template <class Get>
-__global__ __launch_bounds__(kScanBlock) void k_scan_tiles(Get get, uint32_t n, uint32_t* __restrict__ tsum) {
+__global__ __launch_bounds__(kScanBlock) void k_scan_tiles(const Level* __restrict__ lev, Get get,
+                                                          uint32_t* __restrict__ tsum) {
     __shared__ uint32_t s_n;
+    const uint32_t n = lev->n;
     if (threadIdx.x == 0) s_n = 0;
     __syncthreads();
     uint32_t c = 0;
     const uint32_t b0 = blockIdx.x * kScanTile;
     for (uint32_t i = b0 + threadIdx.x; i < n && i < b0 + kScanTile; i += kScanBlock) c += get(i);
-    atomicAdd(&s_n, c);
+    if (c) atomicAdd(&s_n, c);
     __syncthreads();
     if (threadIdx.x == 0) tsum[blockIdx.x] = s_n;
 }
+__global__ __launch_bounds__(kScanBlock) void k_scan_sums(Level* __restrict__ lev, uint32_t makes,
+                                                         const uint32_t* __restrict__ tsum,
+                                                         uint32_t* __restrict__ toff, uint32_t* __restrict__ host) {
+    __shared__ uint32_t s_ws[kScanBlock / 64 + 1];
+    const uint32_t nt = (lev->n + kScanTile - 1) / kScanTile;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < nt; base += kScanBlock) {
+        const uint32_t i = base + threadIdx.x;
+        const uint32_t v = i < nt ? tsum[i] : 0u;
+        uint32_t tot;
+        const uint32_t ex = block_scan<kScanBlock>(v, s_ws, tot);
+        if (i < nt) toff[i] = carry + ex;
+        carry += tot;
+    }
+    if (threadIdx.x == 0) level_next(lev, makes * carry, host);
+}
 template <class Get>
-__global__ __launch_bounds__(kScanBlock) void k_scan_apply(Get get, uint32_t n, const uint32_t* __restrict__ toff,
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const Level* __restrict__ lev, Get get,
+                                                          const uint32_t* __restrict__ toff,
                                                           uint32_t* __restrict__ out) {
     __shared__ uint32_t s_ws[kScanBlock / 64 + 1];
+    const uint32_t n = lev->n, b0 = blockIdx.x * kScanTile;
+    if (b0 >= n) return;
     uint32_t carry = toff[blockIdx.x];
-    const uint32_t b0 = blockIdx.x * kScanTile;
     for (uint32_t base = b0; base < b0 + kScanTile && base < n; base += kScanBlock) {
         const uint32_t i = base + threadIdx.x;
         const uint32_t v = i < n ? get(i) : 0u;
@@ -924,11 +991,13 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(Get get, uint32_t n, 
     }
 }
 
-__global__ void k_emit(const BuildTask* __restrict__ tasks, const SplitOut* __restrict__ so,
-                       const uint32_t* __restrict__ rank, uint32_t ntasks, uint32_t node_base,
-                       BNode* __restrict__ bnodes, BuildTask* __restrict__ next) {
+// (lev[1], the next level, is written by the scan before)
+__global__ void k_emit(const Level* __restrict__ lev, const BuildTask* __restrict__ tasks,
+                       const SplitOut* __restrict__ so, const uint32_t* __restrict__ rank, BNode* __restrict__ bnodes,
+                       BuildTask* __restrict__ next) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ntasks) return;
+    if (i >= lev[0].n) return;
+    const uint32_t node_base = lev[1].first;
     const BuildTask t = tasks[i];
     const SplitOut s = so[i];
     if (s.kind == 0) {
@@ -995,11 +1064,11 @@ __global__ __launch_bounds__(256) void k_sah(const BNode* __restrict__ bnodes, u
 // children and repeatedly opens the inner child of largest surface area until
 // it has 4 children or only leaves; its inner children become the wide nodes
 // of the next level.
-__global__ void k_collapse4(const BNode* __restrict__ bn, const uint32_t* __restrict__ front, uint32_t n,
-                            uint4* __restrict__ cid, uint32_t* __restrict__ ninner) {
+__global__ void k_collapse4(const Level* __restrict__ lev, const BNode* __restrict__ bn,
+                            const uint32_t* __restrict__ front, uint4* __restrict__ cid, uint32_t* __restrict__ ninner) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t L = __float_as_uint(bn[front[i]].lo.w);
+    if (i >= lev->n) return;
+    const uint32_t L = __float_as_uint(bn[front ? front[i] : 0u].lo.w);
     uint32_t c0 = L, c1 = L + 1, c2 = kNoChild, c3 = kNoChild;
     uint32_t cnt = 2;
     for (int it = 0; it < 2; it++) {
@@ -1102,12 +1171,12 @@ __global__ void k_dp_level(const BNode* __restrict__ bn, uint32_t begin, uint32_
 
 // the children of the wide node at binary node front[i]: the forest of 4
 // roots that the choices give under it (left subtree first)
-__global__ void k_collapse4_dp(const BNode* __restrict__ bn, const uint32_t* __restrict__ front, uint32_t n,
-                               const uint32_t* __restrict__ meta, uint4* __restrict__ cid,
-                               uint32_t* __restrict__ ninner) {
+__global__ void k_collapse4_dp(const Level* __restrict__ lev, const BNode* __restrict__ bn,
+                               const uint32_t* __restrict__ front, const uint32_t* __restrict__ meta,
+                               uint4* __restrict__ cid, uint32_t* __restrict__ ninner) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t b = front[i];
+    if (i >= lev->n) return;
+    const uint32_t b = front ? front[i] : 0u;   // the first level is the root alone
     const uint32_t L = __float_as_uint(bn[b].lo.w);
     const uint32_t kl = (meta[b] >> 1) & 3u;
     // (subtree, roots) pairs still to expand; their roots add up to 4, so
@@ -1138,13 +1207,14 @@ __global__ void k_collapse4_dp(const BNode* __restrict__ bn, const uint32_t* __r
 // Writes the wide nodes of one level.  With meta (the SAH-optimal collapse)
 // a child is a leaf when its subtree is one (primitives first[c] ..
 // first[c] + ntri[c] - 1 of the leaf order); without, when it is a binary leaf.
-__global__ void k_write4(const BNode* __restrict__ bn, const uint4* __restrict__ cid, const uint32_t* __restrict__ off,
-                         uint32_t n, uint32_t base_this, uint32_t base_next, uint32_t empty_ref,
-                         float4* __restrict__ nodes4, uint32_t* __restrict__ next_front,
-                         const uint32_t* __restrict__ meta, const uint32_t* __restrict__ ntri,
-                         const uint32_t* __restrict__ first, float plane_scale) {
+__global__ void k_write4(const Level* __restrict__ lev, const BNode* __restrict__ bn, const uint4* __restrict__ cid,
+                         const uint32_t* __restrict__ off, uint32_t empty_ref, float4* __restrict__ nodes4,
+                         uint32_t* __restrict__ next_front, const uint32_t* __restrict__ meta,
+                         const uint32_t* __restrict__ ntri, const uint32_t* __restrict__ first) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i >= lev[0].n) return;
+    const uint32_t base_this = lev[0].first, base_next = lev[1].first;
+    const float plane_scale = plane_scale_of(bn[0].lo, bn[0].hi);
     const uint4 c4 = cid[i];
     float lo[4][3], hi[4][3];
     bool used[4];
@@ -1177,22 +1247,6 @@ __global__ void k_write4(const BNode* __restrict__ bn, const uint4* __restrict__
         }
     }
     encode_node(nodes4 + kWideNodeF4 * (size_t)(base_this + i), lo, hi, used, ref, plane_scale);
-}
-
-// single-block exclusive scan of n uints -> out, total -> *total
-__global__ __launch_bounds__(kScanBlock) void k_scan_u32(const uint32_t* __restrict__ in, uint32_t n,
-                                                        uint32_t* __restrict__ out, uint32_t* __restrict__ total) {
-    __shared__ uint32_t s_ws[kScanBlock / 64 + 1];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < n; base += kScanBlock) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < n ? in[i] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_scan<kScanBlock>(v, s_ws, tot);
-        if (i < n) out[i] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0) *total = carry;
 }
 
 __global__ void k_gather_tris(const float4* __restrict__ tri_world, const uint32_t* __restrict__ idx, uint32_t N,
@@ -1239,8 +1293,111 @@ hipError_t flatten_scene(const InstBuild* d_insts, uint32_t ninst, const MeshRef
     return hipGetLastError();
 }
 
+// ---- workspace of a build ---------------------------------------------------
+namespace {
+struct KeptBlock {
+    std::mutex taken;          // held by the build that uses the block
+    uint8_t* base = nullptr;
+    size_t cap = 0;
+    uint32_t* host = nullptr;
+};
+constexpr int kMaxDevices = 64;
+KeptBlock g_kept[kMaxDevices];
+size_t round256(size_t n) { return (n + 255) / 256 * 256; }
+}  // namespace
+
+BuildWorkspace::BuildWorkspace(int device, size_t bytes) : device_(device) {
+    if (device < 0 || device >= kMaxDevices || !g_kept[device].taken.try_lock()) return;
+    KeptBlock& k = g_kept[device];
+    shared_ = true;
+    if (bytes <= kKeepBytes && k.cap < bytes) {
+        if (k.base) (void)hipFree(k.base);
+        k.base = nullptr;
+        k.cap = 0;
+        if (hipMalloc((void**)&k.base, bytes) == hipSuccess) k.cap = bytes;
+        else (void)hipGetLastError();   // take() allocates piece by piece then
+    }
+    if (!k.host && hipHostMalloc((void**)&k.host, kHostWords * sizeof(uint32_t), 0) != hipSuccess) k.host = nullptr;
+    base_ = k.base;
+    cap_ = k.cap;
+    host_ = k.host;
+}
+
+BuildWorkspace::~BuildWorkspace() {
+    if (!done_) (void)hipDeviceSynchronize();   // a build that failed may still be running
+    for (void* p : more_) (void)hipFree(p);
+    if (shared_) g_kept[device_].taken.unlock();
+    else if (host_) (void)hipHostFree(host_);
+}
+
+hipError_t BuildWorkspace::take(void** p, size_t bytes) {
+    const size_t n = round256(bytes);
+    if (used_ + n <= cap_) {
+        *p = base_ + used_;
+        used_ += n;
+        return hipSuccess;
+    }
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) more_.push_back(*p);
+    return e;
+}
+
+hipError_t BuildWorkspace::host_words(uint32_t** h) {
+    if (!host_) {
+        const hipError_t e = hipHostMalloc((void**)&host_, kHostWords * sizeof(uint32_t), 0);
+        if (e != hipSuccess) {
+            host_ = nullptr;
+            return e;
+        }
+        if (shared_) g_kept[device_].host = host_;
+    }
+    *h = host_;
+    return hipSuccess;
+}
+
+void build_workspace_drop(int device) {
+    if (device < 0 || device >= kMaxDevices) return;
+    KeptBlock& k = g_kept[device];
+    if (!k.taken.try_lock()) return;   // a build is running: its contexts outlive it
+    if (k.base) (void)hipFree(k.base);
+    if (k.host) (void)hipHostFree(k.host);
+    k.base = nullptr;
+    k.host = nullptr;
+    k.cap = 0;
+    k.taken.unlock();
+}
+
+size_t bvh_workspace_bytes(uint32_t N) {
+    const size_t n = N ? N : 1;
+    size_t b = 2 * round256(4 * n) + round256(sizeof(BNode) * 2 * n);                             // idx, tmp, bnodes
+    b += round256(4 * n) + 2 * round256(sizeof(BuildTask) * n) + round256(sizeof(SplitOut) * n);  // rank, tasks, so
+    b += round256(4 * (n / (kTinyTask + 1) + 1)) + 2 * round256(4 * (n / kScanTile + 2));
+    if (N >= kWideMinPrims) b += sizeof(uint32_t) * kPartialWords * (size_t)(kWideBlocks + kWideTasks) + 65536;
+    return b + 65536;
+}
+
+size_t bvh_result_bytes(uint32_t N) {
+    const size_t n = N ? N : 1;
+    return round256(sizeof(float4) * 3 * (n + 1)) + round256(sizeof(float4) * kWideNodeF4 * n) + round256(4 * n) + 1024;
+}
+
+namespace {
+// events of the levels in flight, destroyed at scope exit
+struct LevelEvents {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    hipError_t init() {
+        for (auto& x : e) {
+            const hipError_t r = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+            if (r != hipSuccess) return r;
+        }
+        return hipSuccess;
+    }
+    ~LevelEvents() { for (auto& x : e) if (x) (void)hipEventDestroy(x); }
+};
+}  // namespace
+
 hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float4* d_phi, uint32_t N,
-                     hipStream_t s, BuiltBVH* outp, std::string* err, const BvhOptions& opt) {
+                     hipStream_t s, BuildWorkspace& ws, BuiltBVH* outp, std::string* err, const BvhOptions& opt) {
     BuiltBVH out;
     const uint32_t max_leaf = opt.max_leaf < 1 ? 1u : (opt.max_leaf > kMaxLeaf ? kMaxLeaf : opt.max_leaf);
     if (N == 0) {
@@ -1248,218 +1405,243 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
         *outp = out;
         return hipSuccess;
     }
-    DevBuf<uint32_t> idx, tmp, rank, total;
-    DevBuf<BuildTask> tasks_a, tasks_b;
-    DevBuf<SplitOut> so;
-    DevBuf<BNode> bnodes;
-    DevBuf<BuildStats> st;
-    const size_t max_nodes = 2 * (size_t)N;
-    RTX_TRY(idx.alloc(N));
-    RTX_TRY(tmp.alloc(N));
-    RTX_TRY(rank.alloc(max_nodes));
-    RTX_TRY(total.alloc(1));
-    RTX_TRY(tasks_a.alloc(N));
-    RTX_TRY(tasks_b.alloc(N));
-    RTX_TRY(so.alloc(max_nodes));
-    RTX_TRY(bnodes.alloc(max_nodes));
-    RTX_TRY(st.alloc(1));
-    RTX_TRY(hipMemsetAsync(st.p, 0, sizeof(BuildStats), s));
-    DevBuf<uint32_t> partial, merged, lcount, rb;
-    DevBuf<uint4> wsplit;
+    uint32_t* host = nullptr;
+    RTX_TRY(ws.host_words(&host));
+    LevelEvents ev;
+    RTX_TRY(ev.init());
+    // results that stay in the workspace come first
+    float4 *tris_ws = nullptr, *wide = nullptr;
+    uint32_t* idx = nullptr;
+    if (!opt.owned) {
+        RTX_TRY(ws.get(&wide, kWideNodeF4 * (size_t)N));
+        if (opt.gather) RTX_TRY(ws.get(&tris_ws, 3 * ((size_t)N + 1)));
+        else RTX_TRY(ws.get(&idx, N));
+    }
+    const size_t m_all = ws.mark();
+    uint32_t *tmp = nullptr, *rank = nullptr, *rb = nullptr, *big = nullptr, *nbig = nullptr, *tsum = nullptr,
+             *toff = nullptr, *partial = nullptr, *merged = nullptr, *lcount = nullptr;
+    BuildTask *tasks_a = nullptr, *tasks_b = nullptr;
+    SplitOut* so = nullptr;
+    BNode* bnodes = nullptr;
+    BuildStats* st = nullptr;
+    Level *lev = nullptr, *wlev = nullptr;
+    uint4* wsplit = nullptr;
+    if (!idx) RTX_TRY(ws.get(&idx, N));
+    RTX_TRY(ws.get(&bnodes, 2 * (size_t)N));
+    RTX_TRY(ws.get(&st, 1));
+    RTX_TRY(ws.get(&lev, kMaxLevels + 1));
+    RTX_TRY(ws.get(&wlev, kMaxLevels + 1));
+    RTX_TRY(ws.get(&tsum, (size_t)N / kScanTile + 2));
+    RTX_TRY(ws.get(&toff, (size_t)N / kScanTile + 2));
+    const size_t m_levels = ws.mark();   // from here on: the binary tree's levels, then the collapse's arrays
+    RTX_TRY(ws.get(&tmp, N));
+    RTX_TRY(ws.get(&rank, N));
+    RTX_TRY(ws.get(&tasks_a, N));
+    RTX_TRY(ws.get(&tasks_b, N));
+    RTX_TRY(ws.get(&so, N));
+    RTX_TRY(ws.get(&rb, 6));
     if (N >= kWideMinPrims) {
         // chunks of a wide level: G * tasks <= N / kWideMinChunk; tasks <= N / kWideMinPrims
         const uint32_t nchunks = std::min(kWideBlocks, N / kWideMinChunk);
         const uint32_t nwide = std::min(kWideTasks, N / kWideMinPrims);
-        RTX_TRY(partial.alloc((size_t)nchunks * kPartialWords));
-        RTX_TRY(merged.alloc((size_t)nwide * kPartialWords));
-        RTX_TRY(lcount.alloc(nchunks));
-        RTX_TRY(wsplit.alloc(nwide));
+        RTX_TRY(ws.get(&partial, (size_t)nchunks * kPartialWords));
+        RTX_TRY(ws.get(&merged, (size_t)nwide * kPartialWords));
+        RTX_TRY(ws.get(&lcount, nchunks));
+        RTX_TRY(ws.get(&wsplit, nwide));
     }
-    RTX_TRY(rb.alloc(6));
     // tasks of a small-task level above kTinyTask primitives (at most N / (kTinyTask + 1))
-    DevBuf<uint32_t> big, nbig;
-    RTX_TRY(big.alloc(N / (kTinyTask + 1) + 1));
-    RTX_TRY(nbig.alloc(1));
+    RTX_TRY(ws.get(&big, N / (kTinyTask + 1) + 1));
+    RTX_TRY(ws.get(&nbig, 1));
 
-    hipLaunchKernelGGL(k_iota, dim3(blocks_for(N, 256)), dim3(256), 0, s, idx.p, N);
-    hipLaunchKernelGGL(k_root_init, dim3(1), dim3(64), 0, s, rb.p);
+    hipLaunchKernelGGL(k_iota, dim3(blocks_for(N, 256)), dim3(256), 0, s, idx, N);
+    hipLaunchKernelGGL(k_root_init, dim3(1), dim3(64), 0, s, rb, st, lev, wlev);
     hipLaunchKernelGGL(k_root_bounds, dim3(std::min<uint32_t>(blocks_for(N, 256), kRootBlocks)), dim3(256), 0, s,
-                       d_plo, d_phi, N, rb.p);
-    hipLaunchKernelGGL(k_root_task, dim3(1), dim3(64), 0, s, rb.p, N, tasks_a.p);
+                       d_plo, d_phi, N, rb);
+    hipLaunchKernelGGL(k_root_task, dim3(1), dim3(64), 0, s, rb, N, tasks_a);
     RTX_TRY(hipGetLastError());
 
-    // exclusive scan of so[0, n).kind into rank, the sum into total
-    DevBuf<uint32_t> tsum, toff;
-    RTX_TRY(tsum.alloc((size_t)max_nodes / kScanTile + 2));
-    RTX_TRY(toff.alloc((size_t)max_nodes / kScanTile + 2));
-    auto scan_kind = [&](uint32_t n) {
-        if (n <= 16 * kScanTile) {
-            hipLaunchKernelGGL(k_scan_kind, dim3(1), dim3(kScanBlock), 0, s, so.p, n, rank.p, total.p);
+    // exclusive scan of a level's values (`most` of them at most) into out, the
+    // next level into l[1] and its count to h
+    auto scan = [&](Level* l, auto get, uint32_t most, uint32_t* o, uint32_t* h) {
+        using Get = decltype(get);
+        if (most <= 16 * kScanTile) {
+            hipLaunchKernelGGL(k_scan<Get>, dim3(1), dim3(kScanBlock), 0, s, l, get, o, h);
             return;
         }
-        const uint32_t nt = (n + kScanTile - 1) / kScanTile;
-        hipLaunchKernelGGL(k_scan_tiles<KindOf>, dim3(nt), dim3(kScanBlock), 0, s, KindOf{so.p}, n, tsum.p);
-        hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, s, tsum.p, nt, toff.p, total.p);
-        hipLaunchKernelGGL(k_scan_apply<KindOf>, dim3(nt), dim3(kScanBlock), 0, s, KindOf{so.p}, n, toff.p, rank.p);
-    };
-    // exclusive scan of in[0, n) into out, the sum into total (the same tiles)
-    auto scan_u32 = [&](const uint32_t* in, uint32_t n, uint32_t* out) {
-        if (n <= 16 * kScanTile) {
-            hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, s, in, n, out, total.p);
-            return;
-        }
-        const uint32_t nt = (n + kScanTile - 1) / kScanTile;
-        hipLaunchKernelGGL(k_scan_tiles<U32Of>, dim3(nt), dim3(kScanBlock), 0, s, U32Of{in}, n, tsum.p);
-        hipLaunchKernelGGL(k_scan_u32, dim3(1), dim3(kScanBlock), 0, s, tsum.p, nt, toff.p, total.p);
-        hipLaunchKernelGGL(k_scan_apply<U32Of>, dim3(nt), dim3(kScanBlock), 0, s, U32Of{in}, n, toff.p, out);
+        const uint32_t nt = (most + kScanTile - 1) / kScanTile;
+        hipLaunchKernelGGL(k_scan_tiles<Get>, dim3(nt), dim3(kScanBlock), 0, s, l, get, tsum);
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, s, l, Get::kMakes, tsum, toff, h);
+        hipLaunchKernelGGL(k_scan_apply<Get>, dim3(nt), dim3(kScanBlock), 0, s, l, get, toff, o);
     };
 
-    uint32_t ntasks = 1, nnodes = 1;
-    BuildTask* cur = tasks_a.p;
-    BuildTask* nxt = tasks_b.p;
+    // The levels, one ahead of the device: level d is launched for the most
+    // tasks it can have (two per task of level d - 1) once level d - 2 is done,
+    // which gave level d - 1's count, while level d - 1 runs.  (A wait per level
+    // left the device idle for 30 to 40 us each: with the shared workspace a
+    // level-4 scene builds in 3.8 ms host to host, 8.9 before, and the level-6
+    // one in 21.5, 27.6 before.)  The last level launched is an empty one.
+    BuildTask* cur = tasks_a;
+    BuildTask* nxt = tasks_b;
     std::vector<uint32_t> level_first;   // binary level d: nodes level_first[d] .. level_first[d+1]-1
-    while (ntasks > 0) {
-        level_first.push_back(nnodes - ntasks);
+    uint32_t nnodes = 0;
+    for (uint32_t d = 0, known = 1;; d++) {
+        // known: tasks of level d - 1 (of the root level for d = 0)
+        if (d >= 2) {
+            RTX_TRY(hipEventSynchronize(ev.e[d & 1u]));
+            known = ((volatile uint32_t*)host)[(d - 1) % kMaxLevels];
+            if (known == 0) break;
+        }
+        if (d != 1) {
+            level_first.push_back(nnodes);
+            nnodes += known;
+        }
+        if (d && d % kMaxLevels == 0) hipLaunchKernelGGL(k_level_wrap, dim3(1), dim3(1), 0, s, lev);
+        const uint32_t most = (uint32_t)std::min<uint64_t>(N, d == 0 ? 1u : 2ull * known);
+        Level* l = lev + d % kMaxLevels;
         // a few big tasks: each spread over G chunks (kWideBlocks in all, of
         // kWideMinChunk primitives at least on average), their bins merged by
         // k_merge_wide; a wave per task once tasks average fewer than
         // kSmallTask primitives, and on levels of kTinyLevel tasks or more a
         // thread per task of at most kTinyTask primitives (the same tree every
         // way: binning, SAH and partition do not depend on the split)
-        if (ntasks <= kWideTasks && (uint64_t)N >= (uint64_t)kWideMinPrims * ntasks) {
-            const uint32_t G = std::min(kWideBlocks / ntasks, N / (ntasks * kWideMinChunk));
-            const dim3 gw(G, ntasks);
-            hipLaunchKernelGGL(k_bin_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, cur, d_plo, d_phi, idx.p, G,
-                               partial.p);
-            hipLaunchKernelGGL(k_merge_wide, dim3(kPartialWords / kMergeWords, ntasks), dim3(256), 0, s, G, partial.p,
-                               merged.p);
-            hipLaunchKernelGGL(k_decide_wide<kBuildBlock>, dim3(ntasks), dim3(kBuildBlock), 0, s, cur, 1u, merged.p,
-                               bnodes.p, so.p, wsplit.p, max_leaf);
-            hipLaunchKernelGGL(k_count_wide, dim3((G + 3) / 4, ntasks), dim3(256), 0, s, G, partial.p, wsplit.p,
-                               lcount.p);
-            hipLaunchKernelGGL(k_scatter_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, cur, d_plo, d_phi, idx.p,
-                               tmp.p, G, wsplit.p, lcount.p);
-            hipLaunchKernelGGL(k_copy_wide, gw, dim3(256), 0, s, cur, G, wsplit.p, tmp.p, idx.p);
-        } else if ((uint64_t)N < (uint64_t)kSmallTask * ntasks && ntasks < kTinyLevel) {
-            hipLaunchKernelGGL(k_level<64>, dim3(ntasks), dim3(64), 0, s, cur, d_plo, d_phi, idx.p, tmp.p, bnodes.p,
-                               so.p, max_leaf);
-        } else if ((uint64_t)N < (uint64_t)kSmallTask * ntasks) {
-            RTX_TRY(hipMemsetAsync(nbig.p, 0, sizeof(uint32_t), s));
-            hipLaunchKernelGGL(k_level_tiny, dim3(blocks_for(ntasks, 256)), dim3(256), 0, s, cur, ntasks, d_plo, d_phi,
-                               idx.p, tmp.p, bnodes.p, so.p, max_leaf, big.p, nbig.p);
-            hipLaunchKernelGGL(k_level_list, dim3(std::min(ntasks, kListGrid)), dim3(64), 0, s, cur, big.p, nbig.p,
-                               d_plo, d_phi, idx.p, tmp.p, bnodes.p, so.p, max_leaf);
+        if (most <= kWideTasks && (uint64_t)N >= (uint64_t)kWideMinPrims * most) {
+            const uint32_t G = std::min(kWideBlocks / most, N / (most * kWideMinChunk));
+            const dim3 gw(G, most);
+            hipLaunchKernelGGL(k_bin_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, l, cur, d_plo, d_phi, idx, G,
+                               partial);
+            hipLaunchKernelGGL(k_merge_wide, dim3(kPartialWords / kMergeWords, most), dim3(256), 0, s, l, G, partial,
+                               merged);
+            hipLaunchKernelGGL(k_decide_wide<kBuildBlock>, dim3(most), dim3(kBuildBlock), 0, s, l, cur, 1u, merged,
+                               bnodes, so, wsplit, max_leaf);
+            hipLaunchKernelGGL(k_count_wide, dim3((G + 3) / 4, most), dim3(256), 0, s, l, G, partial, wsplit, lcount);
+            hipLaunchKernelGGL(k_scatter_wide<kBuildBlock>, gw, dim3(kBuildBlock), 0, s, l, cur, d_plo, d_phi, idx,
+                               tmp, G, wsplit, lcount);
+            hipLaunchKernelGGL(k_copy_wide, gw, dim3(256), 0, s, l, cur, G, wsplit, tmp, idx);
+        } else if ((uint64_t)N < (uint64_t)kSmallTask * most && most < kTinyLevel) {
+            hipLaunchKernelGGL(k_level<64>, dim3(most), dim3(64), 0, s, l, cur, d_plo, d_phi, idx, tmp, bnodes, so,
+                               max_leaf);
+        } else if ((uint64_t)N < (uint64_t)kSmallTask * most) {
+            hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, nbig);
+            hipLaunchKernelGGL(k_level_tiny, dim3(blocks_for(most, 256)), dim3(256), 0, s, l, cur, d_plo, d_phi, idx,
+                               tmp, bnodes, so, max_leaf, big, nbig);
+            hipLaunchKernelGGL(k_level_list, dim3(std::min(most, kListGrid)), dim3(64), 0, s, cur, big, nbig, d_plo,
+                               d_phi, idx, tmp, bnodes, so, max_leaf);
         } else
-            hipLaunchKernelGGL(k_level<kBuildBlock>, dim3(ntasks), dim3(kBuildBlock), 0, s, cur, d_plo, d_phi, idx.p,
-                               tmp.p, bnodes.p, so.p, max_leaf);
-        scan_kind(ntasks);
-        hipLaunchKernelGGL(k_emit, dim3(blocks_for(ntasks, 256)), dim3(256), 0, s, cur, so.p, rank.p, ntasks,
-                           nnodes, bnodes.p, nxt);
+            hipLaunchKernelGGL(k_level<kBuildBlock>, dim3(most), dim3(kBuildBlock), 0, s, l, cur, d_plo, d_phi, idx,
+                               tmp, bnodes, so, max_leaf);
+        scan(l, KindOf{so}, most, rank, host + (d + 1) % kMaxLevels);
+        hipLaunchKernelGGL(k_emit, dim3(blocks_for(most, 256)), dim3(256), 0, s, l, cur, so, rank, bnodes, nxt);
         RTX_TRY(hipGetLastError());
-        uint32_t nsplit = 0;
-        RTX_TRY(hipMemcpyAsync(&nsplit, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        RTX_TRY(hipStreamSynchronize(s));
-        nnodes += 2 * nsplit;
-        ntasks = 2 * nsplit;
+        RTX_TRY(hipEventRecord(ev.e[d & 1u], s));
         std::swap(cur, nxt);
     }
+    level_first.push_back(nnodes);
 
-    hipLaunchKernelGGL(k_sah, dim3(std::min(blocks_for(nnodes, 256), kSahBlocks)), dim3(256), 0, s, bnodes.p, nnodes,
-                       st.p);
+    hipLaunchKernelGGL(k_sah, dim3(std::min(blocks_for(nnodes, 256), kSahBlocks)), dim3(256), 0, s, bnodes, nnodes,
+                       st);
     RTX_TRY(hipGetLastError());
     const uint32_t ninner = (nnodes - 1) / 2;
-    BuildStats hst;
-    RTX_TRY(hipMemcpyAsync(&hst, st.p, sizeof(BuildStats), hipMemcpyDeviceToHost, s));
-    BNode root;
-    RTX_TRY(hipMemcpyAsync(&root, bnodes.p, sizeof(BNode), hipMemcpyDeviceToHost, s));
-    RTX_TRY(hipStreamSynchronize(s));
 
     DevBuf<float4> nodes, tris;
+    float4* tris_out = tris_ws;
     if (opt.gather) {
-        RTX_TRY(tris.alloc(3 * ((size_t)N + 1)));
-        hipLaunchKernelGGL(k_gather_tris, dim3(blocks_for((uint64_t)N + 1, 256)), dim3(256), 0, s, d_tri_world,
-                           idx.p, N, tris.p);
-        RTX_TRY(hipGetLastError());
-    }
-
-    level_first.push_back(nnodes);
-#if RTX_DP_COLLAPSE
-    // the collapse's choices, bottom-up by binary level
-    DevBuf<float4> dpc;
-    DevBuf<uint32_t> dp_ntri, dp_first, dp_meta;
-    if (ninner) {
-        RTX_TRY(dpc.alloc(nnodes));
-        RTX_TRY(dp_ntri.alloc(nnodes));
-        RTX_TRY(dp_first.alloc(nnodes));
-        RTX_TRY(dp_meta.alloc(nnodes));
-        for (size_t d = level_first.size() - 1; d-- > 0;) {
-            const uint32_t b = level_first[d], n = level_first[d + 1] - b;
-            if (n == 0) continue;
-            hipLaunchKernelGGL(k_dp_level, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes.p, b, n, dpc.p,
-                               dp_ntri.p, dp_first.p, dp_meta.p, max_leaf);
+        if (opt.owned) {
+            RTX_TRY(tris.alloc(3 * ((size_t)N + 1)));
+            tris_out = tris.p;
         }
+        hipLaunchKernelGGL(k_gather_tris, dim3(blocks_for((uint64_t)N + 1, 256)), dim3(256), 0, s, d_tri_world, idx, N,
+                           tris_out);
         RTX_TRY(hipGetLastError());
     }
-    const uint32_t *wmeta = dp_meta.p, *wntri = dp_ntri.p, *wfirst = dp_first.p;
-#else
-    const uint32_t *wmeta = nullptr, *wntri = nullptr, *wfirst = nullptr;
-#endif
 
-    out.plane_scale = plane_scale_for(std::max(std::max(root.hi.x - root.lo.x, root.hi.y - root.lo.y),
-                                               root.hi.z - root.lo.z));
     // 4-wide nodes: at most one per binary inner node
+    ws.reset(m_levels);
     uint32_t nwide = 0, wide_depth = 0;
     if (ninner) {
-        DevBuf<float4> wide;
-        DevBuf<uint32_t> fa, fb, cnt, off;
-        DevBuf<uint4> cid;
-        RTX_TRY(wide.alloc(kWideNodeF4 * (size_t)ninner));
-        RTX_TRY(fa.alloc(ninner));
-        RTX_TRY(fb.alloc(ninner));
-        RTX_TRY(cnt.alloc(ninner));
-        RTX_TRY(off.alloc(ninner));
-        RTX_TRY(cid.alloc(ninner));
-        const uint32_t zero = 0;
-        RTX_TRY(hipMemcpyAsync(fa.p, &zero, sizeof(uint32_t), hipMemcpyHostToDevice, s));   // the root
-        uint32_t n = 1;
-        uint32_t* cur = fa.p;
-        uint32_t* nxt = fb.p;
-        while (n > 0) {
-            out.level_begin.push_back(nwide);
+        const uint32_t *wmeta = nullptr, *wntri = nullptr, *wfirst = nullptr;
 #if RTX_DP_COLLAPSE
-            hipLaunchKernelGGL(k_collapse4_dp, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes.p, cur, n, dp_meta.p,
-                               cid.p, cnt.p);
-#else
-            hipLaunchKernelGGL(k_collapse4, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes.p, cur, n, cid.p,
-                               cnt.p);
-#endif
-            scan_u32(cnt.p, n, off.p);
-            hipLaunchKernelGGL(k_write4, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes.p, cid.p, off.p, n,
-                               nwide, nwide + n, leaf_ref(N, 1), wide.p, nxt, wmeta, wntri, wfirst, out.plane_scale);
-            RTX_TRY(hipGetLastError());
-            uint32_t nn = 0;
-            RTX_TRY(hipMemcpyAsync(&nn, total.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-            RTX_TRY(hipStreamSynchronize(s));
-            nwide += n;
-            wide_depth++;
-            n = nn;
-            std::swap(cur, nxt);
+        // the collapse's choices, bottom-up by binary level
+        float4* dpc = nullptr;
+        uint32_t *dp_ntri = nullptr, *dp_first = nullptr, *dp_meta = nullptr;
+        RTX_TRY(ws.get(&dpc, nnodes));
+        RTX_TRY(ws.get(&dp_ntri, nnodes));
+        RTX_TRY(ws.get(&dp_first, nnodes));
+        RTX_TRY(ws.get(&dp_meta, nnodes));
+        for (size_t d = level_first.size() - 1; d-- > 0;) {
+            const uint32_t b = level_first[d], n = level_first[d + 1] - b;
+            hipLaunchKernelGGL(k_dp_level, dim3(blocks_for(n, 256)), dim3(256), 0, s, bnodes, b, n, dpc, dp_ntri,
+                               dp_first, dp_meta, max_leaf);
         }
-        RTX_TRY(nodes.alloc(kWideNodeF4 * (size_t)nwide));
-        RTX_TRY(hipMemcpyAsync(nodes.p, wide.p, sizeof(float4) * kWideNodeF4 * (size_t)nwide,
-                               hipMemcpyDeviceToDevice, s));
-    } else {
-        RTX_TRY(nodes.alloc(kWideNodeF4));
+        RTX_TRY(hipGetLastError());
+        wmeta = dp_meta;
+        wntri = dp_ntri;
+        wfirst = dp_first;
+#endif
+        uint32_t *fa = nullptr, *fb = nullptr, *cnt = nullptr, *off = nullptr;
+        uint4* cid = nullptr;
+        if (!wide) RTX_TRY(ws.get(&wide, kWideNodeF4 * (size_t)ninner));
+        RTX_TRY(ws.get(&fa, ninner));
+        RTX_TRY(ws.get(&fb, ninner));
+        RTX_TRY(ws.get(&cnt, ninner));
+        RTX_TRY(ws.get(&off, ninner));
+        RTX_TRY(ws.get(&cid, ninner));
+        // the levels of the 4-wide tree, one ahead of the device like the
+        // binary ones (a node has at most four inner children)
+        uint32_t* whost = host + kMaxLevels;
+        uint32_t* wcur = nullptr;   // the first level is the root alone
+        uint32_t* wnxt = fa;
+        for (uint32_t d = 0, known = 1;; d++) {
+            if (d >= 2) {
+                RTX_TRY(hipEventSynchronize(ev.e[d & 1u]));
+                known = ((volatile uint32_t*)whost)[(d - 1) % kMaxLevels];
+                if (known == 0) break;
+            }
+            if (d != 1) {
+                out.level_begin.push_back(nwide);
+                nwide += known;
+                wide_depth++;
+            }
+            if (d && d % kMaxLevels == 0) hipLaunchKernelGGL(k_level_wrap, dim3(1), dim3(1), 0, s, wlev);
+            const uint32_t most = (uint32_t)std::min<uint64_t>(ninner, d == 0 ? 1u : 4ull * known);
+            Level* l = wlev + d % kMaxLevels;
+            const dim3 g(blocks_for(most, 256)), b(256);
+#if RTX_DP_COLLAPSE
+            hipLaunchKernelGGL(k_collapse4_dp, g, b, 0, s, l, bnodes, wcur, wmeta, cid, cnt);
+#else
+            hipLaunchKernelGGL(k_collapse4, g, b, 0, s, l, bnodes, wcur, cid, cnt);
+#endif
+            scan(l, CountOf{cnt}, most, off, whost + (d + 1) % kMaxLevels);
+            hipLaunchKernelGGL(k_write4, g, b, 0, s, l, bnodes, cid, off, leaf_ref(N, 1), wide, wnxt, wmeta, wntri,
+                               wfirst);
+            RTX_TRY(hipGetLastError());
+            RTX_TRY(hipEventRecord(ev.e[d & 1u], s));
+            wcur = wnxt;
+            wnxt = wnxt == fa ? fb : fa;
+        }
+    }
+    BuildStats* hst = (BuildStats*)(host + 2 * kMaxLevels);
+    BNode* hroot = (BNode*)(hst + 1);
+    static_assert(kMaxLevels % 4 == 0 && sizeof(BuildStats) % 16 == 0, "aligned records");
+    static_assert(8 * kMaxLevels + sizeof(BuildStats) + sizeof(BNode) <= 4 * BuildWorkspace::kHostWords, "host words");
+    RTX_TRY(hipMemcpyAsync(hst, st, sizeof(BuildStats), hipMemcpyDeviceToHost, s));
+    RTX_TRY(hipMemcpyAsync(hroot, bnodes, sizeof(BNode), hipMemcpyDeviceToHost, s));
+    if (opt.owned) {
+        RTX_TRY(nodes.alloc(kWideNodeF4 * (size_t)(nwide ? nwide : 1)));
+        if (nwide)
+            RTX_TRY(hipMemcpyAsync(nodes.p, wide, sizeof(float4) * kWideNodeF4 * (size_t)nwide,
+                                   hipMemcpyDeviceToDevice, s));
     }
     RTX_TRY(hipStreamSynchronize(s));
+    const BNode root = *hroot;
     out.level_begin.push_back(nwide);
 
     const uint32_t root_cnt = __builtin_bit_cast(uint32_t, root.hi.w);
     const float rx = root.hi.x - root.lo.x, ry = root.hi.y - root.lo.y, rz = root.hi.z - root.lo.z;
     const double root_area = 2.0 * ((double)rx * ry + (double)ry * rz + (double)rz * rx);
-    out.nodes = nodes.release();
-    out.tris = tris.release();
-    if (!opt.gather) out.order = idx.release();
+    out.plane_scale = plane_scale_of(root.lo, root.hi);
+    out.nodes = opt.owned ? nodes.release() : wide;
+    out.tris = opt.owned ? tris.release() : tris_ws;
+    if (!opt.gather) out.order = idx;
     out.root_lo[0] = root.lo.x; out.root_lo[1] = root.lo.y; out.root_lo[2] = root.lo.z;
     out.root_hi[0] = root.hi.x; out.root_hi[1] = root.hi.y; out.root_hi[2] = root.hi.z;
     out.root = root_cnt ? leaf_ref(__builtin_bit_cast(uint32_t, root.lo.w), root_cnt) : 0u;
@@ -1468,8 +1650,9 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
     out.wide_depth = wide_depth;
     out.num_leaves = nnodes - ninner;
     out.max_depth = (uint32_t)level_first.size() - 1;
-    out.max_leaf = hst.max_leaf;
-    out.sah = root_area > 0.0 ? hst.sah / root_area : 0.0;
+    out.max_leaf = hst->max_leaf;
+    out.sah = root_area > 0.0 ? hst->sah / root_area : 0.0;
+    ws.reset(m_all);
     *outp = out;
     return hipSuccess;
 }

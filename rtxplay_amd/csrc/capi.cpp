@@ -148,6 +148,11 @@ void noalloc_setup(int device) {
 }
 }  // namespace
 
+// contexts per device: the last one's end drops the device's build workspace
+std::mutex g_ctx_mu;
+constexpr int kMaxDevices = 64;
+int g_ctx_count[kMaxDevices] = {};
+
 struct rtx_ctx {
     int device = 0;
     int num_cus = 0;
@@ -223,6 +228,10 @@ rtx_status rtx_ctx_create(int device, rtx_ctx** out) {
     noalloc_setup(device);
     rtx_ctx* c = new rtx_ctx();
     c->device = device;
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        g_ctx_count[device % kMaxDevices]++;
+    }
     c->num_cus = prop.multiProcessorCount;
     rtx_status st = alloc_scratch(c->render_ls, rtx::render_blocks_per_cu(), c->num_cus, rtx::kRenderBlock);
     if (st == RTX_SUCCESS)
@@ -262,6 +271,12 @@ rtx_status rtx_ctx_destroy(rtx_ctx* c) {
         if (ls->tile_order) (void)hipFree(ls->tile_order);
     }
     if (c->tape) (void)hipFree(c->tape);
+    bool last;
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        last = --g_ctx_count[c->device % kMaxDevices] == 0;
+    }
+    if (last) rtx::build_workspace_drop(c->device);
     delete c;
     return RTX_SUCCESS;
 }
@@ -535,23 +550,25 @@ static rtx_status build_scene_flat(rtx_ctx* c, hipStream_t s, Built** out) {
     std::vector<rtx::MeshRef> mr(c->meshes.size() ? c->meshes.size() : 1);
     for (size_t m = 0; m < c->meshes.size(); m++)
         mr[m] = rtx::MeshRef{c->meshes[m].d_v, c->meshes[m].d_i, c->meshes[m].nv, c->meshes[m].ni};
-    Tmp<rtx::InstBuild> d_ib;
-    Tmp<rtx::MeshRef> d_mr;
-    Tmp<float4> d_plo, d_phi;
+    rtx::BuildWorkspace ws(c->device, rtx::bvh_workspace_bytes((uint32_t)N) + 2 * sizeof(float4) * (size_t)N +
+                                          sizeof(rtx::InstBuild) * ib.size() + sizeof(rtx::MeshRef) * mr.size() + 4096);
+    rtx::InstBuild* d_ib = nullptr;
+    rtx::MeshRef* d_mr = nullptr;
+    float4 *d_plo = nullptr, *d_phi = nullptr;
     hipError_t e;
-    if ((e = hipMalloc((void**)&d_ib.p, sizeof(rtx::InstBuild) * ib.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(insts)"));
-    if ((e = hipMalloc((void**)&d_mr.p, sizeof(rtx::MeshRef) * mr.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(meshes)"));
+    if ((e = ws.get(&d_ib, ib.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(insts)"));
+    if ((e = ws.get(&d_mr, mr.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(meshes)"));
     if ((e = hipMalloc((void**)&b->insts, sizeof(float4) * irec.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(inst records)"));
     if ((e = hipMalloc((void**)&b->tri_world, sizeof(float4) * 3 * (N ? N : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(triangles)"));
-    if ((e = hipMalloc((void**)&d_plo.p, sizeof(float4) * (N ? N : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
-    if ((e = hipMalloc((void**)&d_phi.p, sizeof(float4) * (N ? N : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
-    if ((e = hipMemcpyAsync(d_ib.p, ib.data(), sizeof(rtx::InstBuild) * ib.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload insts"));
-    if ((e = hipMemcpyAsync(d_mr.p, mr.data(), sizeof(rtx::MeshRef) * mr.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload meshes"));
+    if ((e = ws.get(&d_plo, N)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
+    if ((e = ws.get(&d_phi, N)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
+    if ((e = hipMemcpyAsync(d_ib, ib.data(), sizeof(rtx::InstBuild) * ib.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload insts"));
+    if ((e = hipMemcpyAsync(d_mr, mr.data(), sizeof(rtx::MeshRef) * mr.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload meshes"));
     if ((e = hipMemcpyAsync(b->insts, irec.data(), sizeof(float4) * irec.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload inst records"));
-    if ((e = rtx::flatten_scene(d_ib.p, ninst, d_mr.p, (uint32_t)N, b->tri_world, d_plo.p, d_phi.p, s)) != hipSuccess) return bail(hip_fail(e, "flatten"));
+    if ((e = rtx::flatten_scene(d_ib, ninst, d_mr, (uint32_t)N, b->tri_world, d_plo, d_phi, s)) != hipSuccess) return bail(hip_fail(e, "flatten"));
     rtx::BuiltBVH bvh;
     std::string err;
-    if ((e = rtx::build_bvh(b->tri_world, d_plo.p, d_phi.p, (uint32_t)N, s, &bvh, &err)) != hipSuccess)
+    if ((e = rtx::build_bvh(b->tri_world, d_plo, d_phi, (uint32_t)N, s, ws, &bvh, &err)) != hipSuccess)
         return bail(fail(e == hipErrorOutOfMemory ? RTX_ERROR_OUT_OF_MEMORY : RTX_ERROR_HIP, "build_bvh: " + err));
     b->nodes = bvh.nodes;
     b->tris = bvh.tris;
@@ -568,6 +585,7 @@ static rtx_status build_scene_flat(rtx_ctx* c, hipStream_t s, Built** out) {
     if ((e = hipMemcpyAsync(b->d_hdr, &b->hdr, sizeof(rtx::DevScene), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload handle"));
     if ((e = hipEventRecord(e1, s)) != hipSuccess) return bail(hip_fail(e, "hipEventRecord"));
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return bail(hip_fail(e, "hipStreamSynchronize"));
+    ws.done();
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);
@@ -602,18 +620,6 @@ static rtx_status build_scene_flat(rtx_ctx* c, hipStream_t s, Built** out) {
 
 // ---- two-level scenes -------------------------------------------------------
 namespace {
-
-// owned results of build_bvh, freed at scope exit
-struct BvhSet {
-    std::vector<rtx::BuiltBVH> v;
-    ~BvhSet() {
-        for (auto& x : v) {
-            if (x.nodes) (void)hipFree(x.nodes);
-            if (x.tris) (void)hipFree(x.tris);
-            if (x.order) (void)hipFree(x.order);
-        }
-    }
-};
 
 // One instance of a two-level scene: its record (world-to-object rows,
 // object-to-world rows, (root, first global triangle, mesh, 0)) and its world
@@ -739,44 +745,53 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     hipError_t e;
     std::string err;
 
+    // the build's temporaries: the trees' results, and beside them the largest tree's own
+    uint32_t nmax = 0;
+    size_t ws_bytes = 65536 + rtx::bvh_result_bytes(ninst) + (2 * sizeof(float4) + sizeof(uint32_t)) * (size_t)ninst +
+                      (sizeof(rtx::InstBuild) + sizeof(rtx::MeshRef)) * (nm + 1);
+    for (size_t m = 0; m < nm; m++) {
+        if (!used[m]) continue;
+        nmax = std::max(nmax, c->meshes[m].ni);
+        ws_bytes += rtx::bvh_result_bytes(c->meshes[m].ni);
+    }
+    ws_bytes += 5 * sizeof(float4) * (size_t)nmax + rtx::bvh_workspace_bytes(std::max(nmax, ninst));
+    rtx::BuildWorkspace ws(c->device, ws_bytes);
     // bottom level: one tree per mesh in use
-    BvhSet bl;
-    bl.v.resize(nm);
+    std::vector<rtx::BuiltBVH> bl(nm);
     b->blas_root.assign(nm, rtx::kEmptyRoot);
     b->blas_box.assign(6 * (nm ? nm : 1), 0.f);
+    std::vector<rtx::InstBuild> one(nm ? nm : 1);
     {
-        uint32_t nmax = 0;
-        for (size_t m = 0; m < nm; m++)
-            if (used[m]) nmax = std::max(nmax, c->meshes[m].ni);
         std::vector<rtx::MeshRef> mr(nm ? nm : 1);
         for (size_t m = 0; m < nm; m++)
             mr[m] = rtx::MeshRef{c->meshes[m].d_v, c->meshes[m].d_i, c->meshes[m].nv, c->meshes[m].ni};
-        Tmp<rtx::InstBuild> d_one;
-        Tmp<rtx::MeshRef> d_mr;
-        Tmp<float4> d_tw, d_plo, d_phi;
-        if ((e = hipMalloc((void**)&d_one.p, sizeof(rtx::InstBuild) * nm + sizeof(rtx::InstBuild))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(insts)"));
-        if ((e = hipMalloc((void**)&d_mr.p, sizeof(rtx::MeshRef) * mr.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(meshes)"));
-        if ((e = hipMalloc((void**)&d_tw.p, sizeof(float4) * 3 * (nmax ? nmax : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(triangles)"));
-        if ((e = hipMalloc((void**)&d_plo.p, sizeof(float4) * (nmax ? nmax : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
-        if ((e = hipMalloc((void**)&d_phi.p, sizeof(float4) * (nmax ? nmax : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
-        if ((e = hipMemcpyAsync(d_mr.p, mr.data(), sizeof(rtx::MeshRef) * mr.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload meshes"));
+        rtx::InstBuild* d_one = nullptr;
+        rtx::MeshRef* d_mr = nullptr;
+        float4 *d_tw = nullptr, *d_plo = nullptr, *d_phi = nullptr;
+        if ((e = ws.get(&d_one, one.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(insts)"));
+        if ((e = ws.get(&d_mr, mr.size())) != hipSuccess) return bail(hip_fail(e, "hipMalloc(meshes)"));
+        if ((e = ws.get(&d_tw, 3 * (size_t)nmax)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(triangles)"));
+        if ((e = ws.get(&d_plo, nmax)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
+        if ((e = ws.get(&d_phi, nmax)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(bounds)"));
+        if ((e = hipMemcpyAsync(d_mr, mr.data(), sizeof(rtx::MeshRef) * mr.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload meshes"));
+        rtx::BvhOptions opt;
+        opt.owned = false;
         // one identity instance per mesh (object space), uploaded at once
-        std::vector<rtx::InstBuild> one(nm ? nm : 1);
         for (size_t m = 0; m < nm; m++) {
             std::memcpy(one[m].xf, kIdentity, sizeof(one[m].xf));
             one[m].mesh = (uint32_t)m;
             one[m].tri_base = 0;
         }
-        if ((e = hipMemcpyAsync(d_one.p, one.data(), sizeof(rtx::InstBuild) * one.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload insts"));
+        if ((e = hipMemcpyAsync(d_one, one.data(), sizeof(rtx::InstBuild) * one.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload insts"));
         for (size_t m = 0; m < nm; m++) {
             if (!used[m]) continue;
             const uint32_t ni = c->meshes[m].ni;
-            if ((e = rtx::flatten_scene(d_one.p + m, 1, d_mr.p, ni, d_tw.p, d_plo.p, d_phi.p, s)) != hipSuccess) return bail(hip_fail(e, "flatten"));
-            if ((e = rtx::build_bvh(d_tw.p, d_plo.p, d_phi.p, ni, s, &bl.v[m], &err)) != hipSuccess)
+            if ((e = rtx::flatten_scene(d_one + m, 1, d_mr, ni, d_tw, d_plo, d_phi, s)) != hipSuccess) return bail(hip_fail(e, "flatten"));
+            if ((e = rtx::build_bvh(d_tw, d_plo, d_phi, ni, s, ws, &bl[m], &err, opt)) != hipSuccess)
                 return bail(fail(e == hipErrorOutOfMemory ? RTX_ERROR_OUT_OF_MEMORY : RTX_ERROR_HIP, "build_bvh: " + err));
             for (int k = 0; k < 3; k++) {
-                b->blas_box[6 * m + k] = bl.v[m].root_lo[k];
-                b->blas_box[6 * m + 3 + k] = bl.v[m].root_hi[k];
+                b->blas_box[6 * m + k] = bl[m].root_lo[k];
+                b->blas_box[6 * m + 3 + k] = bl[m].root_hi[k];
             }
         }
     }
@@ -793,12 +808,12 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
         tri_base[m] = tri_total;
         tri_total += (uint64_t)c->meshes[m].ni + 1;
         node_off[m] = blas_nodes;
-        blas_nodes += bl.v[m].num_wide;
-        blas_depth = std::max(blas_depth, bl.v[m].max_depth);
-        blas_wide_depth = std::max(blas_wide_depth, bl.v[m].wide_depth);
-        max_leaf = std::max(max_leaf, bl.v[m].max_leaf);
-        num_nodes += bl.v[m].num_nodes;
-        num_leaves += bl.v[m].num_leaves;
+        blas_nodes += bl[m].num_wide;
+        blas_depth = std::max(blas_depth, bl[m].max_depth);
+        blas_wide_depth = std::max(blas_wide_depth, bl[m].wide_depth);
+        max_leaf = std::max(max_leaf, bl[m].max_leaf);
+        num_nodes += bl[m].num_nodes;
+        num_leaves += bl[m].num_leaves;
     }
     if (tri_total > rtx::kLeafFirstMask || tri_total * 48u >= (1ull << 32))
         return bail(fail(RTX_ERROR_LIMIT, "rtx_scene_build: mesh triangles above 2^27-1 or 4 GiB"));
@@ -821,22 +836,21 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
         tphi.push_back(wbox[2 * (size_t)i + 1]);
     }
     const uint32_t M = (uint32_t)tl_inst.size();
-    BvhSet tl;
-    tl.v.resize(1);
-    rtx::BuiltBVH& tb = tl.v[0];
-    Tmp<uint32_t> d_inst_of;
+    rtx::BuiltBVH tb;
+    uint32_t* d_inst_of = nullptr;
     if (M) {
-        Tmp<float4> d_tplo, d_tphi;
-        if ((e = hipMalloc((void**)&d_tplo.p, sizeof(float4) * M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
-        if ((e = hipMalloc((void**)&d_tphi.p, sizeof(float4) * M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
-        if ((e = hipMalloc((void**)&d_inst_of.p, sizeof(uint32_t) * M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance ids)"));
-        if ((e = hipMemcpyAsync(d_tplo.p, tplo.data(), sizeof(float4) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload boxes"));
-        if ((e = hipMemcpyAsync(d_tphi.p, tphi.data(), sizeof(float4) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload boxes"));
-        if ((e = hipMemcpyAsync(d_inst_of.p, tl_inst.data(), sizeof(uint32_t) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload ids"));
+        float4 *d_tplo = nullptr, *d_tphi = nullptr;
+        if ((e = ws.get(&d_tplo, M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
+        if ((e = ws.get(&d_tphi, M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance boxes)"));
+        if ((e = ws.get(&d_inst_of, M)) != hipSuccess) return bail(hip_fail(e, "hipMalloc(instance ids)"));
+        if ((e = hipMemcpyAsync(d_tplo, tplo.data(), sizeof(float4) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload boxes"));
+        if ((e = hipMemcpyAsync(d_tphi, tphi.data(), sizeof(float4) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload boxes"));
+        if ((e = hipMemcpyAsync(d_inst_of, tl_inst.data(), sizeof(uint32_t) * M, hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload ids"));
         rtx::BvhOptions opt;
         opt.max_leaf = 1;
         opt.gather = false;
-        if ((e = rtx::build_bvh(nullptr, d_tplo.p, d_tphi.p, M, s, &tb, &err, opt)) != hipSuccess)
+        opt.owned = false;
+        if ((e = rtx::build_bvh(nullptr, d_tplo, d_tphi, M, s, ws, &tb, &err, opt)) != hipSuccess)
             return bail(fail(e == hipErrorOutOfMemory ? RTX_ERROR_OUT_OF_MEMORY : RTX_ERROR_HIP, "build_bvh (top level): " + err));
     }
     const uint64_t total_nodes = (uint64_t)tb.num_wide + blas_nodes;
@@ -847,15 +861,15 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     if ((e = hipMalloc((void**)&b->tris, sizeof(float4) * 3 * (tri_total ? tri_total : 1))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(triangles)"));
     if (tb.num_wide) {
         if ((e = hipMemcpyAsync(b->nodes, tb.nodes, sizeof(float4) * rtx::kWideNodeF4 * tb.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy top level"));
-        if ((e = rtx::tlas_leaves(b->nodes, tb.num_wide, tb.order, M, d_inst_of.p, ninst, s)) != hipSuccess) return bail(hip_fail(e, "top-level leaves"));
+        if ((e = rtx::tlas_leaves(b->nodes, tb.num_wide, tb.order, M, d_inst_of, ninst, s)) != hipSuccess) return bail(hip_fail(e, "top-level leaves"));
     }
     // one scale for the planes of every tree
     float plane_scale = M ? tb.plane_scale : 1.f;
     for (size_t m = 0; m < nm; m++)
-        if (used[m]) plane_scale = std::max(plane_scale, bl.v[m].plane_scale);
+        if (used[m]) plane_scale = std::max(plane_scale, bl[m].plane_scale);
     for (size_t m = 0; m < nm; m++) {
         if (!used[m]) continue;
-        const rtx::BuiltBVH& x = bl.v[m];
+        const rtx::BuiltBVH& x = bl[m];
         const uint32_t nb = (uint32_t)(tb.num_wide + node_off[m]), tbm = (uint32_t)tri_base[m];
         if (x.num_wide) {
             if ((e = hipMemcpyAsync(b->nodes + (size_t)rtx::kWideNodeF4 * nb, x.nodes, sizeof(float4) * rtx::kWideNodeF4 * x.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy bottom level"));
@@ -894,6 +908,7 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     if ((e = hipMemcpyAsync(b->d_hdr, &b->hdr, sizeof(rtx::DevScene), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload handle"));
     if ((e = hipEventRecord(e1, s)) != hipSuccess) return bail(hip_fail(e, "hipEventRecord"));
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return bail(hip_fail(e, "hipStreamSynchronize"));
+    ws.done();
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);

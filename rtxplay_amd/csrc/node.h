@@ -37,10 +37,13 @@ __device__ inline uint32_t half_up(double v) { return half_down(-v) ^ 0x8000u; }
 // the scale of a tree whose bounds are `extent` wide at most: extents fill
 // 2^11 of the halves' 2^16 range, so that a refit may move things 2^5 times as
 // far apart before planes become infinite (still correct, only looser)
-inline float plane_scale_for(float extent) {
+__host__ __device__ inline float plane_scale_for(float extent) {
     int e = 0;
     (void)frexpf(extent > 1e-30f && extent < 1e30f ? extent : 1.f, &e);
     return ldexpf(1.f, e - 11);
+}
+__host__ __device__ inline float plane_scale_of(const float4& lo, const float4& hi) {
+    return plane_scale_for(fmaxf(fmaxf(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z));
 }
 
 // lo, hi: the children's boxes; used: which slots hold one
