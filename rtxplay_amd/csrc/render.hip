@@ -691,13 +691,36 @@ hipError_t launch_frame(const RenderArgs& a, const LaunchScratch& ls, hipStream_
     return hipGetLastError();
 }
 
+// Finished lanes that trigger a wave's shading step where the caller left the
+// default: a wave that shades together starts its next rays together.  While
+// the lanes' paths are of one length (few samples per pixel: neighbouring
+// pixels at the same bounce) their rays then stay coherent, which is worth
+// the wait; with many samples the lanes drift apart and waiting only idles
+// them.  Measured against 40, flat scenes of levels 2, 4 and 6 / two-level
+// ones at 1080p: 1 to 8 samples 1.10 to 1.25x / 1.00 to 1.09x; 12 to 20
+// samples 1.02 to 1.08x at 50, but 0.98 to 1.15x at 58; 60 samples 1.00x at
+// 50 and 0.94x at 60 (two-level, 20 samples: 1.00x at 44, 0.98x at 56).
+// Batches, whose lanes hold pixels of several frames: 1.03 to 1.15x / 1.01 to
+// 1.05x.  Spread frames and the adjoint (few lanes, long serial paths) gain
+// nothing from more than 40.
+constexpr uint32_t kFewSpp = 8;
+uint32_t frame_batch(const LaunchScratch& ls, const Job& j, uint32_t spp) {
+    if (ls.shade_batch != kShadeBatch) return ls.shade_batch;
+    if (j.sc.xinst) return spp <= kFewSpp ? 52u : 44u;
+    return spp <= kFewSpp ? 58u : 50u;
+}
+uint32_t mixed_batch(const LaunchScratch& ls, const Job& first) {
+    if (ls.shade_batch != kShadeBatch) return ls.shade_batch;
+    return first.sc.xinst ? 48u : 54u;
+}
+
 RenderArgs base_args(const LaunchScratch& ls) {
     RenderArgs a;
     std::memset(&a, 0, sizeof(a));
     a.counter = ls.counter;
     a.gstack = ls.gstack;
     a.gstride = ls.gstride;
-    a.batch = ls.shade_batch ? ls.shade_batch : 40u;
+    a.batch = ls.shade_batch;
     a.inner_frac = ls.inner_frac ? ls.inner_frac : 36u;
     a.tile_log2w = log2u(ls.tile_w ? ls.tile_w : 8u);
     a.iterative = ls.iterative;
@@ -742,6 +765,7 @@ void order_tiles(RenderArgs& a, const LaunchScratch& ls, hipStream_t s) {
     p.dldi = nullptr;
     p.dparams = nullptr;
     p.tape = nullptr;
+    p.batch = frame_batch(ls, a.job, 1u);
     hipLaunchKernelGGL(k_zero_n, dim3((ntiles + 255u) / 256u), dim3(256), 0, s, ls.tile_cost, ntiles);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     const dim3 g(ls.grid), b(kRenderBlock);
@@ -783,9 +807,13 @@ namespace {
 // 0.641 ms).  With two pixels per lane and more the waves stay full, and
 // neighbouring rays share cache lines (1100x640 and 1280x720 at 8 and 4 spp:
 // 2 % slower spread); those of 16+ spp go longest first (kOrderMinSpp).
+// (and sets the shading batch)
 void spread_pixels(RenderArgs& a, const LaunchScratch& ls) {
     const uint32_t waves = ls.grid * (kRenderBlock / 64u);
-    if (a.tile_order || a.nwork >= kOrderMinPixelsPerLane * waves * 64u) return;
+    if (a.tile_order || a.nwork >= kOrderMinPixelsPerLane * waves * 64u) {
+        a.batch = frame_batch(ls, a.job, a.job.lp.spp);
+        return;
+    }
     const uint32_t half = (waves + 1u) / 2u;
     a.lanes = std::min(64u, (a.nwork + half - 1u) / half);
     a.spread = (a.nwork + a.lanes - 1u) / a.lanes;
@@ -825,6 +853,7 @@ hipError_t launch_render_batch(const Job* d_jobs, const Job& first, uint32_t njo
     a.jobs = d_jobs;
     a.njobs = njobs;
     a.nwork = nwork;
+    a.batch = mixed_batch(ls, first);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     const dim3 g(ls.grid), b(kRenderBlock);
     if (first.sc.xinst) {
