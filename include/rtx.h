@@ -254,16 +254,17 @@ rtx_status rtx_get_semantics(rtx_ctx* ctx, int* mode);
  * once != 0 launches the 1x1 picker path (lp->picker).  A frame of 16 or more
  * spp and at least two pixels per lane of the persistent grid first runs a
  * one-sample probe and renders its 64-pixel tiles in descending order of the
- * probe's rays (the pixels do not depend on the order); the first such launch
- * of a context allocates the order's arrays (8 bytes per tile). */
+ * probe's cost, the most expensive pixels in waves of fewer lanes (the pixels
+ * depend on neither); the first such launch of a context allocates the order's
+ * arrays (136 bytes per tile). */
 rtx_status rtx_launch(rtx_ctx* ctx, const rtx_lp_general* lp, int once, void* stream);
 
 /* rtx_launch without device allocation.  No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and the same pixels as rtx_launch; every scratch buffer of the
- * launch (work counter, probe counts and tile order, traversal-stack
- * overflow) lives in one static device array of 48 MiB per GPU, which the
+ * launch (work counter, probe costs and tile order, traversal-stack
+ * overflow) lives in one static device array of 80 MiB per GPU, which the
  * library holds until the process ends.  Limits, each rejected with
  * RTX_ERROR_LIMIT before anything is launched: a frame rendered in probe
  * order (as rtx_launch describes) may have at most 2^18 tiles (2^24
@@ -313,8 +314,8 @@ rtx_status rtx_scene_get_materials(rtx_ctx* ctx, uint64_t is_handle, float* para
  * hold the discrete path structure fixed (hit triangles, reflect/refract and
  * absorb decisions), the interior derivative; pixels whose mean clamps to 0
  * or 1 pass no gradient.  Sums use float atomics, so the last bits vary
- * from run to run.  Frames that rtx_launch renders in probe order are
- * replayed in the same kind of order. */
+ * from run to run.  Frames of 16 or more spp and at least two pixels per five
+ * lanes of the persistent grid are replayed in probe order. */
 rtx_status rtx_launch_adjoint(rtx_ctx* ctx, const rtx_lp_general* lp, const rtx_float3* dL_drgb, float* d_params,
                               void* stream);
 

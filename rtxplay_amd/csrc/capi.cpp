@@ -117,15 +117,16 @@ struct Tmp {
 
 // ---- scratch of rtx_launch_noalloc ------------------------------------------
 // One static device array holds every scratch buffer of a no-allocation
-// launch: the work counter (first 256 bytes), the probe's rays per tile and
-// the tile order (kNoAllocTiles entries each), then the traversal stack's
-// overflow area (the rest).  Each GPU the library runs on holds its own copy
+// launch: the work counter (first 256 bytes), the tiles' costs and the tile
+// order (kNoAllocTiles entries each), the traversal stack's overflow area, and
+// from kNoAllocPixOffset on the probe's cost per pixel.  Each GPU the library runs on holds its own copy
 // until the process ends.  Its device address is looked up once per device
 // (noalloc_setup, from rtx_ctx_create with that device current); host code
 // uses that address, never the array's name.
-constexpr size_t kNoAllocBytes = (size_t)48 << 20;
 constexpr uint32_t kNoAllocTiles = 1u << 18;   // frames of up to 2^24 pixels render in probe order
 constexpr size_t kNoAllocStackOffset = 256 + 2 * sizeof(uint32_t) * (size_t)kNoAllocTiles;
+constexpr size_t kNoAllocPixOffset = (size_t)48 << 20;   // (the stack's area ends here)
+constexpr size_t kNoAllocBytes = kNoAllocPixOffset + sizeof(uint16_t) * 64 * (size_t)kNoAllocTiles;
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
 namespace {
@@ -174,7 +175,7 @@ static rtx_status alloc_scratch(rtx::LaunchScratch& ls, uint32_t blocks_per_cu, 
     ls.grid = blocks_per_cu * (uint32_t)num_cus;
     ls.grid_max = ls.grid;
     ls.gstride = ls.grid * (uint32_t)block;
-    HIP_OK(hipMalloc((void**)&ls.counter, sizeof(uint32_t)));
+    HIP_OK(hipMalloc((void**)&ls.counter, 4 * sizeof(uint32_t)));
     return RTX_SUCCESS;
 }
 
@@ -195,7 +196,7 @@ static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need) {
     return RTX_SUCCESS;
 }
 
-// the probe cost and tile order arrays of ordered frames (a few hundred KB),
+// the probe cost and tile order arrays of ordered frames (136 bytes per tile),
 // allocated by the first launch that needs them and grown with the frame
 static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles) {
     if (ls.tile_cost && ls.tile_cap >= ntiles) return RTX_SUCCESS;
@@ -203,14 +204,18 @@ static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles) {
         HIP_OK(hipDeviceSynchronize());
         HIP_OK(hipFree(ls.tile_cost));
         HIP_OK(hipFree(ls.tile_order));
+        HIP_OK(hipFree(ls.pix_cost));
         ls.tile_cost = ls.tile_order = nullptr;
+        ls.pix_cost = nullptr;
         ls.tile_cap = 0;
     }
     HIP_OK(hipMalloc((void**)&ls.tile_cost, sizeof(uint32_t) * (size_t)ntiles));
     hipError_t e = hipMalloc((void**)&ls.tile_order, sizeof(uint32_t) * (size_t)ntiles);
+    if (e == hipSuccess) e = hipMalloc((void**)&ls.pix_cost, sizeof(uint16_t) * 64u * (size_t)ntiles);
     if (e != hipSuccess) {
         (void)hipFree(ls.tile_cost);
-        ls.tile_cost = nullptr;
+        if (ls.tile_order) (void)hipFree(ls.tile_order);
+        ls.tile_cost = ls.tile_order = nullptr;
         return hip_fail(e, "hipMalloc(tile_order)");
     }
     ls.tile_cap = ntiles;
@@ -269,6 +274,7 @@ rtx_status rtx_ctx_destroy(rtx_ctx* c) {
         if (ls->gstack) (void)hipFree(ls->gstack);
         if (ls->tile_cost) (void)hipFree(ls->tile_cost);
         if (ls->tile_order) (void)hipFree(ls->tile_order);
+        if (ls->pix_cost) (void)hipFree(ls->pix_cost);
     }
     if (c->tape) (void)hipFree(c->tape);
     bool last;
@@ -1137,15 +1143,16 @@ rtx_status rtx_launch_noalloc(rtx_ctx* c, const rtx_lp_general* lp, int once, vo
     rtx::LaunchScratch ls = c->render_ls;
     const uint32_t over = b->stack_need > ls.stack_lds ? b->stack_need - ls.stack_lds : 1u;
     const size_t stack_bytes = sizeof(uint32_t) * (size_t)over * ls.gstride;
-    if (stack_bytes > kNoAllocBytes - kNoAllocStackOffset)
+    if (stack_bytes > kNoAllocPixOffset - kNoAllocStackOffset)
         return fail(RTX_ERROR_LIMIT, "rtx_launch_noalloc: the scene's traversal stack needs " +
                                          std::to_string(stack_bytes) + " bytes of overflow for " +
                                          std::to_string(ls.gstride) + " lanes, more than the " +
-                                         std::to_string(kNoAllocBytes - kNoAllocStackOffset) + " of the static scratch");
+                                         std::to_string(kNoAllocPixOffset - kNoAllocStackOffset) + " of the static scratch");
     ls.counter = (uint32_t*)base;
     ls.tile_cost = (uint32_t*)(base + 256);
     ls.tile_order = ls.tile_cost + kNoAllocTiles;
     ls.tile_cap = kNoAllocTiles;
+    ls.pix_cost = (uint16_t*)(base + kNoAllocPixOffset);
     ls.gstack = (uint32_t*)(base + kNoAllocStackOffset);
     ls.gstack_entries = over;
     HIP_OK(hipSetDevice(c->device));
@@ -1388,7 +1395,7 @@ rtx_status rtx_launch_adjoint(rtx_ctx* c, const rtx_lp_general* lp, const rtx_fl
         HIP_OK(hipMalloc((void**)&c->tape, words * sizeof(uint32_t)));
         c->tape_depth = lp->depth;
     }
-    if (rtx::frame_ordered(*lp, c->render_ls))
+    if (rtx::frame_ordered(*lp, c->render_ls, true))
         if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w))) return st;
     const float3 amb = make_float3(c->ambient.x, c->ambient.y, c->ambient.z);
     hipError_t e = rtx::launch_adjoint(b->hdr, *lp, amb, c->render_ls, dL_drgb, d_params, c->tape,

@@ -16,7 +16,7 @@ constexpr uint32_t kShadeBatch = 40;   // default shading batch (left at it, who
 
 // per-context scratch for the persistent kernels
 struct LaunchScratch {
-    uint32_t* counter = nullptr;   // work counter (device)
+    uint32_t* counter = nullptr;   // work counter and the ordered frames' narrow waves (device, 4 words)
     uint32_t* gstack = nullptr;    // traversal stack overflow (device)
     uint32_t gstride = 0;          // lanes covered by gstack (grid * block)
     uint32_t grid = 0;             // persistent grid size in blocks
@@ -26,25 +26,33 @@ struct LaunchScratch {
     uint32_t stack_lds = kStackLDS;   // render: traversal stack entries per lane in LDS (16 or 32)
     uint32_t grid_max = 0;         // blocks the overflow stack area was sized for
     uint32_t gstack_entries = 0;   // overflow entries per lane (beyond the smallest LDS part)
-    uint32_t* tile_cost = nullptr;   // render: rays per tile of the one-sample probe (device)
+    uint16_t* pix_cost = nullptr;    // render: cost of each work slot's pixel in the one-sample probe (device)
+    uint32_t* tile_cost = nullptr;   // render: cost of each tile from them (device)
     uint32_t* tile_order = nullptr;  // render: the tiles in descending probe cost (device)
-    uint32_t tile_cap = 0;           // tiles the two arrays hold
+    uint32_t tile_cap = 0;           // tiles the three arrays hold
     uint32_t iterative = 0;          // render: 1 = the iterative programs' semantics, 0 = the recursive ones
 };
 
 // Plain frames of at least kOrderMinSpp samples per pixel and at least
 // kOrderMinPixelsPerLane pixels per lane of the persistent grid render their
-// tiles longest first: a one-sample probe launch counts each tile's rays, and
-// the frame takes its tiles in descending order of that count (stable, so
-// equal counts keep their order).  A lane renders whole pixels, so at the end
+// tiles longest first: a one-sample probe launch counts the node visits and
+// rays of each pixel, a tile's cost is the largest sum of a neighbourhood in
+// it, and the frame takes its tiles in descending order of that (stable, so
+// equal costs keep their order).  A lane renders whole pixels, so at the end
 // of a frame a wave waits for its most expensive last pixel; longest first
-// makes the last pixels cheap ones.  A frame with fewer pixels than that has
-// no such tail to shorten, and the probe would only add its time.  No pixel
-// depends on the order.
+// makes the last pixels cheap ones, and the most expensive pixels get waves
+// of fewer lanes.  A smaller frame is spread instead (from 1.4 to 2 pixels per
+// lane, ordered against spread: level 4 1.00 to 1.17x, level 6 0.86x, mixed
+// levels 0.79 to 0.90x).  The adjoint, of whose blocks three of four are
+// resident at once, orders frames from 2 pixels per 5 lanes on (640x360:
+// 1.06x, 480x270: 1.07x, 900x500: 1.07x; 320x180: 0.96x, 200x120: 0.90x).
+// No pixel depends on the order.
 constexpr uint32_t kOrderMinSpp = 16;
 constexpr uint32_t kOrderMinPixelsPerLane = 2;
-inline bool frame_ordered(const rtx_lp_general& lp, const LaunchScratch& ls) {
-    return lp.spp >= kOrderMinSpp && (uint64_t)lp.image_w * lp.image_h >= (uint64_t)kOrderMinPixelsPerLane * ls.gstride;
+inline bool frame_ordered(const rtx_lp_general& lp, const LaunchScratch& ls, bool adjoint = false) {
+    const uint64_t px = (uint64_t)lp.image_w * lp.image_h;
+    return lp.spp >= kOrderMinSpp &&
+           (adjoint ? 5 * px >= 2 * (uint64_t)ls.gstride : px >= (uint64_t)kOrderMinPixelsPerLane * ls.gstride);
 }
 // tiles of a frame (64 work slots each) for a tile width
 inline uint32_t frame_tiles(const rtx_lp_general& lp, uint32_t tile_w) {

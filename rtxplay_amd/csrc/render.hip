@@ -63,8 +63,9 @@ struct RenderArgs {
     uint32_t lds_grad;        // 1: accumulate per block in LDS first (num_insts x 4 floats)
     // plain frames: the tile of each tile slot (nullptr: slot order)
     const uint32_t* tile_order;
-    // probe launch: rays per tile (one sample per pixel, nothing else written)
-    uint32_t* tile_cost;
+    // probe launch: the cost of each work slot's pixel (one sample per pixel,
+    // nothing else written)
+    uint16_t* pix_cost;
     // 1: the iterative programs' semantics (optx/camera_i.cu, optx/optics_i.cu),
     // 0: the recursive ones (optx/camera_r.cu, optx/optics_r.cu)
     uint32_t iterative;
@@ -109,6 +110,32 @@ __device__ __forceinline__ uint32_t find_job(const Job* jobs, uint32_t njobs, ui
 #endif
 constexpr bool kCompactLeaves = RTX_COMPACT_LEAVES != 0;
 
+// Narrow waves.  A lane renders whole pixels, one sample after the other, and
+// a node visit takes 1.6 us in a full wave, whose lanes wait for each other's
+// leaves and shading, but about half of that where few lanes are active.  So
+// in an ordered frame the pixels that would last longer than the frame in a
+// full wave go to waves that use 8, 16 or 32 of their lanes, by their
+// predicted cost (k_tile_order plans them): the last waves of the 720p
+// 50-sample frame ended at 27 ms where the others' mean was 19.5.  A narrow
+// wave stays narrow when it takes further pixels.  Measured (ordered without
+// -> with): 1280x720, 50 samples, level 4 27.4 -> 23.5 ms; 1000x560, 32
+// samples, level 5 19.6 -> 16.6; 1100x620, 100 samples, mixed levels 112 -> 87;
+// 1500x800, 20 samples, level 3 16.3 -> 14.5; 1080p, 100 samples, level 6,
+// which has no such pixels, 100.9 -> 101.1.
+constexpr uint32_t kNarrowGroups = 3;
+__device__ __forceinline__ uint32_t narrow_lanes(uint32_t g) { return 8u << g; }
+// The frame's even time, as a tile cost: kNarrowLevel x pixels per lane x the
+// mean tile cost (0.5, 0.65, 0.8 and 1.0 on the 720p frame: 27.4, 23.5, 24.3
+// and 25.9 ms).  A pixel of cost c lasts c * (kNarrowBase + (1 - kNarrowBase) *
+// lanes / 64).  At most kNarrowMax of the waves are narrow (a half is 9 %
+// slower than 3/8 on the adjoint of a 900x500 frame, whose launch has three
+// quarters of the waves resident).
+constexpr float kNarrowLevel = 0.65f, kNarrowBase = 0.5f, kNarrowMax = 0.375f;
+
+// probe: a ray's start, leaves and shading in node visits (a fifth of the
+// waves' time at some 23 visits a ray)
+constexpr uint32_t kProbeRayCost = 6;
+
 template <int BLOCK, bool COUNT, bool BATCH, int SLDS, bool ADJ = false, bool TL = false, bool PROBE = false,
           int TOPN = 0>
 __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_stack, float* s_grad = nullptr,
@@ -126,7 +153,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
     const Job* J = BATCH ? a.jobs : &a.job;
     DevScene sc = a.job.sc;
     uint32_t W = a.job.lp.image_w, H = a.job.lp.image_h, spp = PROBE ? 1u : a.job.lp.spp, maxd = a.job.lp.depth;
-    uint32_t tslot = 0;   // probe: tile slot of the lane's pixel
+    uint32_t tslot = 0;   // probe: work slot of the lane's pixel
 
     bool active = false, exhausted = false, going = false;
     uint32_t x = 0, y = 0, sample = 0, k = 0, rpp = 0;
@@ -168,16 +195,36 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
     bool newsample = false, cont = false;
     float3 ro = f3(0.f, 0.f, 0.f), rdv = f3(0.f, 0.f, 1.f);
 
+    // a narrow wave starts with its own part of the order's head
+    uint32_t lanes = a.lanes, batch = a.batch, head = ~0u;
+    if (!BATCH && !COUNT && !PROBE && a.tile_order) {
+        const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)));
+        uint32_t w0 = 0, p0 = 0;
+        for (uint32_t g = 0; g < kNarrowGroups && head == ~0u; g++) {
+            const uint32_t n = a.counter[1 + g], nl = narrow_lanes(g);
+            if (wave - w0 < n) {
+                lanes = nl;
+                batch = max(1u, batch * nl / 64u);
+                head = p0 + (wave - w0) * nl;
+            }
+            w0 += n;
+            p0 += n * nl;
+        }
+    }
+
     for (;;) {
         // lanes without a pixel take one; tile slots outside the frame are skipped
         for (;;) {
-            const bool need = !active && !exhausted && lane < a.lanes;
+            const bool need = !active && !exhausted && lane < lanes;
             const uint64_t mask = __ballot(need);
             if (mask == 0) break;
             const uint32_t leader = __ffsll((unsigned long long)mask) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(a.counter, (uint32_t)__popcll(mask));
-            base = __shfl(base, leader, 64);
+            uint32_t base = head;
+            if (head == ~0u) {
+                if (lane == leader) base = atomicAdd(a.counter, (uint32_t)__popcll(mask));
+                base = __shfl(base, leader, 64);
+            }
+            head = ~0u;
             if (need) {
                 const uint32_t wi = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
                 if (wi >= a.nwork) {
@@ -198,7 +245,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
                     }
                     const uint32_t in = li & 63u;
                     const uint32_t tile = !BATCH && a.tile_order ? a.tile_order[li >> 6] : li >> 6;
-                    if (PROBE) tslot = li >> 6;
+                    if (PROBE) tslot = li;
                     x = (tile % J->tiles_x) * tw + (in & (tw - 1u));
                     y = (tile / J->tiles_x) * (64u / tw) + (in >> a.tile_log2w);
                     if (x < W && y < H) {
@@ -248,7 +295,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
         // traverse until a batch of lanes has a final closest hit; the others
         // keep their traversal state and resume after the shading below
         const uint64_t c0 = COUNT ? clock64() : 0;
-        trav_run<BLOCK, COUNT, TL, BATCH, TOPN, CL>(sc, tv, going, active, (int)a.batch,
+        trav_run<BLOCK, COUNT, TL, BATCH, TOPN, CL, PROBE>(sc, tv, going, active, (int)batch,
                                                                      (int)a.inner_frac, stk, &cnt_nodes, &cnt_tris,
                                                                      wave_iters, top, cl);
         if (COUNT) cyc_trav += clock64() - c0;
@@ -430,7 +477,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
             if (++sample == spp && ADJ) {
                 active = false;
             } else if (sample == spp && PROBE) {
-                atomicAdd(&a.tile_cost[tslot], rpp);
+                a.pix_cost[tslot] = (uint16_t)min(cnt_nodes + kProbeRayCost * rpp, 65535u);
                 active = false;
             } else if (sample == spp) {
                 const rtx_lp_general& lp = J->lp;
@@ -506,31 +553,96 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_RENDE
     render_body<BLOCK, false, false, SLDS, false, TL, true, TOPN>(a, s_stack, nullptr, (const lds_f4*)s_top);
 }
 
-__global__ void k_zero_n(uint32_t* p, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
+// The cost of a tile: the largest sum of the probe's costs over the 5x5 pixels
+// (those inside the frame) around any of its pixels; a wave per tile, a lane
+// per pixel.  What a tile delays is its most expensive pixel, and one sample
+// predicts a pixel badly but its neighbourhood well.  The largest end time of
+// the lanes over their mean, from counted node visits and lanes that take the
+// pixels in this order: 1.08 on the 1080p level-6 frame and on the mixed-level
+// one, 1.29 and 1.26 by the tile's summed rays, 1.01 and 1.08 by the tile's true
+// largest cost (rays in place of visits: 1.11 and 1.12; the tile's largest 4x4
+// sum: 1.18 and 1.13).
+constexpr int kCostReach = 2;
+__global__ __launch_bounds__(256) void k_tile_cost(const uint16_t* __restrict__ pix, uint32_t ntiles, uint32_t tiles_x,
+                                                   uint32_t tile_log2w, int W, int H, uint32_t* __restrict__ cost) {
+    const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6), in = threadIdx.x & 63u;
+    if (t >= ntiles) return;
+    const uint32_t log2h = 6u - tile_log2w, mw = (1u << tile_log2w) - 1u, mh = (1u << log2h) - 1u;
+    const int x = (int)(((t % tiles_x) << tile_log2w) + (in & mw));
+    const int y = (int)(((t / tiles_x) << log2h) + (in >> tile_log2w));
+    uint32_t sum = 0;
+    for (int dy = -kCostReach; dy <= kCostReach; dy++)
+        for (int dx = -kCostReach; dx <= kCostReach; dx++) {
+            const int nx = x + dx, ny = y + dy;
+            if (nx < 0 || ny < 0 || nx >= W || ny >= H) continue;
+            const uint32_t nt = ((uint32_t)ny >> log2h) * tiles_x + ((uint32_t)nx >> tile_log2w);
+            sum += pix[(nt << 6) + (((uint32_t)ny & mh) << tile_log2w) + ((uint32_t)nx & mw)];
+        }
+    if (x >= W || y >= H) sum = 0;
+    for (int m = 32; m; m >>= 1) sum = max(sum, (uint32_t)__shfl_xor((int)sum, m, 64));
+    if (in == 0) cost[t] = sum;
 }
 
-// The tiles in descending probe cost, stable: cost quantised to
-// kOrderBuckets classes (class 0 the most rays), a counting sort in one
-// block.  Each chunk of 1024 tiles ranks its tiles within their class by
-// wave ballots (the lanes of a class found bit by bit) and per-wave class
-// counts, so equal classes keep the tiles' order and the result is the same
-// in every run.
-constexpr uint32_t kOrderBuckets = 64;
+// The tiles in descending cost, stable: cost quantised to kOrderBuckets
+// classes of an eighth of an octave (class 0 the most expensive), a counting
+// sort in one block.  Each chunk of 1024 tiles ranks its tiles within their
+// class by wave ballots (the lanes of a class found bit by bit) and per-wave
+// class counts, so equal classes keep the tiles' order and the result is the
+// same in every run.  Also sets the frame's work counter: counter[1..3] the
+// narrow waves of 8, 16 and 32 lanes, counter[0] the pixels they start with.
+constexpr uint32_t kOrderBuckets = 128;
 constexpr uint32_t kOrderBlock = 1024;
-__global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost, uint32_t n, uint32_t cmax,
-                                                            uint32_t* order) {
+// (3 mantissa bits below the exponent: 2^5 and less is the last class, 2^21 the first)
+__device__ __forceinline__ uint32_t cost_class(float c) {
+    const uint32_t f = __float_as_uint(c) >> 20, f0 = (127u + 5u) << 3;
+    return (kOrderBuckets - 1u) - min(f > f0 ? f - f0 : 0u, kOrderBuckets - 1u);
+}
+__device__ __forceinline__ float class_cost(uint32_t k) {   // the lowest of the class
+    return __uint_as_float(((kOrderBuckets - 1u - k) + ((127u + 5u) << 3)) << 20);
+}
+__global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost, uint32_t n, float level,
+                                                            uint32_t max_narrow, uint32_t* order, uint32_t* counter) {
     __shared__ uint32_t start[kOrderBuckets];                 // running start of each class
     __shared__ uint32_t wcnt[kOrderBlock / 64][kOrderBuckets];  // per wave: class counts, then offsets
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
     auto cls = [&](uint32_t t) -> uint32_t {
-        const uint32_t c = cost[t] < cmax ? cost[t] : cmax;
-        return (kOrderBuckets - 1u) - (uint32_t)(((uint64_t)c * (kOrderBuckets - 1u)) / cmax);
+        return cost_class((float)cost[t]);
     };
+    __shared__ uint64_t s_sum;
     if (tid < kOrderBuckets) start[tid] = 0u;
+    if (tid == 0) s_sum = 0;
     __syncthreads();
-    for (uint32_t t = tid; t < n; t += kOrderBlock) atomicAdd(&start[cls(t)], 1u);
+    uint64_t sum = 0;
+    for (uint32_t t = tid; t < n; t += kOrderBlock) {
+        atomicAdd(&start[cls(t)], 1u);
+        sum += cost[t];
+    }
+    atomicAdd((unsigned long long*)&s_sum, (unsigned long long)sum);
+    __syncthreads();
+    // The narrow waves: lane j of the first wave plans them for a time 2^(j/8)
+    // above the even one; the shortest time with few enough of them is taken.
+    if (tid < 64) {
+        const float T = level * ((float)s_sum / (float)n) * exp2f((float)tid * 0.125f);
+        uint32_t need = 0, px[kNarrowGroups] = {0, 0, 0};
+        for (uint32_t k = 0; k < kOrderBuckets; k++) {
+            const float f = (T / class_cost(k) - kNarrowBase) / (1.f - kNarrowBase);
+            if (f < 0.75f) px[f < 0.1875f ? 0 : f < 0.375f ? 1 : 2] += start[k] * 64u;
+        }
+        uint32_t w[kNarrowGroups];
+        for (uint32_t g = 0; g < kNarrowGroups; g++) {
+            w[g] = (px[g] + narrow_lanes(g) - 1u) / narrow_lanes(g);
+            need += w[g];
+        }
+        const uint64_t ok = __ballot(need <= max_narrow);
+        if (ok ? tid == (uint32_t)(__ffsll((unsigned long long)ok) - 1) : tid == 0) {
+            uint32_t h = 0;
+            for (uint32_t g = 0; g < kNarrowGroups; g++) {
+                counter[1 + g] = ok ? w[g] : 0u;
+                h += (ok ? w[g] : 0u) * narrow_lanes(g);
+            }
+            counter[0] = h;
+        }
+    }
     __syncthreads();
     if (tid == 0) {
         uint32_t s = 0;
@@ -546,7 +658,7 @@ __global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost
         const bool valid = t < n;
         const uint32_t b = valid ? cls(t) : kOrderBuckets;   // past the end: a class of its own
         uint64_t m = ~0ull;
-        for (int bit = 0; bit < 7; bit++) {
+        for (int bit = 0; bit < 8; bit++) {
             const uint64_t v = __ballot((b >> bit) & 1u);
             m &= ((b >> bit) & 1u) ? v : ~v;
         }
@@ -754,19 +866,18 @@ uint32_t render_blocks_per_cu() {
 
 namespace {
 // a frame of kOrderMinSpp or more spp (with the scratch in place): the probe
-// launch (one sample per pixel, rays per tile) and the tile order, which the
-// frame's launch then follows (a.tile_order)
+// launch (one sample per pixel, its cost), the tiles' costs and order, which the
+// frame's launch then follows (a.tile_order), and its work counter
 void order_tiles(RenderArgs& a, const LaunchScratch& ls, hipStream_t s) {
     const uint32_t ntiles = a.job.tiles_x * a.job.tiles_y;
-    if (!frame_ordered(a.job.lp, ls) || !ls.tile_cost || ls.tile_cap < ntiles) return;
+    if (!frame_ordered(a.job.lp, ls, a.dldi != nullptr) || !ls.tile_cost || ls.tile_cap < ntiles) return;
     RenderArgs p = a;
-    p.tile_cost = ls.tile_cost;
+    p.pix_cost = ls.pix_cost;
     p.tile_order = nullptr;
     p.dldi = nullptr;
     p.dparams = nullptr;
     p.tape = nullptr;
     p.batch = frame_batch(ls, a.job, 1u);
-    hipLaunchKernelGGL(k_zero_n, dim3((ntiles + 255u) / 256u), dim3(256), 0, s, ls.tile_cost, ntiles);
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     const dim3 g(ls.grid), b(kRenderBlock);
     if (stage_top_nodes(a.job)) {
@@ -786,8 +897,12 @@ void order_tiles(RenderArgs& a, const LaunchScratch& ls, hipStream_t s) {
             else hipLaunchKernelGGL((k_probe<kRenderBlock, 32, false, 0>), g, b, 0, s, p);
         }
     }
-    hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderBlock), 0, s, ls.tile_cost, ntiles, 64u * a.job.lp.depth,
-                       ls.tile_order);
+    hipLaunchKernelGGL(k_tile_cost, dim3((ntiles + 3u) / 4u), dim3(256), 0, s, ls.pix_cost, ntiles, a.job.tiles_x,
+                       a.tile_log2w, (int)a.job.lp.image_w, (int)a.job.lp.image_h, ls.tile_cost);
+    const uint32_t waves = ls.grid * (kRenderBlock / 64u);
+    hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(kOrderBlock), 0, s, ls.tile_cost, ntiles,
+                       kNarrowLevel * (float)a.nwork / (float)(waves * 64u), (uint32_t)(kNarrowMax * (float)waves),
+                       ls.tile_order, ls.counter);
     a.tile_order = ls.tile_order;
 }
 }  // namespace
@@ -830,7 +945,7 @@ hipError_t launch_render(const DevScene& sc, const rtx_lp_general& lp, float3 am
     a.nwork = a.job.work_end;
     order_tiles(a, ls, s);
     spread_pixels(a, ls);
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
+    if (!a.tile_order) hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     return launch_frame<false>(a, ls, s);
 }
 
@@ -882,7 +997,7 @@ hipError_t launch_adjoint(const DevScene& sc, const rtx_lp_general& lp, float3 a
     if (ng) hipLaunchKernelGGL(k_fill, dim3((ng + 255) / 256), dim3(256), 0, s, dparams, ng, 0.f);
     order_tiles(a, ls, s);
     spread_pixels(a, ls);
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
+    if (!a.tile_order) hipLaunchKernelGGL(k_zero, dim3(1), dim3(1), 0, s, ls.counter);
     const size_t shm = a.lds_grad ? sizeof(float) * ng : 0;
     const dim3 g(ls.grid), b(kRenderBlock);
     if (sc.xinst) {

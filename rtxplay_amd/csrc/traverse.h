@@ -592,8 +592,9 @@ __device__ __forceinline__ void leaves_compact(const DevScene& sc, Trav& s, uint
 // CL: the leaf phase spreads the parked leaves' triangles over the wave
 // (leaves_compact, with the wave's kLeafScratchWords of LDS at `cl`);
 // otherwise each lane tests its own leaves.
+// NN: the lane's node visits are counted in *nn (COUNT: so are more).
 template <int BLOCK, bool COUNT = false, bool TL = false, bool G = false, int TOPN = 0, bool CL = false,
-          class Stack>
+          bool NN = false, class Stack>
 __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& going, bool busy, int batch,
                                          int inner_frac, Stack& st, uint32_t* nn = nullptr,
                                          uint32_t* nt = nullptr, uint32_t* wi = nullptr,
@@ -639,10 +640,8 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
             const uint32_t n_inner = (uint32_t)__popcll(__ballot(below) & m_going);
             step = n_inner >= least;
             if (inner && step) {
-                if (COUNT) {
-                    (*nn)++;
-                    if (first_active_lane()) wi[0]++;
-                }
+                if (COUNT || NN) (*nn)++;
+                if (COUNT && first_active_lane()) wi[0]++;
                 // one 4-wide node: five loads.  The ray reads each axis's
                 // entry and exit planes by its direction signs, so the slab
                 // test needs no min/max per axis; the halves go into the FMAs
