@@ -323,9 +323,24 @@ __device__ __forceinline__ void bins_add(LevelLds& L, const TaskGeom& g, const u
             atomicMax(&L.b[ax][b][9 + k], acc[ax][9 + k]);
         }
     };
+    // (the next primitive's box and the index after it are in flight while one
+    // is binned: 8 M-triangle levels over 1024 blocks 260 -> 226 us each; runs
+    // of 1, 2, 4, 8 and 16 primitives a thread instead, which read whole lines,
+    // flush their bins more often: 0.83, 0.97, 1.04, 1.01 and 0.93x of that
+    // scene's build, against 1.03x, and 0.76 to 0.96x of a 0.5 M-triangle one)
+    float4 a_next = make_float4(0.f, 0.f, 0.f, 0.f), h_next = a_next;
+    uint32_t p_next = 0;
+    if (b0 < b1) {
+        const uint32_t p = idx[b0];
+        p_next = idx[min(b0 + 1u, b1 - 1u)];
+        a_next = plo[p];
+        h_next = phi[p];
+    }
     for (uint32_t i = b0; i < b1; i++) {
-        const uint32_t p = idx[i];
-        const float4 a = plo[p], h = phi[p];
+        const float4 a = a_next, h = h_next;
+        a_next = plo[p_next];
+        h_next = phi[p_next];
+        p_next = idx[min(i + 2u, b1 - 1u)];
         const float c[3] = {.5f * (a.x + h.x), .5f * (a.y + h.y), .5f * (a.z + h.z)};
         const uint32_t v[12] = {f2o(a.x), f2o(a.y), f2o(a.z), f2o(h.x), f2o(h.y), f2o(h.z),
                                 f2o(c[0]), f2o(c[1]), f2o(c[2]), f2o(c[0]), f2o(c[1]), f2o(c[2])};
