@@ -251,7 +251,7 @@ rtx_status rtx_get_semantics(rtx_ctx* ctx, int* mode);
 /* Launcher::ignite, optx/launcher.cxx:49-77 (optixLaunch of the raygen program
  * optx/camera_r.cu:23-121 with the closest-hit programs optx/optics_r.cu).
  * Asynchronous on `stream` (the C++ Launcher syncs, as the reference does).
- * once != 0 launches the 1x1 picker path (lp->picker).  A frame of 16 or more
+ * once != 0 launches the 1x1 picker path (lp->picker).  A frame of 10 or more
  * spp and at least two pixels per lane of the persistent grid first runs a
  * one-sample probe and renders its 64-pixel tiles in descending order of the
  * probe's cost, the most expensive pixels in waves of fewer lanes (the pixels
@@ -268,7 +268,7 @@ rtx_status rtx_launch(rtx_ctx* ctx, const rtx_lp_general* lp, int once, void* st
  * library holds until the process ends.  Limits, each rejected with
  * RTX_ERROR_LIMIT before anything is launched: a frame rendered in probe
  * order (as rtx_launch describes) may have at most 2^18 tiles (2^24
- * pixels), and the scene's stack overflow (entries beyond the context's
+ * pixels; above that, one of fewer than 16 spp renders in slot order), and the scene's stack overflow (entries beyond the context's
  * stack_lds, times the persistent grid's lanes, 4 bytes each) must fit the
  * 46 MiB stack part.  All calls on one GPU share that GPU's array, which
  * keeps the last call's contents (the launch clears what must start at zero

@@ -124,6 +124,7 @@ struct Tmp {
 // (noalloc_setup, from rtx_ctx_create with that device current); host code
 // uses that address, never the array's name.
 constexpr uint32_t kNoAllocTiles = 1u << 18;   // frames of up to 2^24 pixels render in probe order
+constexpr uint32_t kNoAllocOrderSpp = 16;      // from so many samples on, larger ones are refused
 constexpr size_t kNoAllocStackOffset = 256 + 2 * sizeof(uint32_t) * (size_t)kNoAllocTiles;
 constexpr size_t kNoAllocPixOffset = (size_t)48 << 20;   // (the stack's area ends here)
 constexpr size_t kNoAllocBytes = kNoAllocPixOffset + sizeof(uint16_t) * 64 * (size_t)kNoAllocTiles;
@@ -1167,7 +1168,9 @@ rtx_status rtx_launch_noalloc(rtx_ctx* c, const rtx_lp_general* lp, int once, vo
         if (lp->spp == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch_noalloc: spp == 0");
         if (lp->depth == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch_noalloc: depth == 0");
         if (!lp->rawRGB) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch_noalloc: rawRGB is NULL");
-        if (rtx::frame_ordered(*lp, ls) && rtx::frame_tiles(*lp, ls.tile_w) > kNoAllocTiles)
+        // (frames of fewer samples that do not fit render in slot order)
+        if (lp->spp >= kNoAllocOrderSpp && rtx::frame_ordered(*lp, ls) &&
+            rtx::frame_tiles(*lp, ls.tile_w) > kNoAllocTiles)
             return fail(RTX_ERROR_LIMIT, "rtx_launch_noalloc: a frame rendered in probe order has " +
                                              std::to_string(rtx::frame_tiles(*lp, ls.tile_w)) +
                                              " tiles, more than the " + std::to_string(kNoAllocTiles) +

@@ -682,11 +682,10 @@ __global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost
     }
 }
 
-// batch: the same loop with a job per lane, whose job state takes
-// registers: the slab test in its (P - o) * idir form keeps flat scenes at
-// 4 waves per SIMD (7 % faster than the FMA form under that register
-// limit, and 20 % faster than 3 waves); two-level ones take the registers
-// of 3 waves
+// batch: the same loop with a job per lane, whose job state takes registers:
+// flat scenes keep 4 waves per SIMD by a few spills outside the node loop
+// (16 registers; 3 waves without are slower), two-level ones take the
+// registers of 3 waves
 template <int BLOCK, int SLDS, bool TL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_BATCH_WAVES))) void k_render_batch(const RenderArgs a) {
     __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
@@ -921,7 +920,7 @@ namespace {
 // 8 and 64 spp: 4.65 -> 3.87 and 31.9 -> 25.9 ms; 640x360, 1 spp: 0.627 ->
 // 0.641 ms).  With two pixels per lane and more the waves stay full, and
 // neighbouring rays share cache lines (1100x640 and 1280x720 at 8 and 4 spp:
-// 2 % slower spread); those of 16+ spp go longest first (kOrderMinSpp).
+// 2 % slower spread); longer ones go longest first (kOrderMinSpp).
 // (and sets the shading batch)
 void spread_pixels(RenderArgs& a, const LaunchScratch& ls) {
     const uint32_t waves = ls.grid * (kRenderBlock / 64u);

@@ -10,7 +10,7 @@ from test_gpu_parity import say
 pytestmark = pytest.mark.gpu
 
 # below and above two pixels per lane (524,288 on 256 CUs), 8 and 9 samples,
-# 15 and 16 (longest tiles first)
+# 10 to 16 (longest tiles first)
 FRAMES = [(300, 200, 8), (1030, 520, 1), (1030, 520, 8), (1030, 520, 9), (1030, 520, 15), (1030, 520, 16)]
 
 
