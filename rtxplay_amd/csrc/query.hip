@@ -17,11 +17,6 @@ namespace {
 #ifndef RTX_TRACE_BATCH
 #define RTX_TRACE_BATCH 64
 #endif
-// Of the traversing lanes, in 64ths, those that must be able to step for the
-// node phase to go on (2 M / 100 k / 5 k rays and 1 M two-level ones, us: 24:
-// 519, 143, 76, 367; 32: 518, 137, 77, 366; 40: 516, 126, 74, 366; 48: 524,
-// 131, 75, 374).
-constexpr int kTraceInner = 40;
 
 // closest hit for a batch of rays (the optixTrace query on its own):
 // persistent grid, each lane takes rays from one work counter (one atomic
@@ -61,7 +56,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(const DevScene sc, const rtx_ra
             }
         }
         if (!__any(held)) break;
-        trav_run<BLOCK, false, TL>(sc, s, going, held, batch, kTraceInner, stk);
+        trav_run<BLOCK, false, TL>(sc, s, going, held, batch, 32, stk);
         if (!held || going) continue;
         held = false;
         const HitFull h = s.h;
