@@ -13,9 +13,9 @@
 //
 // Rounding is outwards: a plane at p is stored at or beyond p moved out by
 // 2^-20 of its distance from the origin, in exact arithmetic.  That margin
-// covers the rounding of the traversal's (origin - o) * inv where it cancels
-// against half * (plane_scale * inv) (up to 2^-22 of that distance); the
-// error relative to (origin - o) * inv itself is covered by kSlabPad in
+// covers the rounding of the traversal's (origin - o) * idir where it cancels
+// against half * (plane_scale * idir) (up to 2^-22 of that distance); the
+// error relative to the distance itself is covered by kBoxPad in
 // traverse.h.  The origin lies a little below the smallest child's lo plane,
 // so that no plane of a box is at distance 0 of it and a ray that runs within
 // a face of a box (parallel to an axis, through vertices) still meets the box.

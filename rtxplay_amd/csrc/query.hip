@@ -32,7 +32,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(const DevScene sc, const rtx_ra
     stk.init(s_stack, gstack + blockIdx.x * BLOCK + threadIdx.x, gstride);
     const uint32_t lane = threadIdx.x & 63u;
     Trav s;
-    trav_begin<TL>(s, sc, stk.bottom, f3(0.f, 0.f, 0.f), f3(0.f, 0.f, 1.f), 0.f, 0.f);
+    trav_begin(s, sc, stk.bottom, f3(0.f, 0.f, 0.f), f3(0.f, 0.f, 1.f), 0.f, 0.f);
     bool going = false, held = false, exhausted = false;
     uint32_t i = 0;
     for (;;) {
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(BLOCK) void k_trace(const DevScene sc, const rtx_ra
                 i = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
                 if (i < n) {
                     const rtx_ray ray = rays[i];
-                    trav_begin<TL>(s, sc, stk.bottom, f3(ray.ori.x, ray.ori.y, ray.ori.z), f3(ray.dir.x, ray.dir.y, ray.dir.z),
+                    trav_begin(s, sc, stk.bottom, f3(ray.ori.x, ray.ori.y, ray.ori.z), f3(ray.dir.x, ray.dir.y, ray.dir.z),
                                ray.tmin, ray.tmax);
                     held = going = true;
                 } else {

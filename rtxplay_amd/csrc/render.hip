@@ -163,7 +163,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
     float3 thr = f3(1, 1, 1);
     float3 acc = f3(0, 0, 0), nacc = f3(0, 0, 0), aacc = f3(0, 0, 0), gN = f3(0, 0, 0), gA = f3(0, 0, 0);
     Trav tv;
-    trav_begin<TL>(tv, sc, stk.bottom, f3(0, 0, 0), f3(0, 0, 1), 1e-3f, 1e16f);
+    trav_begin(tv, sc, stk.bottom, f3(0, 0, 0), f3(0, 0, 1), 1e-3f, 1e16f);
     uint64_t cyc_trav = 0;
     uint32_t wave_iters[2] = {0, 0};
     const uint64_t cyc_start = COUNT ? clock64() : 0;
@@ -287,7 +287,7 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
             gA = f3(0.f, 0.f, 0.f);
         }
         if (newsample || cont) {
-            trav_begin<TL>(tv, sc, stk.bottom, ro, rdv, 1e-3f, 1e16f);     // optx/optics_r.cu:115-132 for a scattered ray
+            trav_begin(tv, sc, stk.bottom, ro, rdv, 1e-3f, 1e16f);     // optx/optics_r.cu:115-132 for a scattered ray
             going = true;
         }
         newsample = cont = false;
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(64) void k_pick(const RenderArgs a) {
     const float3 o = ld(lp.camera.eye) + off;
     const float3 d = ((s * ld(lp.camera.wvec) + t * ld(lp.camera.hvec)) - ld(lp.camera.dvec)) - off;
     TRay r;
-    tray_init<!TL>(r, o, d, 1e-3f, 1e16f);
+    tray_init(r, o, d, 1e-3f);
     HitFull h;
     traverse<64, TL>(a.job.sc, r, 1e16f, h, stk);
     *lp.pick_id = h.tri == kNoHit ? 0xFFFFFFFFu

@@ -30,36 +30,21 @@
 
 namespace rtx {
 
-// Two forms of the slab test.
-//
-// Flat scenes (REL): slab distances are in units of the best hit so far (tau =
-// (t - tmin) / T, T the best hit's t, TRay::inv), so the clamp of the FMAs to
-// [0, 1] takes the place of a maximum with tmin and a minimum with the hit per
-// child: a box is met where entry < exit, and one beyond the hit or behind
-// tmin has both clamped to the same end.  kSlabPad: how far c = (origin - o) * inv - tmin / T is moved out (down for
-// entry planes, up for exit planes), relative to itself: 2^-20, where its two
-// roundings and the FMA's are within 3 * 2^-24 of the larger of c and the
+// The slab test's distances are in units of the ray's t, clamped by a maximum
+// with tmin and a minimum with the best hit, so any tmin and tmax will do.
+// kBoxPad: the far distance is moved out by 2^-18 of itself, where the
+// roundings of an entry and an exit distance are together within 2^-20 of the
 // distance (the planes' own margin covers what is relative to their distance
-// from the origin, node.h).
-constexpr float kSlabPad = 0x1p-20f;
-// kHitBias: a new hit makes T this much larger than its t, for the roundings
-// of the rescaling and of hits at equal distance
-constexpr float kHitBias = 1.f - 0x1p-20f;
-// T stays in this range (a smaller hit culls like one at the low end)
-constexpr float kLeastT = 1e-9f, kMostT = 1e30f;
-// Two-level scenes: distances are in units of t, clamped by maximum and
-// minimum, with the pad on the far distance: 2^-18, where the roundings of an
-// entry and an exit distance are together within 2^-20 of the distance (the
-// planes' own margin covers the rest).  Eight more instructions per visit, but
-// the two-level kernels have no registers for the rescaling (17 spilled; the
-// 1080p mixed-level frame 101.7 ms against 105.7 ms).
-constexpr float kBoxPad = 1.0000038f;
+// from the node's origin, node.h).  Distances relative to the best hit, whose
+// FMAs the clamp to [0, 1] limits for nothing, save eight instructions a visit
+// but gave 0 to 1 % (3 % on a 400x225 frame of 10 samples), and hold neither
+// for a negative tmin nor, with tmin within them, where tmin is close to the hit.
+constexpr float kBoxPad = 0x1p-18f;
 
 struct TRay {
     float3 o, d;
-    float3 inv;     // 1 / (d * T); REL false: 1 / d
+    float3 idir;    // 1 / d
     float tmin;
-    float stmin;    // REL: tmin / T, a little less
     // the watertight test's axis order (kx, ky, kz) as a rotation that puts
     // the dominant axis kz last (rz0: kz = x, rz1: kz = y, else kz = z).
     // Woop et al. (2013) also swap kx and ky when d[kz] < 0 to keep the
@@ -81,10 +66,7 @@ __device__ __forceinline__ float3 permute(const TRay& r, float3 a) {
     return f3(p, q, w);
 }
 
-__device__ __forceinline__ float tray_T(float t) { return fminf(fmaxf(t, kLeastT), kMostT); }
-
-template <bool REL>
-__device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmin, float tmax) {
+__device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmin) {
     r.o = o;
     r.d = d;
     r.tmin = tmin;
@@ -94,29 +76,16 @@ __device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmi
     r.rz0 = kz == 0;
     r.rz1 = kz == 1;
     const float3 dp = permute(r, d);       // (d[kx], d[ky], d[kz])
-    const float3 idir = f3(1.f / (d.x != 0.f ? d.x : 1e-24f), 1.f / (d.y != 0.f ? d.y : 1e-24f),
-                           1.f / (d.z != 0.f ? d.z : 1e-24f));
+    r.idir = f3(1.f / (d.x != 0.f ? d.x : 1e-24f), 1.f / (d.y != 0.f ? d.y : 1e-24f),
+                1.f / (d.z != 0.f ? d.z : 1e-24f));
     // Sz = 1 / d[kz]: that is idir[kz] unless d is the zero vector
-    const float iz = r.rz0 ? idir.x : (r.rz1 ? idir.y : idir.z);
+    const float iz = r.rz0 ? r.idir.x : (r.rz1 ? r.idir.y : r.idir.z);
     r.Sz = dz != 0.f ? iz : __builtin_copysignf(__builtin_inff(), dz);
     r.Sx = dp.x * r.Sz;                     // shear by the reciprocal: no division of its own
     r.Sy = dp.y * r.Sz;
-    r.nx = kNodePlanes[0] + (idir.x >= 0.f ? 0u : 8u);
-    r.ny = kNodePlanes[1] + (idir.y >= 0.f ? 0u : 8u);
-    r.nz = kNodePlanes[2] + (idir.z >= 0.f ? 0u : 8u);
-    const float f = REL ? 1.f / tray_T(tmax) : 1.f;
-    r.inv = REL ? f * idir : idir;
-    // (a little early, for the rounding of (origin - o) * inv where tmin / T cancels it)
-    r.stmin = REL ? f * (tmin - fabsf(tmin) * kSlabPad) : 0.f;
-}
-
-// the best hit moved from told to tnew (the ray's T with it)
-template <bool REL>
-__device__ __forceinline__ void tray_rescale(TRay& r, float told, float tnew) {
-    if (!REL) return;
-    const float f = (tray_T(told) * kHitBias) * __builtin_amdgcn_rcpf(tray_T(tnew));
-    r.inv = f * r.inv;
-    r.stmin = f * r.stmin;
+    r.nx = kNodePlanes[0] + (r.idir.x >= 0.f ? 0u : 8u);
+    r.ny = kNodePlanes[1] + (r.idir.y >= 0.f ? 0u : 8u);
+    r.nz = kNodePlanes[2] + (r.idir.z >= 0.f ? 0u : 8u);
 }
 
 // true with t > tmin and barycentrics (u,v) of v1 and v2 on a hit
@@ -281,12 +250,8 @@ __device__ __forceinline__ float comp4(const float4& v, int j) {
     return j == 0 ? v.x : (j == 1 ? v.y : (j == 2 ? v.z : v.w));
 }
 
-// the distance of a plane, half * ds + c (one v_fma_mix_f32), and the same
-// clamped to [0, 1]
+// the distance of a plane, half * ds + c (one v_fma_mix_f32)
 __device__ __forceinline__ float slab(_Float16 h, float ds, float c) { return __builtin_fmaf((float)h, ds, c); }
-__device__ __forceinline__ float slab01(_Float16 h, float ds, float c) {
-    return __builtin_amdgcn_fmed3f(slab(h, ds, c), 0.f, 1.f);
-}
 
 // A child of a node step as one double, the entry distance's bits above the
 // ref's: doubles order by their high word first, so one v_min_f64 and one
@@ -345,10 +310,9 @@ __device__ __forceinline__ void trav_reset(Trav& s, const DevScene& sc, lds_u32*
     s.inst = kNoHit;
 }
 
-template <bool TL>
 __device__ __forceinline__ void trav_begin(Trav& s, const DevScene& sc, lds_u32* bottom, float3 o, float3 d, float tmin,
                                            float tmax) {
-    tray_init<!TL>(s.r, o, d, tmin, tmax);
+    tray_init(s.r, o, d, tmin);
     trav_reset(s, sc, bottom, tmax);
 }
 
@@ -403,7 +367,7 @@ __device__ __forceinline__ void inst_step(const DevScene& sc, Trav& s, bool goin
         s.inst = id;
         s.node = __float_as_uint(m.x);
     }
-    if (leave || enter) tray_init<false>(s.r, o, d, s.r.tmin, s.h.t);
+    if (leave || enter) tray_init(s.r, o, d, s.r.tmin);
 }
 
 // first active lane of the wave (counts wave-level loop iterations in COUNT mode)
@@ -557,7 +521,6 @@ __device__ __forceinline__ void leaves_compact(const DevScene& sc, Trav& s, uint
             const uint32_t prim = (uint32_t)kk;
             const bool lower = TL ? (s.inst < s.h.inst || (s.inst == s.h.inst && prim < s.h.prim)) : prim < s.h.prim;
             if (t < s.h.t || (t == s.h.t && lower)) {
-                tray_rescale<!TL>(s.r, s.h.t, t);
                 s.h.t = t;
                 s.h.u = bu;
                 s.h.v = bv;
@@ -672,38 +635,19 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
                 // compiler would hold some back to reuse registers: the
                 // 1080p mixed-level frame 109 ms without, 102 ms with)
                 __builtin_amdgcn_sched_barrier(0);
-                const float3 ds = f3(sc.plane_scale * r.inv.x, sc.plane_scale * r.inv.y, sc.plane_scale * r.inv.z);
+                const float3 ds = f3(sc.plane_scale * r.idir.x, sc.plane_scale * r.idir.y, sc.plane_scale * r.idir.z);
                 const float3 oo = f3(og.x - r.o.x, og.y - r.o.y, og.z - r.o.z);
                 double key[4];
-                if (!TL) {
-                    const float3 c = f3(__builtin_fmaf(oo.x, r.inv.x, -r.stmin), __builtin_fmaf(oo.y, r.inv.y, -r.stmin),
-                                        __builtin_fmaf(oo.z, r.inv.z, -r.stmin));
-                    const float3 ce = f3(__builtin_fmaf(fabsf(c.x), -kSlabPad, c.x),
-                                         __builtin_fmaf(fabsf(c.y), -kSlabPad, c.y),
-                                         __builtin_fmaf(fabsf(c.z), -kSlabPad, c.z));
-                    const float3 cx = f3(__builtin_fmaf(fabsf(c.x), kSlabPad, c.x),
-                                         __builtin_fmaf(fabsf(c.y), kSlabPad, c.y),
-                                         __builtin_fmaf(fabsf(c.z), kSlabPad, c.z));
+                const float3 c = f3(oo.x * r.idir.x, oo.y * r.idir.y, oo.z * r.idir.z);
     #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float x0 = slab01(px[j], ds.x, ce.x), x1 = slab01(px[4 + j], ds.x, cx.x);
-                        const float y0 = slab01(py[j], ds.y, ce.y), y1 = slab01(py[4 + j], ds.y, cx.y);
-                        const float z0 = slab01(pz[j], ds.z, ce.z), z1 = slab01(pz[4 + j], ds.z, cx.z);
-                        const float tn = fmaxf(fmaxf(x0, y0), z0);
-                        const float tf = fminf(fminf(x1, y1), z1);
-                        key[j] = child_key(tn < tf ? tn : __builtin_inff(), __float_as_uint(comp4(rf, j)));
-                    }
-                } else {
-                    const float3 c = f3(oo.x * r.inv.x, oo.y * r.inv.y, oo.z * r.inv.z);
-    #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float x0 = slab(px[j], ds.x, c.x), x1 = slab(px[4 + j], ds.x, c.x);
-                        const float y0 = slab(py[j], ds.y, c.y), y1 = slab(py[4 + j], ds.y, c.y);
-                        const float z0 = slab(pz[j], ds.z, c.z), z1 = slab(pz[4 + j], ds.z, c.z);
-                        const float tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
-                        const float tf = fminf(fminf(x1, y1), fminf(z1, s.h.t));
-                        key[j] = child_key(tn <= tf * kBoxPad ? tn : __builtin_inff(), __float_as_uint(comp4(rf, j)));
-                    }
+                for (int j = 0; j < 4; j++) {
+                    const float x0 = slab(px[j], ds.x, c.x), x1 = slab(px[4 + j], ds.x, c.x);
+                    const float y0 = slab(py[j], ds.y, c.y), y1 = slab(py[4 + j], ds.y, c.y);
+                    const float z0 = slab(pz[j], ds.z, c.z), z1 = slab(pz[4 + j], ds.z, c.z);
+                    const float tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, r.tmin));
+                    const float tf = fminf(fminf(x1, y1), fminf(z1, s.h.t));
+                    const bool hit = tn <= __builtin_fmaf(fabsf(tf), kBoxPad, tf);   // (tf may be negative)
+                    key[j] = child_key(hit ? tn : __builtin_inff(), __float_as_uint(comp4(rf, j)));
                 }
                 // ascending by entry distance (misses last): 5 compare-exchanges
                 sort_ce(key[0], key[1]);
@@ -762,7 +706,6 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
                     const bool lower = TL ? (s.inst < s.h.inst || (s.inst == s.h.inst && prim < s.h.prim))
                                           : prim < s.h.prim;
                     if (tt < s.h.t || (tt == s.h.t && lower)) {
-                        tray_rescale<!TL>(s.r, s.h.t, tt);
                         s.h.t = tt;
                         s.h.u = uu;
                         s.h.v = vv;
