@@ -43,7 +43,7 @@ constexpr float kBoxPad = 0x1p-18f;
 
 struct TRay {
     float3 o, d;
-    float3 idir;    // 1 / d
+    float3 idir;    // 1 / d, limited (tray_init)
     float tmin;
     // the watertight test's axis order (kx, ky, kz) as a rotation that puts
     // the dominant axis kz last (rz0: kz = x, rz1: kz = y, else kz = z).
@@ -76,11 +76,16 @@ __device__ __forceinline__ void tray_init(TRay& r, float3 o, float3 d, float tmi
     r.rz0 = kz == 0;
     r.rz1 = kz == 1;
     const float3 dp = permute(r, d);       // (d[kx], d[ky], d[kz])
-    r.idir = f3(1.f / (d.x != 0.f ? d.x : 1e-24f), 1.f / (d.y != 0.f ? d.y : 1e-24f),
-                1.f / (d.z != 0.f ? d.z : 1e-24f));
-    // Sz = 1 / d[kz]: that is idir[kz] unless d is the zero vector
-    const float iz = r.rz0 ? r.idir.x : (r.rz1 ? r.idir.y : r.idir.z);
-    r.Sz = dz != 0.f ? iz : __builtin_copysignf(__builtin_inff(), dz);
+    const float3 q = f3(1.f / d.x, 1.f / d.y, 1.f / d.z);
+    r.Sz = r.rz0 ? q.x : (r.rz1 ? q.y : q.z);
+    // A component 2^72 times smaller than the largest is taken as that much
+    // smaller, so that a zero or subnormal one gives finite distances: boxes
+    // hold the ray's points to within 2^-42 of their size (node.h).  (Between
+    // 2^40 and 2^72 for short directions, so that distances along it stay in range.)
+    const float aS = fabsf(r.Sz);
+    const float lim = __builtin_amdgcn_fmed3f(aS * 0x1p40f, aS * 0x1p72f, 1e30f);
+    r.idir = f3(__builtin_amdgcn_fmed3f(q.x, -lim, lim), __builtin_amdgcn_fmed3f(q.y, -lim, lim),
+                __builtin_amdgcn_fmed3f(q.z, -lim, lim));
     r.Sx = dp.x * r.Sz;                     // shear by the reciprocal: no division of its own
     r.Sy = dp.y * r.Sz;
     r.nx = kNodePlanes[0] + (r.idir.x >= 0.f ? 0u : 8u);

@@ -1,7 +1,8 @@
 """Closest hits over the whole range of what a ray may hold: negative tmin
 (lines and segments that begin behind the origin), tmin just below the hit
-(stepping through hits) and unbounded tmax over tiny scenes.  Flat and
-two-level layouts."""
+(stepping through hits), unbounded tmax over tiny scenes, and direction
+components that are subnormal, zero of either sign or far below the others.
+Flat and two-level layouts."""
 import numpy as np
 import pytest
 
@@ -110,6 +111,39 @@ def test_tmin_just_below_the_hit(rtx, two_level):
                 assert np.array_equal(again[key], first[key]), key
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("two_level", [False, True])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("tiny", [-0., 1e-44, -1e-41, 1e-39, -3e-39, 1e-36, -1e-30, 1e-26, 1e-20])
+def test_tiny_direction_components(rtx, axis, tiny, two_level):
+    """Components whose reciprocal is infinite or huge: the ray is parallel to the axis."""
+    s = _build(rtx, _layers(6, axis, (-4., 4., 4.5)), two_level)
+    try:
+        rays = np.concatenate([_axis_rays(6, axis, 1), _axis_rays(6, axis, -1)])
+        for k in ((1,), (2,), (1, 2)):
+            for j in k:
+                rays[:, 4 + (axis + j) % 3] = tiny
+            say("axis %d, component %g" % (axis, tiny))
+            assert (s.trace(rays)["t"] == np.float32(4)).all()
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("two_level", [False, True])
+@pytest.mark.parametrize("log2", [-90, -70, -50, 40])
+def test_short_and_long_directions(rtx, log2, two_level):
+    """A direction of length 2^k along an axis: the distance is 4 / 2^k."""
+    for axis in (0, 1, 2):
+        s = _build(rtx, _layers(6, axis, (-4., 4., 4.5)), two_level)
+        try:
+            rays = np.concatenate([_axis_rays(6, axis, 1), _axis_rays(6, axis, -1)])
+            rays[:, 4:7] *= np.float32(2.0 ** log2)
+            rays[:, 3], rays[:, 7] = 0., INF
+            say("axis %d, direction 2^%d" % (axis, log2))
+            assert (s.trace(rays)["t"] == np.float32(4 * 2.0 ** -log2)).all()
+        finally:
+            s.close()
 
 
 @pytest.mark.parametrize("two_level", [False, True])
