@@ -35,7 +35,6 @@ struct BuiltBVH {
     uint32_t num_nodes = 0, num_leaves = 0, max_depth = 0, max_leaf = 0;   // of the binary SAH tree
     uint32_t num_wide = 0, wide_depth = 0;                                    // of the 4-wide tree
     float root_lo[3] = {0.f, 0.f, 0.f}, root_hi[3] = {0.f, 0.f, 0.f};      // bounds of all primitives
-    float plane_scale = 1.f;             // of the node planes
     std::vector<uint32_t> level_begin;   // first wide node of each level (+ the total at the end)
     double sah = 0.0;
 };
@@ -101,11 +100,8 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
 
 // ---- two-level scenes (tlas.hip) ----
 // adds node_base / tri_base to the refs of a bottom-level tree of n wide
-// nodes that was copied to nodes[node_base ...] and its triangles to tri_base,
-// and multiplies its planes' halves by plane_factor (a power of two: the
-// tree's own scale over the scene's)
-hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, float plane_factor,
-                         hipStream_t s);
+// nodes that was copied to nodes[node_base ...] and its triangles to tri_base
+hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, hipStream_t s);
 // turns the leaf refs of a top-level tree (n wide nodes at nodes[0], one
 // primitive per leaf, order = its leaf order over nprim primitives) into
 // instance refs kInstLeaf | inst_of[primitive]; empty slots get null_inst
@@ -113,8 +109,8 @@ hipError_t tlas_leaves(float4* nodes, uint32_t n, const uint32_t* order, uint32_
                        uint32_t null_inst, hipStream_t s);
 // refits the top-level boxes from ibox (world lo, hi float4 per instance),
 // deepest level first; null_ref = kInstLeaf | null instance; tbox: scratch of
-// 2 float4 per top-level node (the nodes' own boxes); plane_scale: the scene's
+// 2 float4 per top-level node (the nodes' own boxes)
 hipError_t refit_tlas(float4* nodes, const std::vector<uint32_t>& level_begin, const float4* ibox, float4* tbox,
-                      uint32_t null_ref, float plane_scale, hipStream_t s);
+                      uint32_t null_ref, hipStream_t s);
 
 }  // namespace rtx

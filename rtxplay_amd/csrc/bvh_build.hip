@@ -1229,7 +1229,6 @@ __global__ void k_write4(const Level* __restrict__ lev, const BNode* __restrict_
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= lev[0].n) return;
     const uint32_t base_this = lev[0].first, base_next = lev[1].first;
-    const float plane_scale = plane_scale_of(bn[0].lo, bn[0].hi);
     const uint4 c4 = cid[i];
     float lo[4][3], hi[4][3];
     bool used[4];
@@ -1261,7 +1260,7 @@ __global__ void k_write4(const Level* __restrict__ lev, const BNode* __restrict_
             j++;
         }
     }
-    encode_node(nodes4 + kWideNodeF4 * (size_t)(base_this + i), lo, hi, used, ref, plane_scale);
+    encode_node(nodes4 + kWideNodeF4 * (size_t)(base_this + i), lo, hi, used, ref);
 }
 
 __global__ void k_gather_tris(const float4* __restrict__ tri_world, const uint32_t* __restrict__ idx, uint32_t N,
@@ -1653,7 +1652,6 @@ hipError_t build_bvh(const float4* d_tri_world, const float4* d_plo, const float
     const uint32_t root_cnt = __builtin_bit_cast(uint32_t, root.hi.w);
     const float rx = root.hi.x - root.lo.x, ry = root.hi.y - root.lo.y, rz = root.hi.z - root.lo.z;
     const double root_area = 2.0 * ((double)rx * ry + (double)ry * rz + (double)rz * rx);
-    out.plane_scale = plane_scale_of(root.lo, root.hi);
     out.nodes = opt.owned ? nodes.release() : wide;
     out.tris = opt.owned ? tris.release() : tris_ws;
     if (!opt.gather) out.order = idx;

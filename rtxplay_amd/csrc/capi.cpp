@@ -586,7 +586,6 @@ static rtx_status build_scene_flat(rtx_ctx* c, hipStream_t s, Built** out) {
     b->hdr.root = bvh.root;
     b->hdr.num_prims = (uint32_t)N;
     b->hdr.num_nodes = bvh.num_wide;
-    b->hdr.plane_scale = bvh.plane_scale;
     b->hdr.num_insts = ninst;
     if ((e = hipMalloc((void**)&b->d_hdr, sizeof(rtx::DevScene))) != hipSuccess) return bail(hip_fail(e, "hipMalloc(handle)"));
     if ((e = hipMemcpyAsync(b->d_hdr, &b->hdr, sizeof(rtx::DevScene), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload handle"));
@@ -870,17 +869,13 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
         if ((e = hipMemcpyAsync(b->nodes, tb.nodes, sizeof(float4) * rtx::kWideNodeF4 * tb.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy top level"));
         if ((e = rtx::tlas_leaves(b->nodes, tb.num_wide, tb.order, M, d_inst_of, ninst, s)) != hipSuccess) return bail(hip_fail(e, "top-level leaves"));
     }
-    // one scale for the planes of every tree
-    float plane_scale = M ? tb.plane_scale : 1.f;
-    for (size_t m = 0; m < nm; m++)
-        if (used[m]) plane_scale = std::max(plane_scale, bl[m].plane_scale);
     for (size_t m = 0; m < nm; m++) {
         if (!used[m]) continue;
         const rtx::BuiltBVH& x = bl[m];
         const uint32_t nb = (uint32_t)(tb.num_wide + node_off[m]), tbm = (uint32_t)tri_base[m];
         if (x.num_wide) {
             if ((e = hipMemcpyAsync(b->nodes + (size_t)rtx::kWideNodeF4 * nb, x.nodes, sizeof(float4) * rtx::kWideNodeF4 * x.num_wide, hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy bottom level"));
-            if ((e = rtx::relocate_blas(b->nodes, x.num_wide, nb, tbm, x.plane_scale / plane_scale, s)) != hipSuccess) return bail(hip_fail(e, "relocate"));
+            if ((e = rtx::relocate_blas(b->nodes, x.num_wide, nb, tbm, s)) != hipSuccess) return bail(hip_fail(e, "relocate"));
         }
         if ((e = hipMemcpyAsync(b->tris + 3 * (size_t)tbm, x.tris, sizeof(float4) * 3 * ((size_t)c->meshes[m].ni + 1), hipMemcpyDeviceToDevice, s)) != hipSuccess) return bail(hip_fail(e, "copy triangles"));
         b->blas_root[m] = (x.root & rtx::kLeafFlag) ? x.root + tbm : x.root + nb;
@@ -895,9 +890,8 @@ static rtx_status build_scene_tl(rtx_ctx* c, hipStream_t s, Built** out) {
     if ((e = hipMemcpyAsync(b->ibox, wbox.data(), sizeof(float4) * wbox.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload instance boxes"));
     if ((e = hipMemcpyAsync(b->insts, irec.data(), sizeof(float4) * irec.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return bail(hip_fail(e, "upload inst records"));
     b->tlas_levels = tb.level_begin;
-    b->hdr.plane_scale = plane_scale;
     if (tb.num_wide) {
-        if ((e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, b->hdr.plane_scale, s)) != hipSuccess) return bail(hip_fail(e, "refit"));
+        if ((e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, s)) != hipSuccess) return bail(hip_fail(e, "refit"));
     }
 
     uint32_t root = rtx::kEmptyRoot;
@@ -968,7 +962,7 @@ static rtx_status refit_scene_tl(rtx_ctx* c, Built* b, hipStream_t s) {
     if (e == hipSuccess) e = hipMemcpyAsync(b->xinst, xrec.data(), sizeof(float4) * xrec.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(b->ibox, wbox.data(), sizeof(float4) * wbox.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(b->insts, irec.data(), sizeof(float4) * irec.size(), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && b->tlas_levels.size() > 1) e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, b->hdr.plane_scale, s);
+    if (e == hipSuccess && b->tlas_levels.size() > 1) e = rtx::refit_tlas(b->nodes, b->tlas_levels, b->ibox, b->tbox, rtx::kInstLeaf | ninst, s);
     if (e == hipSuccess) e = hipEventRecord(e1, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     float ms = 0.f;

@@ -14,7 +14,7 @@
 // Rounding is outwards: a plane at p is stored at or beyond p moved out by
 // 2^-20 of its distance from the origin, in exact arithmetic.  That margin
 // covers the rounding of the traversal's (origin - o) * idir where it cancels
-// against half * (plane_scale * idir) (up to 2^-22 of that distance); the
+// against half * (scale * idir) (up to 2^-22 of that distance); the
 // error relative to the distance itself is covered by kBoxPad in
 // traverse.h.  The origin lies a little below the smallest child's lo plane,
 // so that no plane of a box is at distance 0 of it and a ray that runs within
@@ -34,24 +34,23 @@ __device__ inline uint32_t half_down(double v) {
 }
 __device__ inline uint32_t half_up(double v) { return half_down(-v) ^ 0x8000u; }
 
-// the scale of a tree whose bounds are `extent` wide at most: extents fill
-// 2^11 of the halves' 2^16 range, so that a refit may move things 2^5 times as
-// far apart before planes become infinite (still correct, only looser)
-__host__ __device__ inline float plane_scale_for(float extent) {
+// The scale of a node whose planes are `reach` from its origin at most: they
+// fill 2^15 of the halves' 2^16 range.  (Each node has its own, beside its
+// origin: with one scale for a scene a refit that moved things 32 times as far
+// apart had infinite planes, and geometry below 2^-35 of the extent had one
+// plane step for a whole subtree.)
+__device__ inline float node_scale(double reach) {
     int e = 0;
-    (void)frexpf(extent > 1e-30f && extent < 1e30f ? extent : 1.f, &e);
-    return ldexpf(1.f, e - 11);
-}
-__host__ __device__ inline float plane_scale_of(const float4& lo, const float4& hi) {
-    return plane_scale_for(fmaxf(fmaxf(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z));
+    (void)frexp(reach, &e);
+    return ldexpf(1.f, max(e - 15, -126));
 }
 
 // lo, hi: the children's boxes; used: which slots hold one
 __device__ inline void encode_node(float4* o, const float (&lo)[4][3], const float (&hi)[4][3], const bool (&used)[4],
-                                   const uint32_t (&ref)[4], float plane_scale) {
+                                   const uint32_t (&ref)[4]) {
     float org[3] = {0.f, 0.f, 0.f};
     uint2* w = (uint2*)o;
-    const double inv = 1.0 / (double)plane_scale;
+    double reach = 0.0;
     for (int a = 0; a < 3; a++) {
         float least = __builtin_inff();
         float mn = __builtin_inff(), mx = -__builtin_inff();
@@ -66,6 +65,17 @@ __device__ inline void encode_node(float4* o, const float (&lo)[4][3], const flo
             }
         }
         if (mx >= mn && mx - mn < 1e37f) org[a] -= fabsf(org[a]) * 0x1p-21f + (mx - mn) * 0x1p-22f + 1e-36f;
+        for (int k = 0; k < 4; k++) {
+            if (!used[k]) continue;
+            // (infinite planes are infinite halves at any scale)
+            const double l = fabs((double)lo[k][a] - (double)org[a]), h = fabs((double)hi[k][a] - (double)org[a]);
+            if (l < 1e39) reach = fmax(reach, l);
+            if (h < 1e39) reach = fmax(reach, h);
+        }
+    }
+    const float scale = node_scale(reach);
+    const double inv = 1.0 / (double)scale;
+    for (int a = 0; a < 3; a++) {
         const double O = (double)org[a];
         uint32_t bl[4], bh[4];
         for (int k = 0; k < 4; k++) {
@@ -79,24 +89,9 @@ __device__ inline void encode_node(float4* o, const float (&lo)[4][3], const flo
         p[1] = make_uint2(bh[0] | (bh[1] << 16), bh[2] | (bh[3] << 16));
         p[2] = L;
     }
-    o[kNodeOrigin] = make_float4(org[0], org[1], org[2], 0.f);
+    o[kNodeOrigin] = make_float4(org[0], org[1], org[2], scale);
     o[kNodeRefs] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
                                __uint_as_float(ref[3]));
-}
-
-// the planes of a node at another scale: half * factor (a power of two),
-// rounded outwards again where the range ends
-__device__ inline void rescale_node(float4* o, float factor) {
-    uint16_t* b = (uint16_t*)o;
-    for (int a = 0; a < 3; a++) {
-        uint16_t* p = b + kNodePlanes[a] / 2u;
-        for (int k = 0; k < 4; k++) {
-            const double l = (double)__builtin_bit_cast(_Float16, p[k]) * factor;
-            const double h = (double)__builtin_bit_cast(_Float16, p[4 + k]) * factor;
-            p[k] = p[8 + k] = (uint16_t)half_down(l);
-            p[4 + k] = (uint16_t)half_up(h);
-        }
-    }
 }
 
 }  // namespace rtx

@@ -4,10 +4,10 @@
 //   nodes : 4-wide BVH nodes, 128 B each, 112 B used:
 //             0  x planes: lo[4], hi[4], lo[4] as halves (24 B)
 //            24  y planes, the same
-//            48  origin.xyz, 0 (float4)
+//            48  origin.xyz, scale (float4)
 //            64  z planes, the same as x
 //            96  refs[4] (float4 of uint bits)
-//           a plane is at origin + plane_scale * half, rounded outwards
+//           a plane is at origin + scale * half, rounded outwards
 //           (encode_node in node.h); a ray that enters a box through its lo
 //           plane reads an axis from its first lo on, else from hi on, and
 //           gets the entry planes followed by the exit planes either way
@@ -52,7 +52,7 @@ constexpr uint32_t kNoHit = 0xFFFFFFFFu;
 constexpr uint32_t kEmptyRoot = 0xFFFFFFFFu;
 constexpr uint32_t kNoChild = 0x7FFFFFFFu;  // empty slot of a 4-wide node (no leaf flag, no valid node)
 constexpr int kWideNodeF4 = 8;             // float4 per 4-wide node (128 B)
-constexpr int kNodeOrigin = 3;             // the float4 of a node that holds its origin
+constexpr int kNodeOrigin = 3;             // the float4 of a node that holds its origin and scale
 constexpr int kNodeRefs = 6;               // the float4 of a node that holds the refs
 constexpr uint32_t kNodePlanes[3] = {0u, 24u, 64u};   // byte offset of each axis's planes
 constexpr uint32_t kInstLeaf = 0xF8000000u; // top-level leaf of one instance: kInstLeaf | instance id
@@ -102,8 +102,6 @@ struct DevScene {
     uint32_t num_prims;
     uint32_t num_nodes;   // 4-wide nodes in the node array
     uint32_t num_insts;
-    float plane_scale;    // world units of a node plane's half (a power of two)
-    uint32_t pad;         // 0 (headers are compared as bytes)
 };
 
 __host__ __device__ inline uint32_t leaf_ref(uint32_t first, uint32_t count) {

@@ -26,14 +26,11 @@ __device__ __forceinline__ void set_comp(float4& v, int j, float x) {
     if (j == 0) v.x = x; else if (j == 1) v.y = x; else if (j == 2) v.z = x; else v.w = x;
 }
 
-// bottom-level tree copied to node index node_base / triangle index tri_base,
-// its planes at the scene's scale
-__global__ void k_relocate(float4* __restrict__ nodes, uint32_t n, uint32_t node_base, uint32_t tri_base,
-                           float plane_factor) {
+// bottom-level tree copied to node index node_base / triangle index tri_base
+__global__ void k_relocate(float4* __restrict__ nodes, uint32_t n, uint32_t node_base, uint32_t tri_base) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4* o = nodes + (size_t)kWideNodeF4 * (node_base + i);
-    if (plane_factor != 1.f) rescale_node(o, plane_factor);
     float4 rf = o[kNodeRefs];
     for (int j = 0; j < 4; j++) {
         uint32_t r = __float_as_uint(comp(rf, j));
@@ -67,7 +64,7 @@ __global__ void k_tlas_leaves(float4* __restrict__ nodes, uint32_t n, const uint
 // per top-level node, written here one level deeper before); slots of the null
 // instance stay empty
 __global__ void k_refit4(float4* __restrict__ nodes, uint32_t begin, uint32_t n, const float4* __restrict__ ibox,
-                         float4* __restrict__ tbox, uint32_t null_ref, float plane_scale) {
+                         float4* __restrict__ tbox, uint32_t null_ref) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4* o = nodes + (size_t)kWideNodeF4 * (begin + i);
@@ -90,7 +87,7 @@ __global__ void k_refit4(float4* __restrict__ nodes, uint32_t begin, uint32_t n,
             bh[k] = fmaxf(bh[k], hi[j][k]);
         }
     }
-    encode_node(o, lo, hi, used, ref, plane_scale);
+    encode_node(o, lo, hi, used, ref);
     tbox[2 * (size_t)(begin + i)] = make_float4(bl[0], bl[1], bl[2], 0.f);
     tbox[2 * (size_t)(begin + i) + 1] = make_float4(bh[0], bh[1], bh[2], 0.f);
 }
@@ -99,11 +96,9 @@ inline uint32_t blocks256(uint32_t n) { return (n + 255u) / 256u; }
 
 }  // namespace
 
-hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, float plane_factor,
-                         hipStream_t s) {
+hipError_t relocate_blas(float4* nodes, uint32_t n, uint32_t node_base, uint32_t tri_base, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_relocate, dim3(blocks256(n)), dim3(256), 0, s, nodes, n, node_base, tri_base,
-                       plane_factor);
+    hipLaunchKernelGGL(k_relocate, dim3(blocks256(n)), dim3(256), 0, s, nodes, n, node_base, tri_base);
     return hipGetLastError();
 }
 
@@ -116,13 +111,12 @@ hipError_t tlas_leaves(float4* nodes, uint32_t n, const uint32_t* order, uint32_
 }
 
 hipError_t refit_tlas(float4* nodes, const std::vector<uint32_t>& level_begin, const float4* ibox, float4* tbox,
-                      uint32_t null_ref, float plane_scale, hipStream_t s) {
+                      uint32_t null_ref, hipStream_t s) {
     // level_begin: first node of each level, then the node count
     for (size_t l = level_begin.size(); l-- > 1;) {
         const uint32_t b = level_begin[l - 1], n = level_begin[l] - b;
         if (n == 0) continue;
-        hipLaunchKernelGGL(k_refit4, dim3(blocks256(n)), dim3(256), 0, s, nodes, b, n, ibox, tbox, null_ref,
-                           plane_scale);
+        hipLaunchKernelGGL(k_refit4, dim3(blocks256(n)), dim3(256), 0, s, nodes, b, n, ibox, tbox, null_ref);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

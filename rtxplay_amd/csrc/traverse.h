@@ -640,7 +640,7 @@ __device__ __forceinline__ void trav_run(const DevScene& sc, Trav& s, bool& goin
                 // compiler would hold some back to reuse registers: the
                 // 1080p mixed-level frame 109 ms without, 102 ms with)
                 __builtin_amdgcn_sched_barrier(0);
-                const float3 ds = f3(sc.plane_scale * r.idir.x, sc.plane_scale * r.idir.y, sc.plane_scale * r.idir.z);
+                const float3 ds = f3(og.w * r.idir.x, og.w * r.idir.y, og.w * r.idir.z);
                 const float3 oo = f3(og.x - r.o.x, og.y - r.o.y, og.z - r.o.z);
                 double key[4];
                 const float3 c = f3(oo.x * r.idir.x, oo.y * r.idir.y, oo.z * r.idir.z);
