@@ -200,8 +200,11 @@ rtx_status rtx_scene_triangles(rtx_ctx* ctx, uint64_t is_handle, float* tris, ui
 /* Launch tuning of a context (no reference counterpart).  shade_batch: in
  * the render kernel a wave traverses until at least this many of its lanes
  * hold a final closest hit, shades those and resumes the others (1..64; 64 =
- * every lane of the wave finishes first; default 40, which leaves the choice
- * to the launch: 40 to 58 by the frame's size and samples).  inner_frac: a
+ * every lane of the wave finishes first; default 40).  shade_auto: 1 (the
+ * default) leaves that choice to the launch while shade_batch is 40: 40 to 58
+ * by the frame's size and samples; rtx_tuning_set with shade_auto 0 and a
+ * shade_batch, or with any other shade_batch, fixes it, and shade_auto 1 with
+ * shade_batch 40 or 0 gives the choice back.  inner_frac: a
  * traversal round's node phase ends when fewer than inner_frac/64 of the
  * traversing lanes can still step through inner nodes (each lane parks up
  * to two leaves and goes on); the parked leaves are then tested (1..64; 1 = every lane
@@ -220,7 +223,8 @@ typedef struct {
     uint32_t stack_lds;
     uint32_t blocks_per_cu;
     uint32_t max_blocks_per_cu;
-    uint32_t reserved[2];
+    uint32_t shade_auto;
+    uint32_t reserved;
 } rtx_tuning;
 rtx_status rtx_tuning_get(rtx_ctx* ctx, rtx_tuning* t);
 rtx_status rtx_tuning_set(rtx_ctx* ctx, const rtx_tuning* t);

@@ -94,7 +94,8 @@ class SceneStatsC(Structure):
 
 class TuningC(Structure):
     _fields_ = [("shade_batch", c_uint32), ("inner_frac", c_uint32), ("tile_w", c_uint32), ("stack_lds", c_uint32),
-                ("blocks_per_cu", c_uint32), ("max_blocks_per_cu", c_uint32), ("reserved", c_uint32 * 2)]
+                ("blocks_per_cu", c_uint32), ("max_blocks_per_cu", c_uint32), ("shade_auto", c_uint32),
+                ("reserved", c_uint32)]
 
 
 # every exported symbol: name -> (restype, argtypes)

@@ -327,15 +327,18 @@ class Scene:
         return tris, inst
 
     def tuning(self, **kw):
-        """Reads (and with keyword arguments sets) the launch tuning, e.g. shade_batch=40."""
+        """Reads (and with keyword arguments sets) the launch tuning, e.g.
+        shade_batch=40.  Setting shade_batch turns shade_auto off, unless that is set too."""
         t = TuningC()
         call("rtx_tuning_get", self.ctx, byref(t))
         if kw:
+            if "shade_batch" in kw:
+                t.shade_auto = 0
             for k, v in kw.items():
                 setattr(t, k, int(v))
             call("rtx_tuning_set", self.ctx, byref(t))
         return {k: getattr(t, k) for k in ("shade_batch", "inner_frac", "tile_w", "stack_lds", "blocks_per_cu",
-                                           "max_blocks_per_cu")}
+                                           "max_blocks_per_cu", "shade_auto")}
 
     def set_materials(self, params, handle=None, stream=None):
         """Material parameters float32[n,4] (albedo rgb, fuzz per thing) into the

@@ -464,6 +464,7 @@ rtx_status rtx_tuning_get(rtx_ctx* c, rtx_tuning* t) {
     t->stack_lds = c->render_ls.stack_lds;
     t->blocks_per_cu = c->render_ls.grid / (uint32_t)c->num_cus;
     t->max_blocks_per_cu = c->render_ls.grid_max / (uint32_t)c->num_cus;
+    t->shade_auto = c->render_ls.shade_auto;
     return RTX_SUCCESS;
 }
 
@@ -481,7 +482,12 @@ rtx_status rtx_tuning_set(rtx_ctx* c, const rtx_tuning* t) {
     if (t->tile_w) c->render_ls.tile_w = t->tile_w;
     if (t->stack_lds) c->render_ls.stack_lds = t->stack_lds;
     if (t->blocks_per_cu) c->render_ls.grid = t->blocks_per_cu * (uint32_t)c->num_cus;
-    if (t->shade_batch) c->render_ls.shade_batch = t->shade_batch;
+    // (a structure from rtx_tuning_get with another shade_batch written into it fixes that one)
+    const bool lib = t->shade_auto && (t->shade_batch == 0 || t->shade_batch == rtx::kShadeBatch);
+    if (lib || t->shade_batch) {
+        c->render_ls.shade_batch = lib ? rtx::kShadeBatch : t->shade_batch;
+        c->render_ls.shade_auto = lib ? 1u : 0u;
+    }
     if (t->inner_frac) c->render_ls.inner_frac = t->inner_frac;
     return RTX_SUCCESS;
 }
@@ -1193,8 +1199,8 @@ struct rtx_batch {
 
 static bool same_scratch(const rtx::LaunchScratch& a, const rtx::LaunchScratch& b) {
     return a.counter == b.counter && a.gstack == b.gstack && a.gstride == b.gstride && a.grid == b.grid &&
-           a.shade_batch == b.shade_batch && a.inner_frac == b.inner_frac && a.stack_lds == b.stack_lds &&
-           a.iterative == b.iterative;
+           a.shade_batch == b.shade_batch && a.shade_auto == b.shade_auto && a.inner_frac == b.inner_frac &&
+           a.stack_lds == b.stack_lds && a.iterative == b.iterative;
 }
 
 extern "C" {

@@ -12,7 +12,7 @@ namespace rtx {
 constexpr int kRenderBlock = 256;
 constexpr int kTraceBlock = 256;
 
-constexpr uint32_t kShadeBatch = 40;   // default shading batch (left at it, whole frames and batches take a larger one)
+constexpr uint32_t kShadeBatch = 40;   // default shading batch
 
 // per-context scratch for the persistent kernels
 struct LaunchScratch {
@@ -21,6 +21,7 @@ struct LaunchScratch {
     uint32_t gstride = 0;          // lanes covered by gstack (grid * block)
     uint32_t grid = 0;             // persistent grid size in blocks
     uint32_t shade_batch = kShadeBatch;   // render: finished lanes that trigger a wave's shading step
+    uint32_t shade_auto = 1;       // 1: nobody chose shade_batch, and whole frames and batches take a larger one
     uint32_t inner_frac = 36;      // traversal: node phase ends below inner_frac/64 of the going lanes
     uint32_t tile_w = 8;           // render: work tile of tile_w x (64 / tile_w) pixels
     uint32_t stack_lds = kStackLDS;   // render: traversal stack entries per lane in LDS (16 or 32)

@@ -803,7 +803,7 @@ hipError_t launch_frame(const RenderArgs& a, const LaunchScratch& ls, hipStream_
 }
 
 // Finished lanes that trigger a wave's shading step where the caller left the
-// default: a wave that shades together starts its next rays together.  While
+// choice (shade_auto): a wave that shades together starts its next rays together.  While
 // the lanes' paths are of one length (few samples per pixel: neighbouring
 // pixels at the same bounce) their rays then stay coherent, which is worth
 // the wait; with many samples the lanes drift apart and waiting only idles
@@ -812,16 +812,17 @@ hipError_t launch_frame(const RenderArgs& a, const LaunchScratch& ls, hipStream_
 // samples 1.02 to 1.08x at 50, but 0.98 to 1.15x at 58; 60 samples 1.00x at
 // 50 and 0.94x at 60 (two-level, 20 samples: 1.00x at 44, 0.98x at 56).
 // Batches, whose lanes hold pixels of several frames: 1.03 to 1.15x / 1.01 to
-// 1.05x.  Spread frames and the adjoint (few lanes, long serial paths) gain
-// nothing from more than 40.
+// 1.05x.  Ordered adjoints: flat 1.02 to 1.06x at 50 (0.97 to 1.05x at 58),
+// two-level 0.98 to 1.01x at 44.  Spread frames and adjoints (few lanes, long
+// serial paths) gain nothing from more than 40.
 constexpr uint32_t kFewSpp = 8;
 uint32_t frame_batch(const LaunchScratch& ls, const Job& j, uint32_t spp) {
-    if (ls.shade_batch != kShadeBatch) return ls.shade_batch;
+    if (!ls.shade_auto) return ls.shade_batch;
     if (j.sc.xinst) return spp <= kFewSpp ? 52u : 44u;
     return spp <= kFewSpp ? 58u : 50u;
 }
 uint32_t mixed_batch(const LaunchScratch& ls, const Job& first) {
-    if (ls.shade_batch != kShadeBatch) return ls.shade_batch;
+    if (!ls.shade_auto) return ls.shade_batch;
     return first.sc.xinst ? 48u : 54u;
 }
 
