@@ -182,10 +182,11 @@ static rtx_status alloc_scratch(rtx::LaunchScratch& ls, uint32_t blocks_per_cu, 
 
 // the traversal stack overflow area (tens of MB) is allocated by the first
 // launch that needs it, so contexts that only hold a scene for a batch cost
-// nothing beyond the scene; it grows when a scene needs a deeper stack
-static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need) {
-    const uint32_t over = need > (uint32_t)rtx::kMinStackLDS ? need - (uint32_t)rtx::kMinStackLDS : 1u;
-    if (ls.gstack && ls.gstack_entries >= over) return RTX_SUCCESS;
+// nothing beyond the scene; it grows when a scene needs a deeper stack.  lds:
+// the entries that every kernel using it holds in LDS
+static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need, uint32_t lds = rtx::kMinStackLDS) {
+    const uint32_t over = need > lds ? need - lds : 0u;
+    if (ls.gstack_entries >= over) return RTX_SUCCESS;
     if (ls.gstack) {
         HIP_OK(hipDeviceSynchronize());
         HIP_OK(hipFree(ls.gstack));
@@ -1101,7 +1102,6 @@ rtx_status rtx_launch(rtx_ctx* c, const rtx_lp_general* lp, int once, void* stre
     if ((uint64_t)lp->image_w * lp->image_h > 0xFFFFFFFFull / 2)
         return fail(RTX_ERROR_LIMIT, "rtx_launch: image too large");
     HIP_OK(hipSetDevice(c->device));
-    if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
     const float3 amb = make_float3(c->ambient.x, c->ambient.y, c->ambient.z);
     hipError_t e;
     if (once || lp->picker) {
@@ -1113,6 +1113,7 @@ rtx_status rtx_launch(rtx_ctx* c, const rtx_lp_general* lp, int once, void* stre
         if (lp->spp == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: spp == 0");
         if (lp->depth == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: depth == 0");
         if (!lp->rawRGB) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: rawRGB is NULL");
+        if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
         if (rtx::frame_ordered(*lp, c->render_ls))
             if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w))) return st;
         e = rtx::launch_render(b->hdr, *lp, amb, c->render_ls, (hipStream_t)stream);
@@ -1432,7 +1433,7 @@ rtx_status rtx_trace(rtx_ctx* c, uint64_t is_handle, const rtx_ray* rays, uint32
     if (!b) return fail(RTX_ERROR_INVALID_HANDLE, "rtx_trace: unknown handle");
     if (n && (!rays || !hits)) return fail(RTX_ERROR_INVALID_VALUE, "rtx_trace: NULL buffer");
     HIP_OK(hipSetDevice(c->device));
-    if (rtx_status st = ensure_gstack(c->trace_ls, b->stack_need)) return st;
+    if (rtx_status st = ensure_gstack(c->trace_ls, b->stack_need, rtx::kStackLDS)) return st;
     hipError_t e = rtx::launch_trace(b->hdr, rays, n, hits, c->trace_ls, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "rtx_trace");
     return RTX_SUCCESS;

@@ -745,12 +745,15 @@ __global__ void k_get_materials(const float4* __restrict__ insts, uint32_t n, fl
 
 // picker: one primary ray through (pick_x, pick_y), optx/camera_r.cu:26-32 and
 // optx/optics_r.cu:24-28 / optx/camera_r.cu:125-129
+// (one lane: its whole stack is in LDS, so a pick takes no device memory)
+constexpr int kPickStack = 511;
+static_assert(kPickStack >= 2 * 3 * kMaxTreeDepth + 7, "the deepest two-level scene's stack");
 template <bool TL>
 __global__ __launch_bounds__(64) void k_pick(const RenderArgs a) {
-    __shared__ uint32_t s_stack[(kStackLDS + 1) * 64];
+    __shared__ uint32_t s_stack[kPickStack + 1];
     if (threadIdx.x != 0) return;
-    LaneStack<64> stk;
-    stk.init(s_stack, a.gstack, a.gstride);
+    LaneStack<1, kPickStack> stk;
+    stk.init(s_stack, nullptr, 0);
     const rtx_lp_general& lp = a.job.lp;
     const uint32_t W = lp.image_w, H = lp.image_h;
     const uint32_t x = lp.pick_x, y = lp.pick_y;
@@ -765,7 +768,7 @@ __global__ __launch_bounds__(64) void k_pick(const RenderArgs a) {
     TRay r;
     tray_init(r, o, d, 1e-3f);
     HitFull h;
-    traverse<64, TL>(a.job.sc, r, 1e16f, h, stk);
+    traverse<1, TL>(a.job.sc, r, 1e16f, h, stk);
     *lp.pick_id = h.tri == kNoHit ? 0xFFFFFFFFu
                                   : (TL ? h.inst : __float_as_uint(a.job.sc.tris[3 * (size_t)h.tri + 1].w));
 }
