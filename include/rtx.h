@@ -260,7 +260,8 @@ rtx_status rtx_get_semantics(rtx_ctx* ctx, int* mode);
  * one-sample probe and renders its 64-pixel tiles in descending order of the
  * probe's cost, the most expensive pixels in waves of fewer lanes (the pixels
  * depend on neither); the first such launch of a context allocates the order's
- * arrays (136 bytes per tile). */
+ * arrays (136 bytes per tile), and one that cannot, under stream capture or for
+ * want of memory, renders in slot order. */
 rtx_status rtx_launch(rtx_ctx* ctx, const rtx_lp_general* lp, int once, void* stream);
 
 /* rtx_launch without device allocation.  No counterpart in the reference: it

@@ -199,9 +199,16 @@ static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need, uint32_t 
 }
 
 // the probe cost and tile order arrays of ordered frames (136 bytes per tile),
-// allocated by the first launch that needs them and grown with the frame
-static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles) {
+// allocated by the first launch that needs them and grown with the frame.
+// Where they cannot be (the stream is being captured, no memory is left) the
+// frame is rendered in slot order: the order is no launch's due.
+static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles, hipStream_t s) {
     if (ls.tile_cost && ls.tile_cap >= ntiles) return RTX_SUCCESS;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return RTX_SUCCESS;
+    }
     if (ls.tile_cost) {
         HIP_OK(hipDeviceSynchronize());
         HIP_OK(hipFree(ls.tile_cost));
@@ -211,14 +218,15 @@ static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles) {
         ls.pix_cost = nullptr;
         ls.tile_cap = 0;
     }
-    HIP_OK(hipMalloc((void**)&ls.tile_cost, sizeof(uint32_t) * (size_t)ntiles));
-    hipError_t e = hipMalloc((void**)&ls.tile_order, sizeof(uint32_t) * (size_t)ntiles);
+    hipError_t e = hipMalloc((void**)&ls.tile_cost, sizeof(uint32_t) * (size_t)ntiles);
+    if (e == hipSuccess) e = hipMalloc((void**)&ls.tile_order, sizeof(uint32_t) * (size_t)ntiles);
     if (e == hipSuccess) e = hipMalloc((void**)&ls.pix_cost, sizeof(uint16_t) * 64u * (size_t)ntiles);
     if (e != hipSuccess) {
-        (void)hipFree(ls.tile_cost);
+        if (ls.tile_cost) (void)hipFree(ls.tile_cost);
         if (ls.tile_order) (void)hipFree(ls.tile_order);
         ls.tile_cost = ls.tile_order = nullptr;
-        return hip_fail(e, "hipMalloc(tile_order)");
+        (void)hipGetLastError();
+        return e == hipErrorOutOfMemory ? RTX_SUCCESS : hip_fail(e, "hipMalloc(tile_order)");
     }
     ls.tile_cap = ntiles;
     return RTX_SUCCESS;
@@ -1115,7 +1123,7 @@ rtx_status rtx_launch(rtx_ctx* c, const rtx_lp_general* lp, int once, void* stre
         if (!lp->rawRGB) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: rawRGB is NULL");
         if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
         if (rtx::frame_ordered(*lp, c->render_ls))
-            if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w))) return st;
+            if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
         e = rtx::launch_render(b->hdr, *lp, amb, c->render_ls, (hipStream_t)stream);
     }
     if (e != hipSuccess) return hip_fail(e, "rtx_launch");
@@ -1400,7 +1408,7 @@ rtx_status rtx_launch_adjoint(rtx_ctx* c, const rtx_lp_general* lp, const rtx_fl
         c->tape_depth = lp->depth;
     }
     if (rtx::frame_ordered(*lp, c->render_ls, true))
-        if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w))) return st;
+        if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
     const float3 amb = make_float3(c->ambient.x, c->ambient.y, c->ambient.z);
     hipError_t e = rtx::launch_adjoint(b->hdr, *lp, amb, c->render_ls, dL_drgb, d_params, c->tape,
                                        c->render_ls.gstride, (hipStream_t)stream);
