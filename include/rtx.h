@@ -98,6 +98,10 @@ typedef struct rtx_ctx rtx_ctx;
  * owns what Scene owns in the reference (optx/scene.h:37-62). */
 rtx_status rtx_ctx_create(int device, rtx_ctx** ctx);
 rtx_status rtx_ctx_destroy(rtx_ctx* ctx);
+/* Gives back the device memory that scene builds keep for the next one on the
+ * context's device (up to 4 GiB, given back with its last context otherwise).
+ * No reference counterpart; does nothing while another thread builds. */
+rtx_status rtx_ctx_trim(rtx_ctx* ctx);
 
 /* ---- camera ------------------------------------------------------------- */
 /* Camera::set, optx/camera.h:30-48 (host side, FP32) */

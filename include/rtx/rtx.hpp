@@ -174,6 +174,8 @@ class Scene {
     }
     rtx_ctx* context() { return ctx_; }
 
+    // gives back the device memory that builds keep (no reference counterpart)
+    void trim() { check(rtx_ctx_trim(ctx_), "rtx_ctx_trim"); }
     // launch tuning (no reference counterpart); fields left 0 keep their value
     rtx_tuning tuning() {
         rtx_tuning t{};

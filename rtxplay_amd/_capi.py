@@ -103,6 +103,7 @@ SIGNATURES = {
     "rtx_last_error": (c_char_p, []),
     "rtx_ctx_create": (c_int, [c_int, POINTER(c_void_p)]),
     "rtx_ctx_destroy": (c_int, [c_void_p]),
+    "rtx_ctx_trim": (c_int, [c_void_p]),
     "rtx_camera_set": (c_int, [POINTER(CameraC), Float3, Float3, Float3, c_float, c_float, c_float, c_float]),
     "rtx_sphere_mesh": (c_int, [c_float, c_uint32, c_void_p, c_uint32, POINTER(c_uint32), c_void_p, c_uint32,
                                 POINTER(c_uint32)]),

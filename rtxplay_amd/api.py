@@ -225,6 +225,10 @@ class Scene:
             call("rtx_ctx_destroy", self.ctx)
             self.ctx = c_void_p()
 
+    def trim(self):
+        """Gives back the device memory that scene builds keep for the next one."""
+        call("rtx_ctx_trim", self.ctx)
+
     def __del__(self):
         try:
             self.close()

@@ -51,12 +51,16 @@ struct BvhOptions {
 // Allocating and freeing the temporaries took 7.5 ms of the 28 ms of the
 // 8M-triangle level-6 scene and 9 of 18 ms of the mixed two-level one (now,
 // with the levels launched ahead, 21.5 and 8.0 ms, host to host).  The
-// block is kept between builds up to kKeepBytes and freed with the device's
-// last context (build_workspace_drop).  A build ends with its stream
+// block is kept between builds up to kKeepBytes; it shrinks once kShrinkAfter
+// builds in a row took less than an eighth of it, and is freed with the
+// device's last context, by rtx_ctx_trim, and where an allocation of the
+// library finds no memory (build_workspace_drop).  A build ends with its stream
 // synchronized, so the next one may use the block on any stream.
 class BuildWorkspace {
 public:
     static constexpr size_t kKeepBytes = (size_t)4 << 30;
+    static constexpr size_t kShrinkBytes = (size_t)64 << 20;   // smaller blocks do not shrink
+    static constexpr uint32_t kShrinkAfter = 8;
     // for a build that takes `bytes` at once at most (with that device current)
     BuildWorkspace(int device, size_t bytes);
     ~BuildWorkspace();
@@ -81,7 +85,9 @@ private:
     size_t cap_ = 0, used_ = 0;
     std::vector<void*> more_;
 };
-void build_workspace_drop(int device);
+// frees the block of a device unless a build uses it; false: nothing to free.
+// Not for the thread of a running build.
+bool build_workspace_drop(int device);
 // the workspace bytes that build_bvh over N primitives usually takes (what
 // goes beyond is allocated then) and that its result takes when not owned
 size_t bvh_workspace_bytes(uint32_t N);

@@ -1313,6 +1313,7 @@ struct KeptBlock {
     std::mutex taken;          // held by the build that uses the block
     uint8_t* base = nullptr;
     size_t cap = 0;
+    uint32_t small = 0;        // builds in a row that took a small part of it
     uint32_t* host = nullptr;
 };
 constexpr int kMaxDevices = 64;
@@ -1324,7 +1325,9 @@ BuildWorkspace::BuildWorkspace(int device, size_t bytes) : device_(device) {
     if (device < 0 || device >= kMaxDevices || !g_kept[device].taken.try_lock()) return;
     KeptBlock& k = g_kept[device];
     shared_ = true;
-    if (bytes <= kKeepBytes && k.cap < bytes) {
+    k.small = k.cap > kShrinkBytes && bytes < k.cap / 8 ? k.small + 1 : 0;
+    if (bytes <= kKeepBytes && (k.cap < bytes || k.small == kShrinkAfter)) {
+        k.small = 0;
         if (k.base) (void)hipFree(k.base);
         k.base = nullptr;
         k.cap = 0;
@@ -1369,16 +1372,19 @@ hipError_t BuildWorkspace::host_words(uint32_t** h) {
     return hipSuccess;
 }
 
-void build_workspace_drop(int device) {
-    if (device < 0 || device >= kMaxDevices) return;
+bool build_workspace_drop(int device) {
+    if (device < 0 || device >= kMaxDevices) return false;
     KeptBlock& k = g_kept[device];
-    if (!k.taken.try_lock()) return;   // a build is running: its contexts outlive it
+    if (!k.taken.try_lock()) return false;   // a build is running
+    const bool had = k.base != nullptr;
     if (k.base) (void)hipFree(k.base);
     if (k.host) (void)hipHostFree(k.host);
     k.base = nullptr;
     k.host = nullptr;
     k.cap = 0;
+    k.small = 0;
     k.taken.unlock();
+    return had;
 }
 
 size_t bvh_workspace_bytes(uint32_t N) {

@@ -172,6 +172,17 @@ extern "C" {
 
 const char* rtx_last_error(void) { return g_err.c_str(); }
 
+// hipMalloc; where there is no memory, again without what builds keep (not
+// for the thread of a running build)
+static hipError_t dev_alloc(int device, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && rtx::build_workspace_drop(device)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 static rtx_status alloc_scratch(rtx::LaunchScratch& ls, uint32_t blocks_per_cu, int num_cus, int block) {
     ls.grid = blocks_per_cu * (uint32_t)num_cus;
     ls.grid_max = ls.grid;
@@ -184,7 +195,7 @@ static rtx_status alloc_scratch(rtx::LaunchScratch& ls, uint32_t blocks_per_cu, 
 // launch that needs it, so contexts that only hold a scene for a batch cost
 // nothing beyond the scene; it grows when a scene needs a deeper stack.  lds:
 // the entries that every kernel using it holds in LDS
-static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need, uint32_t lds = rtx::kMinStackLDS) {
+static rtx_status ensure_gstack(int device, rtx::LaunchScratch& ls, uint32_t need, uint32_t lds = rtx::kMinStackLDS) {
     const uint32_t over = need > lds ? need - lds : 0u;
     if (ls.gstack_entries >= over) return RTX_SUCCESS;
     if (ls.gstack) {
@@ -193,7 +204,7 @@ static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need, uint32_t 
         ls.gstack = nullptr;
         ls.gstack_entries = 0;
     }
-    HIP_OK(hipMalloc((void**)&ls.gstack, sizeof(uint32_t) * (size_t)over * ls.gstride));
+    HIP_OK(dev_alloc(device, (void**)&ls.gstack, sizeof(uint32_t) * (size_t)over * ls.gstride));
     ls.gstack_entries = over;
     return RTX_SUCCESS;
 }
@@ -202,7 +213,7 @@ static rtx_status ensure_gstack(rtx::LaunchScratch& ls, uint32_t need, uint32_t 
 // allocated by the first launch that needs them and grown with the frame.
 // Where they cannot be (the stream is being captured, no memory is left) the
 // frame is rendered in slot order: the order is no launch's due.
-static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles, hipStream_t s) {
+static rtx_status ensure_order(int device, rtx::LaunchScratch& ls, uint32_t ntiles, hipStream_t s) {
     if (ls.tile_cost && ls.tile_cap >= ntiles) return RTX_SUCCESS;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
@@ -218,9 +229,9 @@ static rtx_status ensure_order(rtx::LaunchScratch& ls, uint32_t ntiles, hipStrea
         ls.pix_cost = nullptr;
         ls.tile_cap = 0;
     }
-    hipError_t e = hipMalloc((void**)&ls.tile_cost, sizeof(uint32_t) * (size_t)ntiles);
-    if (e == hipSuccess) e = hipMalloc((void**)&ls.tile_order, sizeof(uint32_t) * (size_t)ntiles);
-    if (e == hipSuccess) e = hipMalloc((void**)&ls.pix_cost, sizeof(uint16_t) * 64u * (size_t)ntiles);
+    hipError_t e = dev_alloc(device, (void**)&ls.tile_cost, sizeof(uint32_t) * (size_t)ntiles);
+    if (e == hipSuccess) e = dev_alloc(device, (void**)&ls.tile_order, sizeof(uint32_t) * (size_t)ntiles);
+    if (e == hipSuccess) e = dev_alloc(device, (void**)&ls.pix_cost, sizeof(uint16_t) * 64u * (size_t)ntiles);
     if (e != hipSuccess) {
         if (ls.tile_cost) (void)hipFree(ls.tile_cost);
         if (ls.tile_order) (void)hipFree(ls.tile_order);
@@ -294,6 +305,13 @@ rtx_status rtx_ctx_destroy(rtx_ctx* c) {
     }
     if (last) rtx::build_workspace_drop(c->device);
     delete c;
+    return RTX_SUCCESS;
+}
+
+rtx_status rtx_ctx_trim(rtx_ctx* c) {
+    if (!c) return fail(RTX_ERROR_INVALID_VALUE, "rtx_ctx_trim: ctx is NULL");
+    HIP_OK(hipSetDevice(c->device));
+    (void)rtx::build_workspace_drop(c->device);
     return RTX_SUCCESS;
 }
 
@@ -412,8 +430,8 @@ rtx_status rtx_mesh_add(rtx_ctx* c, const rtx_float3* vces, uint32_t nv, const r
     MeshRec m;
     m.nv = nv;
     m.ni = ni;
-    HIP_OK(hipMalloc((void**)&m.d_v, sizeof(rtx_float3) * (nv ? nv : 1)));
-    HIP_OK(hipMalloc((void**)&m.d_i, sizeof(rtx_uint3) * (ni ? ni : 1)));
+    HIP_OK(dev_alloc(c->device, (void**)&m.d_v, sizeof(rtx_float3) * (nv ? nv : 1)));
+    HIP_OK(dev_alloc(c->device, (void**)&m.d_i, sizeof(rtx_uint3) * (ni ? ni : 1)));
     if (nv) HIP_OK(hipMemcpy(m.d_v, vces, sizeof(rtx_float3) * nv, hipMemcpyHostToDevice));
     if (ni) HIP_OK(hipMemcpy(m.d_i, ices, sizeof(rtx_uint3) * ni, hipMemcpyHostToDevice));
     *mesh_id = (uint32_t)c->meshes.size();
@@ -989,8 +1007,14 @@ static rtx_status refit_scene_tl(rtx_ctx* c, Built* b, hipStream_t s) {
     return RTX_SUCCESS;
 }
 
-static rtx_status build_scene(rtx_ctx* c, hipStream_t s, Built** out) {
-    return c->build_mode == RTX_BUILD_TWO_LEVEL ? build_scene_tl(c, s, out) : build_scene_flat(c, s, out);
+static rtx_status build_scene(rtx_ctx* c, bool two_level, hipStream_t s, Built** out) {
+    rtx_status st = two_level ? build_scene_tl(c, s, out) : build_scene_flat(c, s, out);
+    if (st == RTX_ERROR_OUT_OF_MEMORY && rtx::build_workspace_drop(c->device)) {
+        // again without the block that a larger build may have left
+        (void)hipGetLastError();
+        st = two_level ? build_scene_tl(c, s, out) : build_scene_flat(c, s, out);
+    }
+    return st;
 }
 
 rtx_status rtx_scene_set_build_mode(rtx_ctx* c, int mode) {
@@ -1011,7 +1035,7 @@ rtx_status rtx_scene_get_build_mode(rtx_ctx* c, int* mode) {
 rtx_status rtx_scene_build(rtx_ctx* c, void* stream, uint64_t* is_handle) {
     if (!c || !is_handle) return fail(RTX_ERROR_INVALID_VALUE, "rtx_scene_build: NULL argument");
     Built* b = nullptr;
-    rtx_status st = build_scene(c, (hipStream_t)stream, &b);
+    rtx_status st = build_scene(c, c->build_mode == RTX_BUILD_TWO_LEVEL, (hipStream_t)stream, &b);
     if (st != RTX_SUCCESS) return st;
     drop_built(c);
     c->built = b;
@@ -1035,7 +1059,7 @@ rtx_status rtx_scene_update(rtx_ctx* c, uint64_t is_handle, void* stream) {
     if (c->built->two_level && c->built->hdr.num_insts == (uint32_t)c->things.size())
         return refit_scene_tl(c, c->built, s);
     Built* b = nullptr;
-    rtx_status st = c->built->two_level ? build_scene_tl(c, s, &b) : build_scene_flat(c, s, &b);
+    rtx_status st = build_scene(c, c->built->two_level, s, &b);
     if (st != RTX_SUCCESS) return st;
     Built* old = c->built;
     HIP_OK(hipMemcpyAsync(old->d_hdr, &b->hdr, sizeof(rtx::DevScene), hipMemcpyHostToDevice, s));
@@ -1078,11 +1102,11 @@ rtx_status rtx_scene_triangles(rtx_ctx* c, uint64_t is_handle, float* tris, uint
         Tmp<rtx::InstBuild> d_ib;
         Tmp<rtx::MeshRef> d_mr;
         Tmp<float4> d_tw, d_plo, d_phi;
-        HIP_OK(hipMalloc((void**)&d_ib.p, sizeof(rtx::InstBuild) * b->ib.size()));
-        HIP_OK(hipMalloc((void**)&d_mr.p, sizeof(rtx::MeshRef) * mr.size()));
-        HIP_OK(hipMalloc((void**)&d_tw.p, sizeof(float4) * h.size()));
-        HIP_OK(hipMalloc((void**)&d_plo.p, sizeof(float4) * N));
-        HIP_OK(hipMalloc((void**)&d_phi.p, sizeof(float4) * N));
+        HIP_OK(dev_alloc(c->device, (void**)&d_ib.p, sizeof(rtx::InstBuild) * b->ib.size()));
+        HIP_OK(dev_alloc(c->device, (void**)&d_mr.p, sizeof(rtx::MeshRef) * mr.size()));
+        HIP_OK(dev_alloc(c->device, (void**)&d_tw.p, sizeof(float4) * h.size()));
+        HIP_OK(dev_alloc(c->device, (void**)&d_plo.p, sizeof(float4) * N));
+        HIP_OK(dev_alloc(c->device, (void**)&d_phi.p, sizeof(float4) * N));
         HIP_OK(hipMemcpy(d_ib.p, b->ib.data(), sizeof(rtx::InstBuild) * b->ib.size(), hipMemcpyHostToDevice));
         HIP_OK(hipMemcpy(d_mr.p, mr.data(), sizeof(rtx::MeshRef) * mr.size(), hipMemcpyHostToDevice));
         HIP_OK(rtx::flatten_scene(d_ib.p, ninst, d_mr.p, N, d_tw.p, d_plo.p, d_phi.p, nullptr));
@@ -1121,9 +1145,9 @@ rtx_status rtx_launch(rtx_ctx* c, const rtx_lp_general* lp, int once, void* stre
         if (lp->spp == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: spp == 0");
         if (lp->depth == 0) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: depth == 0");
         if (!lp->rawRGB) return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch: rawRGB is NULL");
-        if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
+        if (rtx_status st = ensure_gstack(c->device, c->render_ls, b->stack_need)) return st;
         if (rtx::frame_ordered(*lp, c->render_ls))
-            if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
+            if (rtx_status st = ensure_order(c->device, c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
         e = rtx::launch_render(b->hdr, *lp, amb, c->render_ls, (hipStream_t)stream);
     }
     if (e != hipSuccess) return hip_fail(e, "rtx_launch");
@@ -1252,7 +1276,7 @@ rtx_status rtx_batch_create(rtx_ctx* c, const rtx_lp_general* lps, uint32_t n, i
     HIP_OK(hipSetDevice(c->device));
     uint32_t need = 1;
     for (uint32_t i = 0; i < n; i++) need = std::max(need, built[i]->stack_need);
-    if (rtx_status st = ensure_gstack(c->render_ls, need)) return st;
+    if (rtx_status st = ensure_gstack(c->device, c->render_ls, need)) return st;
     rtx_batch* b = new rtx_batch();
     b->ctx = c;
     b->njobs = n;
@@ -1263,7 +1287,7 @@ rtx_status rtx_batch_create(rtx_ctx* c, const rtx_lp_general* lps, uint32_t n, i
     b->handles.resize(n);
     for (uint32_t k = 0; k < n; k++) b->handles[k] = lps[order[k]].is_handle;
     b->use_graph = use_graph != 0;
-    hipError_t e = hipMalloc((void**)&b->d_jobs, sizeof(rtx::Job) * n);
+    hipError_t e = dev_alloc(c->device, (void**)&b->d_jobs, sizeof(rtx::Job) * n);
     if (e == hipSuccess) e = hipMemcpy(b->d_jobs, jobs.data(), sizeof(rtx::Job) * n, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         if (b->d_jobs) (void)hipFree(b->d_jobs);
@@ -1297,7 +1321,7 @@ rtx_status rtx_batch_launch(rtx_batch* b, void* stream) {
         HIP_OK(hipStreamSynchronize(s));
         HIP_OK(hipMemcpy(b->d_jobs, b->jobs.data(), sizeof(rtx::Job) * b->njobs, hipMemcpyHostToDevice));
         b->first = b->jobs[0];
-        if (rtx_status st = ensure_gstack(b->ctx->render_ls, need)) return st;
+        if (rtx_status st = ensure_gstack(b->ctx->device, b->ctx->render_ls, need)) return st;
         if (b->exec) {
             // the captured kernel arguments hold the first job: capture again
             (void)hipGraphExecDestroy(b->exec);
@@ -1391,7 +1415,7 @@ rtx_status rtx_launch_adjoint(rtx_ctx* c, const rtx_lp_general* lp, const rtx_fl
     if (lp->depth > 64) return fail(RTX_ERROR_LIMIT, "rtx_launch_adjoint: depth > 64");
     if (b->hdr.num_insts >= (1u << 24)) return fail(RTX_ERROR_LIMIT, "rtx_launch_adjoint: 2^24 or more instances");
     HIP_OK(hipSetDevice(c->device));
-    if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
+    if (rtx_status st = ensure_gstack(c->device, c->render_ls, b->stack_need)) return st;
     if (c->tape_depth < lp->depth) {
         // path records of 14 words for every lane of the grid: a path records
         // each hit it shades, at most depth - 1 under the recursive programs
@@ -1404,11 +1428,11 @@ rtx_status rtx_launch_adjoint(rtx_ctx* c, const rtx_lp_general* lp, const rtx_fl
             c->tape_depth = 0;
         }
         const size_t words = (size_t)lp->depth * rtx::kAdjointTapeWords * c->render_ls.gstride;
-        HIP_OK(hipMalloc((void**)&c->tape, words * sizeof(uint32_t)));
+        HIP_OK(dev_alloc(c->device, (void**)&c->tape, words * sizeof(uint32_t)));
         c->tape_depth = lp->depth;
     }
     if (rtx::frame_ordered(*lp, c->render_ls, true))
-        if (rtx_status st = ensure_order(c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
+        if (rtx_status st = ensure_order(c->device, c->render_ls, rtx::frame_tiles(*lp, c->render_ls.tile_w), (hipStream_t)stream)) return st;
     const float3 amb = make_float3(c->ambient.x, c->ambient.y, c->ambient.z);
     hipError_t e = rtx::launch_adjoint(b->hdr, *lp, amb, c->render_ls, dL_drgb, d_params, c->tape,
                                        c->render_ls.gstride, (hipStream_t)stream);
@@ -1424,7 +1448,7 @@ rtx_status rtx_launch_counted(rtx_ctx* c, const rtx_lp_general* lp, uint64_t* no
     if (lp->image_w == 0 || lp->image_h == 0 || lp->spp == 0 || lp->depth == 0 || !lp->rawRGB)
         return fail(RTX_ERROR_INVALID_VALUE, "rtx_launch_counted: bad launch parameters");
     HIP_OK(hipSetDevice(c->device));
-    if (rtx_status st = ensure_gstack(c->render_ls, b->stack_need)) return st;
+    if (rtx_status st = ensure_gstack(c->device, c->render_ls, b->stack_need)) return st;
     rtx::TraceCounters tc;
     tc.nodes = node_visits;
     tc.tris = tri_tests;
@@ -1441,7 +1465,7 @@ rtx_status rtx_trace(rtx_ctx* c, uint64_t is_handle, const rtx_ray* rays, uint32
     if (!b) return fail(RTX_ERROR_INVALID_HANDLE, "rtx_trace: unknown handle");
     if (n && (!rays || !hits)) return fail(RTX_ERROR_INVALID_VALUE, "rtx_trace: NULL buffer");
     HIP_OK(hipSetDevice(c->device));
-    if (rtx_status st = ensure_gstack(c->trace_ls, b->stack_need, rtx::kStackLDS)) return st;
+    if (rtx_status st = ensure_gstack(c->device, c->trace_ls, b->stack_need, rtx::kStackLDS)) return st;
     hipError_t e = rtx::launch_trace(b->hdr, rays, n, hits, c->trace_ls, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "rtx_trace");
     return RTX_SUCCESS;
@@ -1473,7 +1497,9 @@ rtx_status rtx_pp_none(const rtx_float3* src, rtx_uchar4* dst, int w, int h, voi
 // ---- plumbing ---------------------------------------------------------------
 rtx_status rtx_malloc(void** p, size_t bytes) {
     if (!p) return fail(RTX_ERROR_INVALID_VALUE, "rtx_malloc: NULL argument");
-    HIP_OK(hipMalloc(p, bytes ? bytes : 1));
+    int device = 0;
+    HIP_OK(hipGetDevice(&device));
+    HIP_OK(dev_alloc(device, p, bytes ? bytes : 1));
     return RTX_SUCCESS;
 }
 rtx_status rtx_free(void* p) {
