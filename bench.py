@@ -18,7 +18,7 @@ x rays per second measured here, against 256 CUs x 2.4 GHz x one wave
 instruction per CU per clock.  Beside it: the share of lanes active per VALU
 instruction, the HBM bytes per launch from the FETCH_SIZE / WRITE_SIZE
 counters (scaled by a copy kernel of known size) against the 8 TB/s peak,
-and the bytes per ray that the traversal touches (node visits x 76 B +
+and the bytes per ray that the traversal touches (node visits x 80 B +
 triangle tests x 48 B + shading 80 B + ray in/out 48 B: bytes served by
 L1, L2 and the MALL, most of them never from HBM).
 
@@ -55,10 +55,11 @@ HBM_PEAK_GBS = 8000.0
 # VALU issue: one wave instruction per CU per clock, 256 CUs at the 2.4 GHz peak clock
 CUS, PEAK_GHZ = 256, 2.4
 VALU_PEAK_GINST = CUS * PEAK_GHZ
-# bytes per 4-wide node visit (6 plane float4 + the refs float4), per
+# bytes per 4-wide node visit (three axes' planes, 16 B each as halves, the
+# origin and scale, and the refs), per
 # triangle test, per shading step (hit triangle 48 + instance record 32) and
 # per ray for its own input/output (ray 32 in, hit 16 out)
-NODE_BYTES, TRI_BYTES, SHADE_BYTES, IO_BYTES = 76, 48, 80, 48
+NODE_BYTES, TRI_BYTES, SHADE_BYTES, IO_BYTES = 80, 48, 80, 48
 PROFILES = os.path.join(ROOT, "profiles")
 # the sphere list of every leg but the batch: RTWO::load on the reference's
 # own rand() stream (optx/rtwo.cxx:137-244), the scene its batch binary renders

@@ -520,7 +520,8 @@ __device__ __forceinline__ void render_body(const RenderArgs& a, uint32_t* s_sta
 // whose lanes split between LDS and global nodes issue both loads for too
 // little latency saved (measured with 128-byte float nodes).  So frames of at
 // least kOrderMinSpp samples per pixel of scenes of at least kLdsTopMinNodes
-// nodes take the staged kernels.
+// nodes take the staged kernels (11 and 14 samples, staged against not: 1080p
+// 1.01x both, 720p 1.00x both).
 #ifndef RTX_LDS_TOP
 #define RTX_LDS_TOP 24
 #endif
@@ -544,7 +545,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_RENDE
     render_body<BLOCK, COUNT, false, SLDS, false, TL, false, TOPN>(a, s_stack, nullptr, (const lds_f4*)s_top);
 }
 
-// the probe of a plain frame: one sample per pixel, rays counted per tile
+// the probe of an ordered frame: one sample per pixel, each pixel's node visits
+// and kProbeRayCost for each of its rays to pix_cost
 template <int BLOCK, int SLDS, bool TL, int TOPN>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_RENDER_WAVES))) void k_probe(const RenderArgs a) {
     __shared__ uint32_t s_stack[(SLDS + 1) * BLOCK];
@@ -779,7 +781,6 @@ uint32_t log2u(uint32_t v) {
     return l;
 }
 
-// the frame kernel for the scene's kind (flat / two-level) and the LDS stack size
 // the frame kernel for the scene's kind (flat / two-level), the LDS stack
 // size and whether the top nodes go to LDS (large scenes, not the counted launch)
 template <bool COUNT, int TOPN>
