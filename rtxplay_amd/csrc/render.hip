@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kOrderBlock) void k_tile_order(const uint32_t* cost
 
 // batch: the same loop with a job per lane, whose job state takes registers:
 // flat scenes keep 4 waves per SIMD by a few spills outside the node loop
-// (16 registers; 3 waves without are slower), two-level ones take the
+// (4 registers; 3 waves without are slower), two-level ones take the
 // registers of 3 waves
 template <int BLOCK, int SLDS, bool TL>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RTX_BATCH_WAVES))) void k_render_batch(const RenderArgs a) {
